@@ -30,7 +30,8 @@ HIP_FLAGS = [
     "-Wall", "-Wno-unused-function", "-Wno-unused-variable",
     "-I", INCLUDE,
 ]
-HIP_SOURCES = ["alv_step.hip", "alv_capi.hip", "alv_mlp.hip", "alv_contact.hip", "alv_sample.hip"]
+HIP_SOURCES = ["alv_step.hip", "alv_capi.hip", "alv_mlp.hip", "alv_contact.hip", "alv_sample.hip",
+               "alv_volume.hip"]
 LIB = os.path.join(PKG, "libalv.so")
 
 

@@ -285,6 +285,7 @@ struct alv_pile {
   float gravity[3] = {0.f, 0.f, 0.f};
   unsigned max_num_contacts = 0;
   float* peirce = nullptr;  // device, 120 floats
+  float peirce_host[120];
   // rigid contacts: collision vertices per body (host, body frame), their
   // concatenation on the device, and the contact buffers
   std::vector<std::vector<float>> coll_verts;
@@ -681,10 +682,10 @@ int alv_pile_create_ex(alv_pile** out, unsigned max_num_contacts, int volume_met
   p->volume_method = volume_method;
   // max_num_pellets_ is 0 for volume maps (pile.hpp:162-163)
   p->max_pellets = volume_method == ALV_PELLETS ? max_num_pellets : 0u;
-  float table[120];
-  peirce_table(table);
-  hipError_t e = hipMalloc(&p->peirce, sizeof(table));
-  if (e == hipSuccess) e = hipMemcpy(p->peirce, table, sizeof(table), hipMemcpyHostToDevice);
+  peirce_table(p->peirce_host);
+  hipError_t e = hipMalloc(&p->peirce, sizeof(p->peirce_host));
+  if (e == hipSuccess)
+    e = hipMemcpy(p->peirce, p->peirce_host, sizeof(p->peirce_host), hipMemcpyHostToDevice);
   if (e != hipSuccess) {
     delete p;
     return fail(ALV_ERR_HIP, hipGetErrorString(e));
@@ -852,21 +853,29 @@ int place_boundary(alv_pile* pile, int slot, const alv_const* cn, const alv_dist
   alv_consti cni;
   memset(&cni, 0, sizeof(cni));
   SimParams p = make_params(*cn, cni, 0, 0);
-  const unsigned chunk = 1u << 20;
-  for (unsigned b = 0; !pellets && b < B.geom.num_nodes; b += chunk) {
-    unsigned e = std::min(B.geom.num_nodes, b + chunk);
-    if (dmap)  // update_volume_field from the distance map (runner.hpp:1616-1658)
-      launch_volume_field_grid(p, B.geom, dmap, vol, sign, pile->peirce, b, e, 0);
-    else
-      launch_volume_field_analytic(p, B, vol, pile->peirce, b, e, 0);
-    ALV_HIP(hipGetLastError());
-  }
   unsigned char* flags = nullptr;
   if (!pellets) {
-    ALV_HIP(hipMalloc(&flags, std::max<size_t>(size_t(res[0]) * res[1] * res[2], 1)));
-    launch_map_flags(B.geom, vol, flags, nullptr);
-    ALV_HIP(hipGetLastError());
-    ALV_HIP(hipDeviceSynchronize());
+    void* ws = nullptr;
+    hipError_t e = hipMalloc(&ws, volume_field_workspace(B.geom, dmap != nullptr));
+    if (e == hipSuccess)
+      e = hipMalloc(&flags, std::max<size_t>(size_t(res[0]) * res[1] * res[2], 1));
+    if (e == hipSuccess) {
+      if (dmap)  // update_volume_field from the distance map (runner.hpp:1616-1658)
+        launch_volume_field_grid(p, B.geom, dmap, vol, sign, pile->peirce, pile->peirce_host, ws, 0);
+      else
+        launch_volume_field_analytic(p, B, vol, pile->peirce, pile->peirce_host, ws, 0);
+      launch_map_flags(B.geom, vol, flags, nullptr);
+      e = hipGetLastError();
+      const hipError_t done = hipDeviceSynchronize();
+      if (e == hipSuccess) e = done;
+    }
+    (void)hipFree(ws);
+    if (e != hipSuccess) {
+      (void)hipFree(flags);
+      (void)hipFree(vol);
+      (void)hipFree(dmap);
+      return fail(ALV_ERR_HIP, std::string("volume map: ") + hipGetErrorString(e));
+    }
   }
   B.cell_nz = flags;
   std::array<float, 3> I = {inertia ? inertia[0] : 1.f, inertia ? inertia[1] : 1.f,
@@ -2718,16 +2727,19 @@ int alv_volume_from_distance_map(const alv_const* cn, const float dmin[3], const
   float table[120];
   peirce_table(table);
   float *dd = nullptr, *dv = nullptr, *dp = nullptr;
-  ALV_HIP(hipMalloc(&dd, size_t(num_nodes) * sizeof(float)));
-  ALV_HIP(hipMalloc(&dv, size_t(num_nodes) * sizeof(float)));
-  ALV_HIP(hipMalloc(&dp, sizeof(table)));
-  hipError_t e = hipMemcpy(dd, distance, size_t(num_nodes) * sizeof(float), hipMemcpyHostToDevice);
+  void* ws = nullptr;
+  hipError_t e = hipMalloc(&dd, size_t(num_nodes) * sizeof(float));
+  if (e == hipSuccess) e = hipMalloc(&dv, size_t(num_nodes) * sizeof(float));
+  if (e == hipSuccess) e = hipMalloc(&dp, sizeof(table));
+  if (e == hipSuccess) e = hipMalloc(&ws, volume_field_workspace(g, true));
+  if (e == hipSuccess)
+    e = hipMemcpy(dd, distance, size_t(num_nodes) * sizeof(float), hipMemcpyHostToDevice);
   if (e == hipSuccess) e = hipMemcpy(dp, table, sizeof(table), hipMemcpyHostToDevice);
   if (e == hipSuccess) {
     alv_consti cni;
     memset(&cni, 0, sizeof(cni));
     SimParams p = make_params(*cn, cni, 0, 0);
-    launch_volume_field_grid(p, g, dd, dv, sign, dp, 0, num_nodes, 0);
+    launch_volume_field_grid(p, g, dd, dv, sign, dp, table, ws, 0);
     e = hipGetLastError();
   }
   if (e == hipSuccess)
@@ -2735,6 +2747,7 @@ int alv_volume_from_distance_map(const alv_const* cn, const float dmin[3], const
   (void)hipFree(dd);
   (void)hipFree(dv);
   (void)hipFree(dp);
+  (void)hipFree(ws);
   if (e != hipSuccess) return fail(ALV_ERR_HIP, hipGetErrorString(e));
   return ALV_OK;
 }

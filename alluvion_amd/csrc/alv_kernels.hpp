@@ -342,14 +342,15 @@ void launch_export_boundary(const Launch& L, const DevArrays& A, float4* rec, fl
 void launch_export_iisph(const Launch& L, const DevArrays& A, float* const scalar[4],
                          float* const vec[3], hipStream_t s);
 
-// volume maps (setup)
+// volume maps (setup, alv_volume.hip): the Peirce constants on the device and
+// on the host, and a workspace of volume_field_workspace bytes
+size_t volume_field_workspace(const GridGeomDev& g, bool distance_map);
 void launch_volume_field_analytic(const SimParams& p, const BoundaryDev& b, float* volume,
-                                  const float* peirce, unsigned begin, unsigned end,
+                                  const float* peirce, const float* peirce_host, void* workspace,
                                   hipStream_t s);
-void launch_volume_field_grid(const SimParams& p, const GridGeomDev& g,
-                              const float* distance, float* volume, float sign,
-                              const float* peirce, unsigned begin, unsigned end,
-                              hipStream_t s);
+void launch_volume_field_grid(const SimParams& p, const GridGeomDev& g, const float* distance,
+                              float* volume, float sign, const float* peirce,
+                              const float* peirce_host, void* workspace, hipStream_t s);
 void launch_node_positions(const GridGeomDev& g, float* out, hipStream_t s);
 // element-wise device arithmetic of the kernel functions (alv_check_math)
 void launch_check_math(const SimParams& p, int op, const float* a, const float* b, float* out,

@@ -2297,74 +2297,6 @@ __global__ __launch_bounds__(256) void k_export_iisph(SceneTab T, DevArrays A, f
   if (pacc) st3(pacc, i, ld3(A.pacc[s]));
 }
 
-// ---------------------------------------------------------------------------
-// Volume maps (update_volume_field, runner.hpp:1616-1694).  Peirce constants
-// are packed as cosphi[30], sinphi[30], b[30], r[15], c[15].
-// ---------------------------------------------------------------------------
-constexpr float kPiF = 3.14159265358979323846f;
-
-__global__ __launch_bounds__(256) void k_volume_analytic(SimParams p, BoundaryDev B,
-                                                         float* volume, const float* pc,
-                                                         unsigned begin, unsigned end) {
-  const unsigned l = begin + blockIdx.x * kBlock + threadIdx.x;
-  if (l >= end) return;
-  const float* cosphi = pc;
-  const float* sinphi = pc + 30;
-  const float* kb = pc + 60;
-  const float* kr = pc + 90;
-  const float* kc = pc + 105;
-  vec3 x = node_position(B.geom, l);
-  float sum = 0.0f;
-  for (unsigned i = 0; i < 60; ++i) {
-    float theta = 2.0f * kPiF * float(i + 1) / 60.0f;
-    float ct = cosf(theta), st = sinf(theta);
-    for (unsigned j = 0; j < 30; ++j) {
-      for (unsigned k = 0; k < 15; ++k) {
-        float wijk = 2.0f * kPiF * kb[j] * kc[k] / 60.0f;
-        vec3 u = mk(sinphi[j] * ct, sinphi[j] * st, cosphi[j]);
-        vec3 q = (p.h * kr[k]) * u;
-        float dist = sdf_eval(B, x + q);
-        float dm = dist * B.sign;
-        sum += wijk * (dm <= 0.0f ? 1.0f : W_dist(dm, p) / p.w0);
-      }
-    }
-  }
-  volume[l] = sum * p.h2 * p.h;
-}
-
-__global__ __launch_bounds__(256) void k_volume_grid(SimParams p, GridGeomDev g,
-                                                     const float* __restrict__ dist,
-                                                     float* volume, float sign,
-                                                     const float* pc, unsigned begin,
-                                                     unsigned end) {
-  const unsigned l = begin + blockIdx.x * kBlock + threadIdx.x;
-  if (l >= end) return;
-  const float* cosphi = pc;
-  const float* sinphi = pc + 30;
-  const float* kb = pc + 60;
-  const float* kr = pc + 90;
-  const float* kc = pc + 105;
-  vec3 x = node_position(g, l);
-  float sum = 0.0f;
-  const float wi = 2.0f * kPiF / 60.0f;
-  for (unsigned i = 0; i < 60; ++i) {
-    float theta = 2.0f * kPiF * float(i + 1) / 60.0f;
-    float ct = cosf(theta), st = sinf(theta);
-    for (unsigned j = 0; j < 30; ++j) {
-      vec3 u = mk(sinphi[j] * ct, sinphi[j] * st, cosphi[j]);
-      float wij = wi * kb[j];
-      for (unsigned k = 0; k < 15; ++k) {
-        float wijk = wij * kc[k];
-        vec3 q = (p.h * kr[k]) * u;
-        float d = grid_sample(g, dist, x + q, FLT_MAX);
-        float dm = d * sign;
-        sum += wijk * (dm <= 0.0f ? 1.0f : W_dist(dm, p) / p.w0);
-      }
-    }
-  }
-  volume[l] = sum * p.h2 * p.h;
-}
-
 __global__ __launch_bounds__(256) void k_node_positions(GridGeomDev g, float* out) {
   const unsigned l = blockIdx.x * kBlock + threadIdx.x;
   if (l >= g.num_nodes) return;
@@ -2885,20 +2817,6 @@ void launch_export_iisph(const Launch& L, const DevArrays& A, float* const scala
                          float* const vec[3], hipStream_t s) {
   ALV_LAUNCH(k_export_iisph, L, s, A, scalar[0], scalar[1], scalar[2], scalar[3], vec[0],
              vec[1], vec[2]);
-}
-void launch_volume_field_analytic(const SimParams& p, const BoundaryDev& b, float* volume,
-                                  const float* peirce, unsigned begin, unsigned end,
-                                  hipStream_t s) {
-  if (end <= begin) return;
-  hipLaunchKernelGGL(k_volume_analytic, dim3(grid_for(end - begin)), dim3(kBlock), 0, s, p, b,
-                     volume, peirce, begin, end);
-}
-void launch_volume_field_grid(const SimParams& p, const GridGeomDev& g, const float* distance,
-                              float* volume, float sign, const float* peirce, unsigned begin,
-                              unsigned end, hipStream_t s) {
-  if (end <= begin) return;
-  hipLaunchKernelGGL(k_volume_grid, dim3(grid_for(end - begin)), dim3(kBlock), 0, s, p, g,
-                     distance, volume, sign, peirce, begin, end);
 }
 // The device arithmetic the kernel functions are built on, element-wise
 // (alv_check_math): 0 sqrt_rn(a), 1 div_known(a, b, RN(1/b)), 2 gradW_scale
