@@ -179,10 +179,12 @@ SimParams make_params(const alv_const& cn, const alv_consti& cni, unsigned num_b
   for (int a = 0; a < 3; ++a) {
     p.g[a] = cn.gravity[a];
     float L = cn.wrap_length[a];
-    p.wrap_len[a] = L;
-    p.wrap_min[a] = L * -0.5f;
-    p.wrap_max[a] = L * 0.5f;
-    if (L > 0.0f) p.wrap_mask |= 1 << a;
+    // an axis that is not periodic never wraps (wrap1)
+    const bool on = L > 0.0f;
+    p.wrap_len[a] = on ? L : 0.0f;
+    p.wrap_min[a] = on ? L * -0.5f : -INFINITY;
+    p.wrap_max[a] = on ? L * 0.5f : INFINITY;
+    if (on) p.wrap_mask |= 1 << a;
     p.res[a] = int(cni.grid_res[a]);
     p.off[a] = cni.grid_offset[a];
   }
@@ -1531,8 +1533,8 @@ static int solver_alloc(alv_solver* S) {
     ALV_ALLOC(A.density_err, cap);
     ALV_ALLOC(A.pacc, cap);
   }
-  ALV_ALLOC(A.partials, grid_for(cap) + 1);
-  ALV_ALLOC(A.fpartials, grid_for(cap) + 1);
+  ALV_ALLOC(A.partials, (grid_for(cap) + 1) * (kBlock / kDeepBlock));
+  ALV_ALLOC(A.fpartials, (grid_for(cap) + 1) * (kBlock / kDeepBlock));
   ALV_ALLOC(A.body_partials, std::max<size_t>(1, max_bnd) * 256 * 6);
   if (pcap) {
     A.pcap = pcap;
@@ -1821,6 +1823,20 @@ int alv_solver_get_report(const alv_solver* S, alv_solver_report* r) {
 }  // extern "C"
 
 namespace {
+// The cells of the grid fill the box of every periodic axis, so that a cell
+// relation over an end is a displacement of one length, and cells are so many
+// (five) that no other candidate lies near half a length away.
+int wrap_is_tight(const SimParams& p) {
+  for (int a = 0; a < 3; ++a) {
+    if (!(p.wrap_mask & (1 << a))) continue;
+    const double h = p.h, len = p.wrap_len[a];
+    if (p.res[a] < 5 || std::fabs(p.res[a] * h - len) > 1e-3 * h ||
+        std::fabs(p.off[a] * h + 0.5 * len) > 1e-3 * h)
+      return 0;
+  }
+  return 1;
+}
+
 // Scene parameters of every scene, uploaded when they changed, and the
 // launch description.  A single-scene solver follows num_particles.
 int solver_launch(alv_solver* S, Launch* L) {
@@ -1839,6 +1855,7 @@ int solver_launch(alv_solver* S, Launch* L) {
       p.res[a] = int(sc.res[a]);
       p.off[a] = sc.off[a];
     }
+    p.wrap_tight = wrap_is_tight(p);
     p.num_cells = sc.num_cells;
     p.first = sc.first;
     p.span = sc.span;
@@ -1869,6 +1886,8 @@ int solver_launch(alv_solver* S, Launch* L) {
   L->scenes = unsigned(ns);
   L->active = active;
   L->tiles = S->A.use_tiles;
+  L->deep = !L->tiles && pblocks <= kDeepMaxBlocks;
+  L->quad = !L->tiles && pblocks <= kQuadMaxBlocks;
   L->p0 = S->par_host[0];
   return ALV_OK;
 }
@@ -2315,7 +2334,7 @@ int alv_solver_step(alv_solver* S) {
       // with the divergence solve, its density-change passes computed the
       // viscosity
       if (L.active && !div) launch_df_viscosity(L, A, st);
-      launch_update_dt(L, A, st);
+      launch_update_dt(L, A, div, st);
       if (L.active) {
         launch_df_integrate_np(L, A, div, st);
         if (dens) {
@@ -2345,7 +2364,7 @@ int alv_solver_step(alv_solver* S) {
     if (rc != ALV_OK) return rc;
     launch_pellet_lists(L, Lp, A, st);
     if (L.active) launch_pellet_viscosity(L, A, st);
-    launch_update_dt(L, A, st);
+    launch_update_dt(L, A, 0, st);
     if (L.active) {
       launch_is_prepare_pellets(L, A, st);
       rc = run_loop(S, false, S->set.max_density_solve, &S->last_dens,
@@ -2359,7 +2378,7 @@ int alv_solver_step(alv_solver* S) {
     rc = neighbor_phase(S, L, 0);
     if (rc != ALV_OK) return rc;
     if (L.active) launch_ii_viscosity_predict(L, A, st);
-    launch_update_dt(L, A, st);
+    launch_update_dt(L, A, 0, st);
     if (L.active) {
       launch_is_prepare(L, A, st);
       rc = run_loop(S, false, S->set.max_density_solve, &S->last_dens,
@@ -2373,7 +2392,7 @@ int alv_solver_step(alv_solver* S) {
     rc = neighbor_phase(S, L, 0);
     if (rc != ALV_OK) return rc;
     if (L.active) launch_ii_viscosity_predict(L, A, st);
-    launch_update_dt(L, A, st);
+    launch_update_dt(L, A, 0, st);
     if (L.active) {
       launch_ii_predict(L, A, st);
       rc = run_loop(S, false, S->set.max_density_solve, &S->last_dens,

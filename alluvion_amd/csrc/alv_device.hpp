@@ -555,17 +555,18 @@ __device__ inline unsigned cell_linear(const int ip[3], const SimParams& p) {
   return (unsigned(ip[0]) * unsigned(p.res[1]) + unsigned(ip[1])) * unsigned(p.res[2]) +
          unsigned(ip[2]);
 }
+// Periodic wrap of a displacement on every axis (d - len from len / 2 on, d +
+// len below -len / 2), without a branch: the host gives an axis that is not
+// periodic the length 0 and infinite bounds.
 __device__ inline float wrap1(float d, float len, float lo, float hi) {
-  if (d >= hi)
-    d -= len;
-  else if (d < lo)
-    d += len;
-  return d;
+  float t = d >= hi ? len : 0.0f;
+  t = d < lo ? -len : t;
+  return d - t;
 }
 __device__ inline vec3 wrap_disp(vec3 d, const SimParams& p) {
-  if (p.wrap_mask & 1) d.x = wrap1(d.x, p.wrap_len[0], p.wrap_min[0], p.wrap_max[0]);
-  if (p.wrap_mask & 2) d.y = wrap1(d.y, p.wrap_len[1], p.wrap_min[1], p.wrap_max[1]);
-  if (p.wrap_mask & 4) d.z = wrap1(d.z, p.wrap_len[2], p.wrap_min[2], p.wrap_max[2]);
+  d.x = wrap1(d.x, p.wrap_len[0], p.wrap_min[0], p.wrap_max[0]);
+  d.y = wrap1(d.y, p.wrap_len[1], p.wrap_min[1], p.wrap_max[1]);
+  d.z = wrap1(d.z, p.wrap_len[2], p.wrap_min[2], p.wrap_max[2]);
   return d;
 }
 

@@ -120,6 +120,21 @@ constexpr unsigned kBlock = 256;
 // from global memory (2 or 4; the lanes of a particle lie in one quad).
 constexpr unsigned kLPP = 2;
 static_assert(kLPP == 2u || kLPP == 4u, "a particle's lanes lie in one quad");
+// How a neighbour pass reads its neighbours: gathers from global memory, the
+// block's LDS tile, or the deep form for few particles: four lanes per
+// particle with all of a particle's gathers in flight at once, in blocks of
+// kDeepBlock particles.
+enum { kGather = 0, kTile = 1, kDeep = 2 };
+constexpr unsigned kDeepLanes = 4;
+constexpr unsigned kDeepBlock = 64;
+// Particle blocks up to which a launch set takes the deep passes and the
+// four-lane search.  Whole DFSPH steps on an MI355X with the one and the other
+// form of the passes: 80,000 particles 258 and 237 us, 101,000 259 and 258,
+// 130,000 263 and 284 (four lanes waste the lists' tails and the chip is
+// full); of the search: 60,000 218 and 202, 80,000 258 and 251, 101,000 259
+// and 264, periodic 85,000 281 and 290.
+constexpr unsigned kDeepMaxBlocks = 384;
+constexpr unsigned kQuadMaxBlocks = 320;
 
 // Neighbour slots are stored in groups of four (one uint4 per particle and
 // group).  Each 64-particle wave owns one contiguous [groups][64] tile of
@@ -163,7 +178,13 @@ struct Launch {
   unsigned active;   // particles in all scenes
   SimParams p0;      // scene 0 (shared constants, wrap flags)
   int tiles;         // launch the LDS-tile instances of the neighbour passes
+  int deep;          // launch the deep instances (few particles)
+  int quad;          // launch the four-lane neighbour search (few particles)
 };
+// partial sums and maxima of a pass per 256-particle block
+inline unsigned parts_per_block(const Launch& L) {
+  return L.deep ? kBlock / kDeepBlock : 1u;
+}
 
 // Particle-kernel prologue: this block's particle index s (blocks remapped
 // per XCD, or linear), its scene's parameters p, and the scene's control
@@ -175,16 +196,15 @@ struct Launch {
   (A).ctl += scene_;                                     \
   (A).bnd += p.bnd_base
 #define ALV_SCENE(T, A, s) ALV_SCENE_AT(T, A, s, xcd_block())
-// Prologue of the density-change passes: with ONE (their LDS-tile
-// instances) one lane per particle as ALV_SCENE, else kLPP lanes per
-// particle in blocks of kLPP * 256 threads (one block per particle block);
-// q is the lane within the particle's lanes.
-#define ALV_SCENE_PASS(T, A, s, q, ONE)                                               \
-  constexpr unsigned lpp_ = (ONE) ? 1u : kLPP;                                        \
+// Prologue of the neighbour passes in mode M: LPP lanes per particle, in
+// blocks of kDeepBlock particles in the deep form, else of 256; q is the lane
+// within the particle's lanes, qblk_ the block.
+#define ALV_SCENE_PASS(T, A, s, q, M, LPP)                                            \
+  constexpr unsigned lpp_ = (LPP), ppb_ = (M) == kDeep ? kDeepBlock : kBlock;         \
   const unsigned qblk_ = xcd_block();                                                 \
   const unsigned q = threadIdx.x & (lpp_ - 1u);                                       \
-  const unsigned s = qblk_ * kBlock + threadIdx.x / lpp_;                             \
-  const unsigned scene_ = (T).blk_scene[qblk_];                                       \
+  const unsigned s = qblk_ * ppb_ + threadIdx.x / lpp_;                               \
+  const unsigned scene_ = (T).blk_scene[qblk_ / (kBlock / ppb_)];                     \
   const SimParams p = (T).par[scene_];                                                \
   (A).ctl += scene_;                                                                  \
   (A).bnd += p.bnd_base
@@ -232,7 +252,9 @@ void launch_df_div_iteration(const Launch& L, const DevArrays& A, hipStream_t s)
 // the viscosity of a step without a divergence solve (with one, that solve's
 // density-change passes compute it)
 void launch_df_viscosity(const Launch& L, const DevArrays& A, hipStream_t s);
-void launch_update_dt(const Launch& L, const DevArrays& A, hipStream_t s);
+// pass_parts: the maxima come from a density-change pass (in its form's
+// blocks), else from k_viscosity
+void launch_update_dt(const Launch& L, const DevArrays& A, int pass_parts, hipStream_t s);
 // fin: the divergence solve ran (and computed the viscosity): also finish it
 // and add the bodies' viscous reactions
 void launch_df_integrate_np(const Launch& L, const DevArrays& A, int fin, hipStream_t s);

@@ -40,6 +40,18 @@ __device__ inline vec3 wrapd(vec3 d, const SimParams& p) {
   return d;
 }
 
+// Whether any listed neighbour of the wave's active lanes may need the wrap: a
+// list reaches over a periodic end only from within h of it (with a margin
+// over rounding), when the grid's cells fill the periodic box exactly (tight).
+template <bool W>
+__device__ inline bool wave_wraps(vec3 x, const SimParams& p) {
+  if constexpr (!W) return false;
+  const float r = 1.01f * p.h;
+  const bool near = fabsf(x.x) > p.wrap_max[0] - r || fabsf(x.y) > p.wrap_max[1] - r ||
+                    fabsf(x.z) > p.wrap_max[2] - r;
+  return !p.wrap_tight || __ballot(near) != 0ull;
+}
+
 // Neighbour loops run in batches: the kNB indices, then all gathers of the
 // batch, are issued before any arithmetic, so a wave waits for two memory
 // latencies per batch instead of two per neighbour.  Empty slots point at the
@@ -481,19 +493,26 @@ __device__ inline bool stage_x(const DevArrays& A, unsigned blk, TileX& t) {
 // the reference order (dx outer, dz inner); inside a cell in ascending
 // particle id, which is ascending sorted index.
 // ---------------------------------------------------------------------------
-// Candidates staged per wave: the 64 particles of a wave mostly lie in one
-// (x, y) column of cells, so for each (dx, dy) row their candidate spans lie
-// in one range of about 64 + 2 cells' particles, which the wave copies into
-// LDS with coalesced loads; the lanes then read their own spans from LDS
-// instead of gathering from L2.  A row whose range exceeds kStage (a wave
-// across two columns) reads global memory.  The stage keeps kCB slots of
-// slack past kStage, so that a batch may read up to kCB - 1 entries past its
-// span's end (masked out of its hits) without clamping its addresses.
-constexpr unsigned kStage = 120;
-// List slots per lane that the staged search keeps in LDS ([slot][lane]) until
-// the density and factor pass, which stores them to the list four at a time
-// for the whole wave (one coalesced 1 KB store per group); slots from
-// kListLds on are written to the list during the search.
+// Candidates staged per wave: the 64 particles of a wave lie, in sorted order,
+// in a few (x, y) columns of cells, each a run of consecutive lanes.  For each
+// (dx, dy) row the candidates of a run are one range of particles, from the
+// cell below the run's first to the cell above its last; the wave copies the
+// ranges of its runs into LDS with coalesced loads, and the lanes then read
+// their own spans from LDS instead of gathering from L2.  The ranges of all
+// rows are found at once, one lane per (run, row), and a row's copy is loaded
+// while the row before is scanned.  A row whose ranges exceed kStage reads
+// global memory, and so does a wave with more than kRuns runs or with a
+// particle outside the grid (whose order is not the cells').  The stage keeps
+// kCB slots of slack past kStage, so that a batch may read up to kCB - 1
+// entries past its span's end (masked out of its hits) without clamping its
+// addresses.
+constexpr unsigned kStage = 160;
+constexpr unsigned kRuns = 4;
+static_assert(kRuns * 16u == 64u, "one lane per run and row, rows padded to 16");
+// List slots per lane that the search keeps in LDS ([slot][lane]) until the
+// density and factor pass, which stores them to the list four at a time for
+// the whole wave (one coalesced 1 KB store per group); slots from kListLds on
+// are written to the list during the search.
 constexpr unsigned kListLds = 32;
 static_assert(kListLds % 4u == 0u, "LDS slots end on a group boundary");
 
@@ -504,28 +523,76 @@ __device__ inline void wave_lds_sync() {
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
+__device__ inline unsigned readlane(unsigned v, unsigned lane) {
+  return unsigned(__builtin_amdgcn_readlane(int(v), int(lane)));
+}
 
-// The staged instance holds 40 KB of LDS per block (4 blocks, 4 waves per
-// SIMD); the others are bounded to 64 VGPRs for 8 waves per SIMD.
+// The boundary terms and the results of a particle's search: list length,
+// density, viscosity coefficient, DFSPH factor (mode 1, 2) and the divergence
+// warm start (mode 2), from the sums over its list.
+__device__ inline void search_finish(const SimParams& p, const DevArrays& A, unsigned s, unsigned nn,
+                                     int with_factor, vec3 vi, float dens, float sgk, vec3 gpi,
+                                     float div) {
+  const bool ws = with_factor == 2;
+  unsigned mask = A.bmask[s];
+  while (mask) {
+    const unsigned b = __builtin_ctz(mask);
+    mask &= mask - 1u;
+    const size_t o = size_t(b) * A.cap + s;
+    float4 bk = A.bker[o];
+    dens += bk.w;
+    gpi += mk(bk.x, bk.y, bk.z);
+    if (ws) div += dot(vi - rigid_velocity(A.bnd[b], ld3(A.brec[o])), mk(bk.x, bk.y, bk.z));
+  }
+  A.nnb[s] = nn;
+  const float rho = dens * p.rho0;
+  A.density[s] = rho;
+  reinterpret_cast<float*>(A.v + s)[3] = visc_coefficient(p, rho);
+  if (with_factor) {
+    sgk += length_sqr(gpi);
+    A.alpha[s] = sgk > p.eps ? -1.0f / sgk : 0.0f;
+  }
+  if (ws) {
+    // density_change, then the warm start of the stored stiffness
+    float da = std_max(div, 0.0f);
+    if (nn < 20u) da = 0.0f;
+    const float dt = A.ctl->dt;
+    const float kv_prev = A.kappa_v[s];
+    const float kv = (da > 0.0f) ? 0.5f * std_max(kv_prev, -0.5f) / dt : 0.0f;
+    A.kappa_v[s] = kv;
+    set_kw(A, s, kv);
+  }
+}
+
+// shift of the run that holds stage slot k (runs 1, 2, 3 start at o1, o2, o3)
+__device__ inline unsigned run_shift(unsigned k, unsigned o1, unsigned o2, unsigned o3, unsigned s0,
+                                     unsigned s1, unsigned s2, unsigned s3) {
+  unsigned at = k >= o1 ? s1 : s0;
+  at = k >= o2 ? s2 : at;
+  return k >= o3 ? s3 : at;
+}
+
+// One wave per block (its LDS is its own), so that few particles spread over
+// the chip: 10.9 KB a wave, 14 waves per CU.  The tile instance keeps blocks
+// of 256 particles (its tiles') and is bounded to 64 VGPRs.
 template <bool W, bool TL>
-__global__ __launch_bounds__(256, (!W && !TL) ? 4 : 8) void k_neighbors(SceneTab T, DevArrays A,
-                                                                          int with_factor) {
-  // LDS staging and the LDS list for the gather instance without the
-  // periodic wrap (its rows are single spans); the others keep the
-  // lane-private scan
-  constexpr bool kWaveStage = !W && !TL;
-  __shared__ float4 stage_[kWaveStage ? 4 : 1][kWaveStage ? kStage + kCB : 1];
-  __shared__ unsigned list_[kWaveStage ? 4 : 1][kWaveStage ? kListLds : 1][64];
-  ALV_SCENE(T, A, s);
+__global__ __launch_bounds__(TL ? 256 : 64, TL ? 8 : 4) void k_neighbors(SceneTab T, DevArrays A,
+                                                                         int with_factor) {
+  constexpr bool kWaveStage = !TL;
+  __shared__ float4 st[kWaveStage ? kStage + kCB : 1];
+  __shared__ unsigned list_[kWaveStage ? kListLds : 1][64];
+  __shared__ int4 runs_[kWaveStage ? kRuns : 1];  // column x, y and first and last cell z
+  ALV_SCENE_PASS(T, A, s, q_, TL ? kTile : kDeep, 1u);
   // candidate positions from the block's LDS tile when it has one
   TileX tile_;
   bool tiled_ = false;
   if constexpr (TL) tiled_ = stage_x(A, s / kBlock, tile_);
   const bool live = s < p.first + p.n;
   if (!kWaveStage && !live) return;
+  const unsigned lane = threadIdx.x & 63u;
   const unsigned K = p.kmax;
   // this lane's LDS list slots: slot t at lst[t * 64]
-  unsigned* lst = &list_[kWaveStage ? threadIdx.x >> 6 : 0][0][kWaveStage ? threadIdx.x & 63u : 0];
+  unsigned* lst = &list_[0][kWaveStage ? lane : 0];
   const vec3 xi = live ? ld3(A.x[s]) : mk(0.f, 0.f, 0.f);
   int ip[3];
   cell_ipos(xi, p, ip);
@@ -584,7 +651,8 @@ __global__ __launch_bounds__(256, (!W && !TL) ? 4 : 8) void k_neighbors(SceneTab
   // branch-free and give a bit mask of hits, which are then appended in
   // ascending j.  X(j0, u) is candidate j0 + u; kClamp: X must not be read
   // past je - 1 (global memory), else reads past the span are harmless.
-  auto scan_span = [&](unsigned jb, unsigned je, auto&& X, auto clamp_tag, bool own_row) {
+  // D(x_j) is the displacement.
+  auto scan_span = [&](unsigned jb, unsigned je, auto&& X, auto&& D, auto clamp_tag, bool own_row) {
     constexpr bool kClamp = decltype(clamp_tag)::value;
     for (unsigned j0 = jb; j0 < je; j0 += kCB) {
       float4 xc[kCB];
@@ -592,10 +660,7 @@ __global__ __launch_bounds__(256, (!W && !TL) ? 4 : 8) void k_neighbors(SceneTab
       for (int u = 0; u < kCB; ++u) xc[u] = kClamp ? X(min(j0 + u, je - 1u), 0u) : X(j0, u);
       unsigned hits = 0u;
 #pragma unroll
-      for (int u = 0; u < kCB; ++u) {
-        const vec3 d = wrapd<W>(xi - ld3(xc[u]), p);
-        hits |= unsigned(length_sqr(d) < p.h2) << u;
-      }
+      for (int u = 0; u < kCB; ++u) hits |= unsigned(length_sqr(D(ld3(xc[u]))) < p.h2) << u;
       // the batch's slots past the span and, in the particle's own row, the
       // particle itself, once per batch rather than per candidate
       hits &= __builtin_amdgcn_ubfe(0xffu, 0u, min(je - j0, kCB));
@@ -622,75 +687,182 @@ __global__ __launch_bounds__(256, (!W && !TL) ? 4 : 8) void k_neighbors(SceneTab
   };
   using Clamp = std::integral_constant<bool, true>;
   using NoClamp = std::integral_constant<bool, false>;
-  // The 27 cells in the reference order (dx outer, dz inner): for each
-  // (dx, dy) row the up-to-3 cells along z are contiguous in the sorted
-  // order unless a periodic wrap splits them, so each row is 1-3 spans.
-  for (int r = 0; r < 9; ++r) {
+  auto global_x = [&](unsigned j, unsigned) { return A.x[j]; };
+  auto wrapped_d = [&](vec3 x) { return wrapd<W>(xi - x, p); };
+  // the column of row r, wrapped on periodic axes, whether it can hold a
+  // neighbour, and the cells above and below that can
+  struct Row {
+    unsigned column;
+    bool ok;
+    int dz_lo, dz_hi, raw_x, raw_y;
+  };
+  auto row_of = [&](int r) {
+    Row w;
     const int ddx = r / 3 - 1, ddy = r % 3 - 1;
     const float ex = ddx < 0 ? lo_d[0] : (ddx > 0 ? hi_d[0] : 0.0f);
     const float ey = ddy < 0 ? lo_d[1] : (ddy > 0 ? hi_d[1] : 0.0f);
     const float base = ex * ex + ey * ey;
-    const int dz_lo = base + lo_d[2] * lo_d[2] < reach2 ? -1 : 0;
-    const int dz_hi = base + hi_d[2] * hi_d[2] < reach2 ? 1 : 0;
-    int nx = ip[0] + ddx, ny = ip[1] + ddy;
-    if (p.wrap_mask & 1) nx = nx >= p.res[0] ? nx - p.res[0] : (nx < 0 ? nx + p.res[0] : nx);
-    if (p.wrap_mask & 2) ny = ny >= p.res[1] ? ny - p.res[1] : (ny < 0 ? ny + p.res[1] : ny);
-    const bool row_ok = live && base < reach2 && nx >= 0 && nx < p.res[0] && ny >= 0 &&
-                        ny < p.res[1];
-    const unsigned row = (unsigned(nx) * unsigned(p.res[1]) + unsigned(ny)) * unsigned(p.res[2]);
-    if constexpr (kWaveStage) {
-      // one span: cells nz_lo .. nz_hi of the row, clipped to the grid
-      const int z0 = max(ip[2] + dz_lo, 0), z1 = min(ip[2] + dz_hi, p.res[2] - 1);
-      unsigned jb = 0u, je = 0u;
-      if (row_ok && z0 <= z1) {
-        jb = A.cell_start[p.cell_base + row + unsigned(z0)];
-        je = A.cell_start[p.cell_base + row + unsigned(z1) + 1u];
+    w.dz_lo = base + lo_d[2] * lo_d[2] < reach2 ? -1 : 0;
+    w.dz_hi = base + hi_d[2] * hi_d[2] < reach2 ? 1 : 0;
+    int nx = w.raw_x = ip[0] + ddx, ny = w.raw_y = ip[1] + ddy;
+    if (W && (p.wrap_mask & 1)) nx = nx >= p.res[0] ? nx - p.res[0] : (nx < 0 ? nx + p.res[0] : nx);
+    if (W && (p.wrap_mask & 2)) ny = ny >= p.res[1] ? ny - p.res[1] : (ny < 0 ? ny + p.res[1] : ny);
+    w.ok = live && base < reach2 && nx >= 0 && nx < p.res[0] && ny >= 0 && ny < p.res[1];
+    w.column = p.cell_base + (unsigned(nx) * unsigned(p.res[1]) + unsigned(ny)) * unsigned(p.res[2]);
+    return w;
+  };
+  bool staged = false;
+  if constexpr (kWaveStage) {
+    // runs of lanes in one column
+    const bool in_grid = within_grid(ip, p);
+    const unsigned long long lives = __ballot(live);
+    const unsigned col = unsigned(ip[0]) * unsigned(p.res[1]) + unsigned(ip[1]);
+    const unsigned before = unsigned(__shfl_up(int(col), 1, 64));
+    const unsigned long long heads = __ballot(live && (lane == 0u || col != before));
+    const unsigned nruns = unsigned(__popcll(heads));
+    staged = __ballot(live && !in_grid) == 0ull && nruns <= kRuns && (!W || p.wrap_tight);
+    if (staged && lives != 0ull) {
+      const unsigned run = unsigned(__popcll(heads & (~0ull >> (63u - lane)))) - 1u;
+      if (live && (heads >> lane & 1ull)) {
+        // the last lane of the run: before the next head, or the last live one
+        const unsigned long long later = lane == 63u ? 0ull : heads >> (lane + 1u);
+        const unsigned last = later ? lane + unsigned(__builtin_ctzll(later))
+                                    : 63u - unsigned(__builtin_clzll(lives));
+        runs_[run] = make_int4(ip[0], ip[1], ip[2], int(last));
       }
-      unsigned lo = jb < je ? jb : ~0u, hi = jb < je ? je : 0u;
-#pragma unroll
-      for (int o = 32; o > 0; o >>= 1) {
-        lo = min(lo, unsigned(__shfl_xor(int(lo), o, 64)));
-        hi = max(hi, unsigned(__shfl_xor(int(hi), o, 64)));
-      }
-      const bool fits = hi > lo && hi - lo <= kStage;
-      float4* st = stage_[threadIdx.x >> 6];
-      wave_lds_sync();  // the previous row's reads are done
-      if (fits)
-        for (unsigned k = threadIdx.x & 63u; k < hi - lo; k += 64u) st[k] = A.x[lo + k];
       wave_lds_sync();
-      if (jb < je) {
-        if (fits)
-          scan_span(jb, je, [&](unsigned j0, unsigned u) { return st[j0 - lo + u]; }, NoClamp(),
-                    r == 4 || self_any_row);
-        else
-          scan_span(jb, je, [&](unsigned j, unsigned) { return A.x[j]; }, Clamp(),
-                    r == 4 || self_any_row);
-      }
-    } else {
-      if (!row_ok) continue;
-      unsigned span_b[3], span_e[3], nspan = 0;
-      int prev = -2;
-      for (int dz = dz_lo; dz <= dz_hi; ++dz) {
-        int nz = ip[2] + dz;
-        if (p.wrap_mask & 4) nz = nz >= p.res[2] ? nz - p.res[2] : (nz < 0 ? nz + p.res[2] : nz);
-        if (nz < 0 || nz >= p.res[2]) continue;
-        const unsigned c = p.cell_base + row + unsigned(nz);
-        if (nz == prev + 1) {
-          span_e[nspan - 1] = A.cell_start[c + 1];
-        } else {
-          span_b[nspan] = A.cell_start[c];
-          span_e[nspan] = A.cell_start[c + 1];
-          ++nspan;
+      // lane 16 g + r: the candidates of run g in row r
+      const unsigned tr = lane & 15u, tg = lane >> 4;
+      const int4 rn = runs_[min(tg, nruns - 1u)];
+      const int z_last = __shfl(ip[2], rn.w, 64);
+      unsigned start = 0u, len = 0u;
+      {
+        int nx = rn.x + int(tr) / 3 - 1, ny = rn.y + int(tr) % 3 - 1;
+        if (W && (p.wrap_mask & 1)) nx = nx >= p.res[0] ? nx - p.res[0] : (nx < 0 ? nx + p.res[0] : nx);
+        if (W && (p.wrap_mask & 2)) ny = ny >= p.res[1] ? ny - p.res[1] : (ny < 0 ? ny + p.res[1] : ny);
+        if (tr < 9u && tg < nruns && nx >= 0 && nx < p.res[0] && ny >= 0 && ny < p.res[1]) {
+          const unsigned c = p.cell_base +
+                             (unsigned(nx) * unsigned(p.res[1]) + unsigned(ny)) * unsigned(p.res[2]);
+          start = A.cell_start[c + unsigned(max(rn.z - 1, 0))];
+          len = A.cell_start[c + unsigned(min(z_last + 1, p.res[2] - 1)) + 1u] - start;
         }
-        prev = nz;
       }
-      for (unsigned q = 0; q < nspan; ++q) {
+      unsigned off = 0u;  // the run's place in the row's stage
+      for (unsigned g = 1; g < kRuns; ++g) {
+        const unsigned l = unsigned(__shfl_up(int(len), int(16u * g), 64));
+        off += tg >= g ? l : 0u;
+      }
+      const unsigned shift = start - off;  // particle index of a run's stage slot, minus the slot
+      // the lane's span in row r, and the row's stage: three slots per lane
+      struct Fetched {
+        unsigned jb, je;
+        float4 f0, f1, f2;
+      };
+      auto fetch = [&](int r) {
+        const Row w = row_of(r);
+        const int z0 = max(ip[2] + w.dz_lo, 0), z1 = min(ip[2] + w.dz_hi, p.res[2] - 1);
+        const unsigned z_b = w.ok ? w.column + unsigned(z0) : 0u, z_e = w.ok ? w.column + unsigned(z1) + 1u : 0u;
+        Fetched n;
+        n.jb = A.cell_start[z_b];  // an empty span where the row holds nothing
+        n.je = A.cell_start[z_e];
+        const unsigned total = readlane(off + len, 48u + unsigned(r));
+        const unsigned o1 = readlane(off, 16u + unsigned(r)), o2 = readlane(off, 32u + unsigned(r)),
+                       o3 = readlane(off, 48u + unsigned(r));
+        const unsigned s0 = readlane(shift, unsigned(r)), s1 = readlane(shift, 16u + unsigned(r)),
+                       s2 = readlane(shift, 32u + unsigned(r)), s3 = readlane(shift, 48u + unsigned(r));
+        // past the ranges: the particle itself
+        n.f0 = A.x[lane < total ? lane + run_shift(lane, o1, o2, o3, s0, s1, s2, s3) : s];
+        n.f1 = A.x[64u + lane < total ? 64u + lane + run_shift(64u + lane, o1, o2, o3, s0, s1, s2, s3) : s];
+        n.f2 = n.f1;
+        if (total > 128u)  // uniform
+          n.f2 = A.x[128u + lane < total ? 128u + lane + run_shift(128u + lane, o1, o2, o3, s0, s1, s2, s3) : s];
+        return n;
+      };
+      Fetched next = fetch(0);
+#pragma unroll 1
+      for (int r = 0; r < 9; ++r) {
+        const unsigned total = readlane(off + len, 48u + unsigned(r));
+        const bool fits = total <= kStage;
+        const unsigned b = next.jb, e = next.je;
+        wave_lds_sync();  // the row before has been read
+        if (fits) {
+          st[lane] = next.f0;
+          st[64u + lane] = next.f1;
+          if (lane < kStage - 128u) st[128u + lane] = next.f2;
+        }
+        wave_lds_sync();
+        const unsigned mine = unsigned(__shfl(int(shift), int((run & 3u) * 16u + unsigned(r)), 64));
+        if (r < 8) next = fetch(r + 1);
+        const bool own = r == 4;
+        if constexpr (W) {
+          // cells reached over a periodic end: x_j lies a length away, in the
+          // columns of the whole row and, along z, in the cell before the
+          // first (scanned first) or after the last (scanned last)
+          const Row w = row_of(r);
+          const float tx = w.raw_x < 0 ? -p.wrap_len[0] : (w.raw_x >= p.res[0] ? p.wrap_len[0] : 0.0f);
+          const float ty = w.raw_y < 0 ? -p.wrap_len[1] : (w.raw_y >= p.res[1] ? p.wrap_len[1] : 0.0f);
+          const bool wz = w.ok && (p.wrap_mask & 4);
+          if (wz && ip[2] + w.dz_lo < 0) {
+            const unsigned c = w.column + unsigned(p.res[2]) - 1u;
+            scan_span(A.cell_start[c], A.cell_start[c + 1u], global_x, wrapped_d, Clamp(), false);
+          }
+          auto shifted_d = [&](vec3 x) {
+            vec3 d = xi - x;
+            d.x -= tx;
+            d.y -= ty;
+            return d;
+          };
+          if (!fits)
+            scan_span(b, e, global_x, wrapped_d, Clamp(), own);
+          else if (__ballot(w.ok && (tx != 0.0f || ty != 0.0f)) != 0ull)
+            scan_span(b, e, [&](unsigned j0, unsigned u) { return st[j0 - mine + u]; }, shifted_d,
+                      NoClamp(), own);
+          else
+            scan_span(b, e, [&](unsigned j0, unsigned u) { return st[j0 - mine + u]; },
+                      [&](vec3 x) { return xi - x; }, NoClamp(), own);
+          if (wz && ip[2] + w.dz_hi >= p.res[2]) {
+            const unsigned c = w.column;
+            scan_span(A.cell_start[c], A.cell_start[c + 1u], global_x, wrapped_d, Clamp(), false);
+          }
+        } else {
+          if (fits)
+            scan_span(b, e, [&](unsigned j0, unsigned u) { return st[j0 - mine + u]; },
+                      [&](vec3 x) { return xi - x; }, NoClamp(), own);
+          else
+            scan_span(b, e, global_x, wrapped_d, Clamp(), own);
+        }
+      }
+    }
+  }
+  // The 27 cells in the reference order (dx outer, dz inner): for each
+  // (dx, dy) row the up-to-3 cells along z are contiguous in the sorted
+  // order unless a periodic wrap splits them, so each row is 1-3 spans.
+  if (!staged) {
+#pragma unroll 1
+    for (int r = 0; r < 9; ++r) {
+      const Row w = row_of(r);
+      if (!w.ok) continue;
+      unsigned b = 0u, e = 0u;  // the span being extended
+      int prev = -2;
+#pragma unroll 1
+      for (int dz = w.dz_lo; dz <= w.dz_hi + 1; ++dz) {
+        int nz = ip[2] + dz;
+        if (W && (p.wrap_mask & 4)) nz = nz >= p.res[2] ? nz - p.res[2] : (nz < 0 ? nz + p.res[2] : nz);
+        const bool use = dz <= w.dz_hi && nz >= 0 && nz < p.res[2];
+        const unsigned c = w.column + unsigned(nz);
+        if (use && nz == prev + 1) {
+          e = A.cell_start[c + 1u];
+          prev = nz;
+          continue;
+        }
         if (tiled_)
-          scan_span(span_b[q], span_e[q], [&](unsigned j, unsigned) { return tile_.X(j); },
-                    Clamp(), r == 4 || self_any_row);
+          scan_span(b, e, [&](unsigned j, unsigned) { return tile_.X(j); }, wrapped_d, Clamp(),
+                    r == 4 || self_any_row);
         else
-          scan_span(span_b[q], span_e[q], [&](unsigned j, unsigned) { return A.x[j]; },
-                    Clamp(), r == 4 || self_any_row);
+          scan_span(b, e, global_x, wrapped_d, Clamp(), r == 4 || self_any_row);
+        b = use ? A.cell_start[c] : 0u;
+        e = use ? A.cell_start[c + 1u] : 0u;
+        prev = use ? nz : -2;
       }
     }
   }
@@ -711,74 +883,55 @@ __global__ __launch_bounds__(256, (!W && !TL) ? 4 : 8) void k_neighbors(SceneTab
   // evaluation for every candidate.  The lanes walk their lists in step, so
   // the LDS slots of group q are stored for the whole wave at once.
   const bool ws = with_factor == 2;  // divergence warm start 0 on this walk
+  const bool wraps = wave_wraps<W>(xi, p);
   const vec3 vi = ws ? ld3(A.v[s]) : mk(0.f, 0.f, 0.f);
   float div = 0.0f;  // sum_j V (v_i - v_j) . gradW_ij, in list order
-  for (unsigned t0 = 0; t0 < nn; t0 += kNB) {
-    unsigned jn[kNB];
-    if (kWaveStage && t0 < kListLds) {
-      const uint4 g = make_uint4(lst[t0 * 64u], lst[(t0 + 1u) * 64u], lst[(t0 + 2u) * 64u],
-                                 lst[(t0 + 3u) * 64u]);
-      A.nbr[nbr_group(A, t0 >> 2, s)] = g;
-      jn[0] = t0 + 0 < nn ? g.x : s;
-      jn[1] = t0 + 1 < nn ? g.y : s;
-      jn[2] = t0 + 2 < nn ? g.z : s;
-      jn[3] = t0 + 3 < nn ? g.w : s;
-    } else {
-      batch_ids(A, s, nn, t0, jn);
-    }
-    float4 xj[kNB], vj[kNB];
+  auto walk = [&](auto wrap_tag) {
+    constexpr bool kWrap = decltype(wrap_tag)::value;
+    for (unsigned t0 = 0; t0 < nn; t0 += kNB) {
+      unsigned jn[kNB];
+      if (kWaveStage && t0 < kListLds) {
+        const uint4 g = make_uint4(lst[t0 * 64u], lst[(t0 + 1u) * 64u], lst[(t0 + 2u) * 64u],
+                                   lst[(t0 + 3u) * 64u]);
+        A.nbr[nbr_group(A, t0 >> 2, s)] = g;
+        jn[0] = t0 + 0 < nn ? g.x : s;
+        jn[1] = t0 + 1 < nn ? g.y : s;
+        jn[2] = t0 + 2 < nn ? g.z : s;
+        jn[3] = t0 + 3 < nn ? g.w : s;
+      } else {
+        batch_ids(A, s, nn, t0, jn);
+      }
+      float4 xj[kNB], vj[kNB];
 #pragma unroll
-    for (int u = 0; u < kNB; ++u) xj[u] = tiled_ ? tile_.X(jn[u]) : A.x[jn[u]];
-    if (ws) {
+      for (int u = 0; u < kNB; ++u) xj[u] = tiled_ ? tile_.X(jn[u]) : A.x[jn[u]];
+      if (ws) {
 #pragma unroll
-      for (int u = 0; u < kNB; ++u) vj[u] = A.v[jn[u]];
-    }
-    // An empty slot holds the particle itself (d = 0): its W term is
-    // replaced by +0 and its gradient and divergence terms are signed zeros,
-    // so every slot is added without a branch (sums that start at +0 never
-    // become -0).
+        for (int u = 0; u < kNB; ++u) vj[u] = A.v[jn[u]];
+      }
+      // An empty slot holds the particle itself (d = 0): its W term is
+      // replaced by +0 and its gradient and divergence terms are signed zeros,
+      // so every slot is added without a branch (sums that start at +0 never
+      // become -0).
 #pragma unroll
-    for (int u = 0; u < kNB; ++u) {
-      vec3 d = wrapd<W>(xi - ld3(xj[u]), p);
-      const float w = W_d2(length_sqr(d), p);
-      dens += p.vol * (t0 + u < nn ? w : 0.0f);
-      if (with_factor) {
-        const vec3 g = gradW_rn(d, p);
-        vec3 gp = (-p.vol) * g;
-        sgk += length_sqr(gp);
-        gpi -= gp;
-        if (ws) div += p.vol * dot(vi - ld3(vj[u]), g);
+      for (int u = 0; u < kNB; ++u) {
+        vec3 d = wrapd<kWrap>(xi - ld3(xj[u]), p);
+        const float w = W_d2(length_sqr(d), p);
+        dens += p.vol * (t0 + u < nn ? w : 0.0f);
+        if (with_factor) {
+          const vec3 g = gradW_rn(d, p);
+          vec3 gp = (-p.vol) * g;
+          sgk += length_sqr(gp);
+          gpi -= gp;
+          if (ws) div += p.vol * dot(vi - ld3(vj[u]), g);
+        }
       }
     }
-  }
-  unsigned mask = A.bmask[s];
-  while (mask) {
-    const unsigned b = __builtin_ctz(mask);
-    mask &= mask - 1u;
-    const size_t o = size_t(b) * A.cap + s;
-    float4 bk = A.bker[o];
-    dens += bk.w;
-    gpi += mk(bk.x, bk.y, bk.z);
-    if (ws) div += dot(vi - rigid_velocity(A.bnd[b], ld3(A.brec[o])), mk(bk.x, bk.y, bk.z));
-  }
-  A.nnb[s] = nn;
-  const float rho = dens * p.rho0;
-  A.density[s] = rho;
-  reinterpret_cast<float*>(A.v + s)[3] = visc_coefficient(p, rho);
-  if (with_factor) {
-    sgk += length_sqr(gpi);
-    A.alpha[s] = sgk > p.eps ? -1.0f / sgk : 0.0f;
-  }
-  if (ws) {
-    // density_change, then the warm start of the stored stiffness
-    float da = std_max(div, 0.0f);
-    if (nn < 20u) da = 0.0f;
-    const float dt = A.ctl->dt;
-    const float kv_prev = A.kappa_v[s];
-    const float kv = (da > 0.0f) ? 0.5f * std_max(kv_prev, -0.5f) / dt : 0.0f;
-    A.kappa_v[s] = kv;
-    set_kw(A, s, kv);
-  }
+  };
+  if (wraps)
+    walk(std::integral_constant<bool, W>());
+  else
+    walk(std::integral_constant<bool, false>());
+  search_finish(p, A, s, nn, with_factor, vi, dens, sgk, gpi, div);
 }
 
 // ---------------------------------------------------------------------------
@@ -847,18 +1000,19 @@ __device__ inline float density_change(const SimParams& p, const DevArrays& A, u
 // The value of lane Q of this lane's particle.  Every lane of the quad is
 // active where it is called, so bound_ctrl never applies; it lets the
 // compiler fold the move into the add (v_add_f32_dpp).
-template <int Q>
+template <int Q, unsigned L = kLPP>
 __device__ inline float lane_of_particle(float v) {
-  constexpr int ctl = kLPP == 4u ? Q * 0x55 : (Q | Q << 2 | (2 + Q) << 4 | (2 + Q) << 6);
+  constexpr int ctl = L == 4u ? Q * 0x55 : (Q | Q << 2 | (2 + Q) << 4 | (2 + Q) << 6);
   return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), ctl, 0xf, 0xf, true));
 }
 // acc + (the particle's lanes' t, in lane order)
+template <unsigned L = kLPP>
 __device__ inline float add_in_slot_order(float acc, float t) {
-  acc += lane_of_particle<0>(t);
-  acc += lane_of_particle<1>(t);
-  if constexpr (kLPP == 4u) {
-    acc += lane_of_particle<2>(t);
-    acc += lane_of_particle<3>(t);
+  acc += lane_of_particle<0, L>(t);
+  acc += lane_of_particle<1, L>(t);
+  if constexpr (L == 4u) {
+    acc += lane_of_particle<2, L>(t);
+    acc += lane_of_particle<3, L>(t);
   }
   return acc;
 }
@@ -884,8 +1038,9 @@ __device__ inline void lane_slots(const DevArrays& A, unsigned s, unsigned q, un
   jb = t0 + kLPP + q < nn ? jb : s;
 }
 
-// velocity_divergence over the fluid list, kLPP lanes per particle; the
-// boundary terms are added by every lane of the particle.  A slot past the
+// velocity_divergence's sum over the fluid list, kLPP lanes per particle (the
+// boundary terms follow in velocity_divergence_m, added by every lane of the
+// particle).  A slot past the
 // count holds the particle itself, whose term is an exact zero (x_i - x_i =
 // +0, so gradW is a signed zero and so is the term), so every slot's term is
 // added without a test: a sum that starts at +0 never becomes -0 under
@@ -923,6 +1078,276 @@ __device__ inline float velocity_divergence_q(const SimParams& p, const DevArray
     }
   }
   if constexpr (V) *visc = av;
+  return acc;
+}
+// ---------------------------------------------------------------------------
+// Deep form: few particles.  A pass over few particles is bound by latency:
+// with one or two lanes per particle the chip holds one or two waves per SIMD
+// (or none), and each group of four slots waits for its list load and then
+// for its gathers.  Here lane q of four takes slots 4 k + q, and the list
+// loads and then the gathers of kDeepSlots slots per lane (all neighbours of
+// most particles) are issued before any is used: two latencies per pass.
+// The terms are the other forms', added in slot order, so the sums are the
+// same bits.
+// ---------------------------------------------------------------------------
+constexpr unsigned kDeepSlots = 10;
+constexpr unsigned kDeepSure = 6;  // slots per lane evaluated without a look at the wave's counts
+// slots t0 + 4 k + q of particle s (s itself past the count); the loads do not
+// wait for the count
+__device__ inline void deep_slots(const DevArrays& A, unsigned s, unsigned q, unsigned t0,
+                                  unsigned nn, unsigned (&j)[kDeepSlots]) {
+  const unsigned* row = reinterpret_cast<const unsigned*>(A.nbr + nbr_group(A, 0u, s)) + q;
+  const unsigned last = nbr_groups(A.kmax) - 1u;
+#pragma unroll
+  for (unsigned k = 0; k < kDeepSlots; ++k) j[k] = row[min((t0 >> 2) + k, last) * 256u];
+#pragma unroll
+  for (unsigned k = 0; k < kDeepSlots; ++k) asm volatile("" : "+v"(j[k]));
+#pragma unroll
+  for (unsigned k = 0; k < kDeepSlots; ++k) j[k] = t0 + 4u * k + q < nn ? j[k] : s;
+}
+// keeps the gathers that may go unused with the others (the compiler would
+// move them behind the look at the counts, one more latency)
+__device__ inline void deep_pin(float4 (&v)[kDeepSlots]) {
+#pragma unroll
+  for (unsigned k = kDeepSure; k < kDeepSlots; ++k)
+    asm volatile("" : "+v"(v[k].x), "+v"(v[k].y), "+v"(v[k].z), "+v"(v[k].w));
+}
+// velocity_divergence_q's sums in the deep form
+template <bool W, bool V = false>
+__device__ inline float velocity_divergence_deep(const SimParams& p, const DevArrays& A,
+                                                 unsigned s, unsigned q, vec3 xi, vec3 vi,
+                                                 unsigned nn, vec3* visc = nullptr) {
+  float acc = 0.0f;
+  vec3 av = mk(0.f, 0.f, 0.f);
+  const float e2 = 0.01f * p.h2;
+  for (unsigned t0 = 0; t0 < nn; t0 += 4u * kDeepSlots) {
+    unsigned j[kDeepSlots];
+    deep_slots(A, s, q, t0, nn, j);
+    float4 xj[kDeepSlots], vj[kDeepSlots];
+#pragma unroll
+    for (unsigned k = 0; k < kDeepSlots; ++k) {
+      xj[k] = A.x[j[k]];
+      vj[k] = A.v[j[k]];
+    }
+    deep_pin(xj);
+    deep_pin(vj);
+#pragma unroll
+    for (unsigned k = 0; k < kDeepSlots; ++k) {
+      if (k >= kDeepSure && __ballot(t0 + 4u * k < nn) == 0ull) break;  // no list of the wave is so long
+      const vec3 d = wrapd<W>(xi - ld3(xj[k]), p);
+      const vec3 g = gradW_rn(d, p);
+      const vec3 u = vi - ld3(vj[k]);
+      acc = add_in_slot_order<4>(acc, p.vol * dot(u, g));
+      if constexpr (V) {
+        const vec3 w = div_rn(vj[k].w * dot(d, g), length_sqr(d) + e2) * u;
+        av.x = add_in_slot_order<4>(av.x, w.x);
+        av.y = add_in_slot_order<4>(av.y, w.y);
+        av.z = add_in_slot_order<4>(av.z, w.z);
+      }
+    }
+  }
+  if constexpr (V) *visc = av;
+  return acc;
+}
+// ---------------------------------------------------------------------------
+// The search for few particles: four lanes per particle, 16 particles per
+// wave.  With a lane per particle a wave works through about 7,800
+// instructions one after another, and few particles are few waves: 16,384
+// leave three of four SIMDs idle.  Here the lanes of a particle test four
+// consecutive candidates at a time, read from L2 (one line per quad); a hit's
+// place in the list is the hits before it in the quad and the steps before,
+// so the list is the same.  It then serves the density phase from LDS, in the
+// deep form of the passes: the lanes evaluate four consecutive slots and add
+// the terms in slot order.
+// ---------------------------------------------------------------------------
+constexpr unsigned kQuadList = 64;  // list slots kept in LDS; later ones go to the list at once
+// bit q set when lane q of the quad hits
+__device__ inline unsigned quad_bits(bool hit, unsigned q) {
+  int b = hit ? int(1u << q) : 0;
+  b |= __builtin_amdgcn_mov_dpp(b, 0xB1, 0xf, 0xf, true);  // lanes 1 0 3 2
+  b |= __builtin_amdgcn_mov_dpp(b, 0x4E, 0xf, 0xf, true);  // lanes 2 3 0 1
+  return unsigned(b);
+}
+template <bool W>
+__global__ __launch_bounds__(64) void k_neighbors_quad(SceneTab T, DevArrays A, int with_factor) {
+  __shared__ unsigned list_[kQuadList][16];
+  const unsigned qblk_ = xcd_block();
+  const unsigned lane = threadIdx.x, q = lane & 3u;
+  const unsigned s = qblk_ * 16u + (lane >> 2);
+  const unsigned scene_ = T.blk_scene[qblk_ / (kBlock / 16u)];
+  const SimParams p = T.par[scene_];
+  A.ctl += scene_;
+  A.bnd += p.bnd_base;
+  if (s >= p.first + p.n) return;  // whole quads
+  const unsigned K = p.kmax;
+  unsigned* lst = &list_[0][lane >> 2];
+  const vec3 xi = ld3(A.x[s]);
+  int ip[3];
+  cell_ipos(xi, p, ip);
+  // see k_neighbors
+  float lo_d[3], hi_d[3];
+  float mag = p.h;
+  {
+    const float xs[3] = {xi.x, xi.y, xi.z};
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+      const float c0 = float(ip[a] + p.off[a]) * p.h;
+      lo_d[a] = xs[a] - c0;
+      hi_d[a] = c0 + p.h - xs[a];
+      mag = fmaxf(mag, fabsf(xs[a]) + p.h);
+    }
+  }
+  const float reach = p.h * 1.00005f + mag * 9.5367431640625e-7f;
+  const float reach2 = reach * reach;
+  unsigned cnt = 0;  // the same in the four lanes
+  unsigned* row_list = reinterpret_cast<unsigned*>(A.nbr + nbr_group(A, 0u, s));
+  const unsigned below = (1u << q) - 1u;
+  auto put = [&](unsigned slot, unsigned j) {
+    if (slot < kQuadList)
+      lst[slot * 16u] = j;
+    else
+      row_list[(slot >> 2) * 256u + (slot & 3u)] = j;
+  };
+  // candidates [b, e), 16 per particle and round: all loads of a round first
+  auto scan = [&](unsigned b, unsigned e, auto&& D) {
+    for (unsigned j0 = b; j0 < e; j0 += 16u) {
+      float4 xc[4];
+#pragma unroll
+      for (unsigned u = 0; u < 4u; ++u) xc[u] = A.x[min(j0 + 4u * u + q, e - 1u)];
+#pragma unroll
+      for (unsigned u = 0; u < 4u; ++u) {
+        const unsigned j = j0 + 4u * u + q;
+        const bool hit = length_sqr(D(ld3(xc[u]))) < p.h2 && j < e && j != s;
+        const unsigned bits = quad_bits(hit, q);
+        const unsigned at = cnt + unsigned(__builtin_popcount(bits & below));
+        cnt += unsigned(__builtin_popcount(bits));
+        // at most K slots; the last one keeps the latest neighbour
+        if (hit && (at + 1u < K || (bits >> q) == 1u)) put(min(at, K - 1u), j);
+      }
+    }
+  };
+  const bool wraps = wave_wraps<W>(xi, p);
+  const bool plain = !wraps && __ballot(!within_grid(ip, p)) == 0ull;
+  if (plain) {
+    // no cell lies over a periodic end: one span per row, all found first
+    unsigned jb[9], je[9];
+#pragma unroll
+    for (int r = 0; r < 9; ++r) {
+      const int ddx = r / 3 - 1, ddy = r % 3 - 1;
+      const float ex = ddx < 0 ? lo_d[0] : (ddx > 0 ? hi_d[0] : 0.0f);
+      const float ey = ddy < 0 ? lo_d[1] : (ddy > 0 ? hi_d[1] : 0.0f);
+      const float base = ex * ex + ey * ey;
+      const int nx = ip[0] + ddx, ny = ip[1] + ddy;
+      const int z0 = max(ip[2] + (base + lo_d[2] * lo_d[2] < reach2 ? -1 : 0), 0);
+      const int z1 = min(ip[2] + (base + hi_d[2] * hi_d[2] < reach2 ? 1 : 0), p.res[2] - 1);
+      const bool ok = base < reach2 && nx >= 0 && nx < p.res[0] && ny >= 0 && ny < p.res[1];
+      const unsigned c =
+          p.cell_base + (unsigned(ok ? nx : 0) * unsigned(p.res[1]) + unsigned(ok ? ny : 0)) * unsigned(p.res[2]);
+      jb[r] = A.cell_start[c + unsigned(z0)];
+      je[r] = A.cell_start[c + unsigned(z1) + 1u];
+      if (!ok) jb[r] = je[r] = 0u;
+    }
+#pragma unroll
+    for (int r = 0; r < 9; ++r) scan(jb[r], je[r], [&](vec3 x) { return xi - x; });
+  } else {
+#pragma unroll 1
+    for (int r = 0; r < 9; ++r) {
+      const int ddx = r / 3 - 1, ddy = r % 3 - 1;
+      const float ex = ddx < 0 ? lo_d[0] : (ddx > 0 ? hi_d[0] : 0.0f);
+      const float ey = ddy < 0 ? lo_d[1] : (ddy > 0 ? hi_d[1] : 0.0f);
+      const float base = ex * ex + ey * ey;
+      const int dz_lo = base + lo_d[2] * lo_d[2] < reach2 ? -1 : 0;
+      const int dz_hi = base + hi_d[2] * hi_d[2] < reach2 ? 1 : 0;
+      int nx = ip[0] + ddx, ny = ip[1] + ddy;
+      if (W && (p.wrap_mask & 1)) nx = nx >= p.res[0] ? nx - p.res[0] : (nx < 0 ? nx + p.res[0] : nx);
+      if (W && (p.wrap_mask & 2)) ny = ny >= p.res[1] ? ny - p.res[1] : (ny < 0 ? ny + p.res[1] : ny);
+      if (!(base < reach2 && nx >= 0 && nx < p.res[0] && ny >= 0 && ny < p.res[1])) continue;
+      const unsigned column =
+          p.cell_base + (unsigned(nx) * unsigned(p.res[1]) + unsigned(ny)) * unsigned(p.res[2]);
+#pragma unroll 1
+      for (int dz = dz_lo; dz <= dz_hi; ++dz) {
+        int nz = ip[2] + dz;
+        if (W && (p.wrap_mask & 4)) nz = nz >= p.res[2] ? nz - p.res[2] : (nz < 0 ? nz + p.res[2] : nz);
+        if (nz < 0 || nz >= p.res[2]) continue;
+        scan(A.cell_start[column + unsigned(nz)], A.cell_start[column + unsigned(nz) + 1u],
+             [&](vec3 x) { return wrapd<W>(xi - x, p); });
+      }
+    }
+  }
+  if (cnt > K) A.anomaly[2] = 1u;
+  const unsigned nn = min(cnt, K);
+  const bool ws = with_factor == 2;
+  const vec3 vi = ws ? ld3(A.v[s]) : mk(0.f, 0.f, 0.f);
+  float dens = p.vol * p.w0;
+  float sgk = 0.0f, div = 0.0f;
+  vec3 gpi = mk(0.f, 0.f, 0.f);
+  __threadfence_block();  // the lanes' list writes, LDS and global
+  const unsigned last = nbr_groups(A.kmax) - 1u;
+  auto walk = [&](auto wrap_tag) {
+    constexpr bool kWrap = decltype(wrap_tag)::value;
+    constexpr unsigned kRound = 5;  // slots per lane in flight
+    for (unsigned t0 = 0; t0 < nn; t0 += 4u * kRound) {
+      unsigned j[kRound];
+#pragma unroll
+      for (unsigned k = 0; k < kRound; ++k) {
+        const unsigned t = t0 + 4u * k + q, g = min(t >> 2, last);
+        if (t < kQuadList) {
+          j[k] = lst[t * 16u];
+          if (t0 + 4u * k < nn) row_list[g * 256u + q] = j[k];
+        } else {
+          j[k] = row_list[g * 256u + q];
+        }
+        j[k] = t < nn ? j[k] : s;
+      }
+      float4 xj[kRound], vj[kRound];
+#pragma unroll
+      for (unsigned k = 0; k < kRound; ++k) xj[k] = A.x[j[k]];
+      if (ws) {
+#pragma unroll
+        for (unsigned k = 0; k < kRound; ++k) vj[k] = A.v[j[k]];
+      }
+#pragma unroll
+      for (unsigned k = 0; k < kRound; ++k) {
+        const vec3 d = wrapd<kWrap>(xi - ld3(xj[k]), p);
+        const float w = W_d2(length_sqr(d), p);
+        dens = add_in_slot_order<4>(dens, p.vol * (t0 + 4u * k + q < nn ? w : 0.0f));
+        if (with_factor) {
+          const vec3 g = gradW_rn(d, p);
+          const vec3 gp = (-p.vol) * g;
+          sgk = add_in_slot_order<4>(sgk, length_sqr(gp));
+          gpi.x = add_in_slot_order<4>(gpi.x, -gp.x);
+          gpi.y = add_in_slot_order<4>(gpi.y, -gp.y);
+          gpi.z = add_in_slot_order<4>(gpi.z, -gp.z);
+          if (ws) div = add_in_slot_order<4>(div, p.vol * dot(vi - ld3(vj[k]), g));
+        }
+      }
+    }
+  };
+  if (wraps)
+    walk(std::integral_constant<bool, W>());
+  else
+    walk(std::integral_constant<bool, false>());
+  if (q == 0u) search_finish(p, A, s, nn, with_factor, vi, dens, sgk, gpi, div);
+}
+
+// lanes per particle of the density-change and of the stiffness passes
+constexpr unsigned change_lanes(int M) { return M == kTile ? 1u : (M == kDeep ? kDeepLanes : kLPP); }
+constexpr unsigned stiffness_lanes(int M) { return M == kDeep ? kDeepLanes : 1u; }
+constexpr unsigned pass_threads(int M, unsigned lanes) {
+  return (M == kDeep ? kDeepBlock : kBlock) * lanes;
+}
+// velocity_divergence_q in mode M's form (kGather or kDeep)
+template <bool W, int M, bool V = false>
+__device__ inline float velocity_divergence_m(const SimParams& p, const DevArrays& A, unsigned s,
+                                              unsigned q, vec3 xi, vec3 vi, unsigned nn,
+                                              vec3* visc = nullptr) {
+  float acc;
+  if (wave_wraps<W>(xi, p))
+    acc = M == kDeep ? velocity_divergence_deep<W, V>(p, A, s, q, xi, vi, nn, visc)
+                     : velocity_divergence_q<W, V>(p, A, s, q, xi, vi, nn, visc);
+  else
+    acc = M == kDeep ? velocity_divergence_deep<false, V>(p, A, s, q, xi, vi, nn, visc)
+                     : velocity_divergence_q<false, V>(p, A, s, q, xi, vi, nn, visc);
   unsigned mask = A.bmask[s];
   while (mask) {
     const unsigned b = __builtin_ctz(mask);
@@ -934,29 +1359,29 @@ __device__ inline float velocity_divergence_q(const SimParams& p, const DevArray
   }
   return acc;
 }
-template <bool W>
+template <bool W, int M>
 __device__ inline float density_change_q(const SimParams& p, const DevArrays& A, unsigned s,
                                          unsigned q) {
   const vec3 xi = ld3(A.x[s]), vi = ld3(A.v[s]);
   const unsigned nn = A.nnb[s];
-  float da = velocity_divergence_q<W>(p, A, s, q, xi, vi, nn);
+  float da = velocity_divergence_m<W, M>(p, A, s, q, xi, vi, nn);
   da = std_max(da, 0.0f);
   if (nn < 20u) da = 0.0f;
   return da;
 }
 
 // The density-change passes run with one lane per particle when they read
-// neighbours from the block's LDS tile (TL), else with kLPP lanes per
+// neighbours from the block's LDS tile, else with change_lanes(M) lanes per
 // particle (global gathers); q is the lane within the particle's lanes.
-template <bool W, bool TL>
+template <bool W, int M>
 __device__ inline float pass_density_change(const SimParams& p, const DevArrays& A,
                                             unsigned s, unsigned q, bool tiled,
                                             const TileXV& tile) {
-  if constexpr (TL)
+  if constexpr (M == kTile)
     return tiled ? density_change<W>(p, A, s, tile)
                  : density_change<W>(p, A, s, GlobalXV{A.x, A.v});
   else
-    return density_change_q<W>(p, A, s, q);
+    return density_change_q<W, M>(p, A, s, q);
 }
 
 // compute_density_adv (runner.hpp:3493-3523)
@@ -968,16 +1393,16 @@ __device__ inline float density_adv(const SimParams& p, const DevArrays& A, unsi
   float delta = velocity_divergence<W>(p, A, s, xi, vi, nn, src);
   return std_max(A.density[s] / p.rho0 + dt * delta, 1.0f);
 }
-template <bool W, bool TL>
+template <bool W, int M>
 __device__ inline float pass_density_adv(const SimParams& p, const DevArrays& A, unsigned s,
                                          unsigned q, float dt, bool tiled, const TileXV& tile) {
-  if constexpr (TL) {
+  if constexpr (M == kTile) {
     return tiled ? density_adv<W>(p, A, s, dt, tile)
                  : density_adv<W>(p, A, s, dt, GlobalXV{A.x, A.v});
   } else {
     const vec3 xi = ld3(A.x[s]), vi = ld3(A.v[s]);
     const unsigned nn = A.nnb[s];
-    float delta = velocity_divergence_q<W>(p, A, s, q, xi, vi, nn);
+    float delta = velocity_divergence_m<W, M>(p, A, s, q, xi, vi, nn);
     return std_max(A.density[s] / p.rho0 + dt * delta, 1.0f);
   }
 }
@@ -1000,26 +1425,58 @@ __device__ inline vec3 stiffness_dv(const SimParams& p, const DevArrays& A, unsi
 #pragma unroll
     for (int u = 0; u < kNB; ++u) xj[u] = src.X(j[u]);
     // Every slot's term is computed and a skipped one (past the count, or
-    // |k_i + k_j| <= eps, where the reference adds nothing) is replaced by
-    // +0, which leaves the sum's bits unchanged; the gradient's division is
-    // the correctly rounded div_rn (the same bits as the IEEE division).
+    // |k_i + k_j| <= eps, where the reference adds nothing) has its
+    // coefficient replaced by 0: a signed zero, which leaves the sum's bits
+    // unchanged.
 #pragma unroll
     for (int u = 0; u < kNB; ++u) {
       const float k_sum = k_i + xj[u].w;
       const bool use = t0 + u < nn && fabsf(k_sum) > p.eps;
       const vec3 d = wrapd<W>(xi - ld3(xj[u]), p);
-      vec3 term;
       if (kDivergenceForm)
-        term = (dt * k_sum) * ((-p.vol) * gradW_rn(d, p));
+        dv -= (use ? dt * k_sum : 0.0f) * ((-p.vol) * gradW_rn(d, p));
       else
-        term = ((dt * k_sum) * p.vol) * gradW_rn(d, p);
-      term = use ? term : mk(0.f, 0.f, 0.f);
-      if (kDivergenceForm)
-        dv -= term;
-      else
-        dv += term;
+        dv += (use ? (dt * k_sum) * p.vol : 0.0f) * gradW_rn(d, p);
     }
   }
+  return dv;
+}
+// the same sum in the deep form (kDeepLanes lanes per particle, every one of
+// which holds it)
+template <bool W, bool kDivergenceForm>
+__device__ inline vec3 stiffness_dv_deep(const SimParams& p, const DevArrays& A, unsigned s,
+                                         unsigned q, float k_i, float dt) {
+  const vec3 xi = ld3(A.x[s]);
+  const unsigned nn = A.nnb[s];
+  vec3 dv = mk(0.f, 0.f, 0.f);
+  for (unsigned t0 = 0; t0 < nn; t0 += 4u * kDeepSlots) {
+    unsigned j[kDeepSlots];
+    deep_slots(A, s, q, t0, nn, j);
+    float4 xj[kDeepSlots];
+#pragma unroll
+    for (unsigned k = 0; k < kDeepSlots; ++k) xj[k] = A.x[j[k]];
+    deep_pin(xj);
+#pragma unroll
+    for (unsigned k = 0; k < kDeepSlots; ++k) {
+      if (k >= kDeepSure && __ballot(t0 + 4u * k < nn) == 0ull) break;
+      const float k_sum = k_i + xj[k].w;
+      const bool use = t0 + 4u * k + q < nn && fabsf(k_sum) > p.eps;
+      const vec3 d = wrapd<W>(xi - ld3(xj[k]), p);
+      vec3 term;
+      if (kDivergenceForm)
+        term = -((use ? dt * k_sum : 0.0f) * ((-p.vol) * gradW_rn(d, p)));  // dv -= term
+      else
+        term = (use ? (dt * k_sum) * p.vol : 0.0f) * gradW_rn(d, p);
+      dv.x = add_in_slot_order<4>(dv.x, term.x);
+      dv.y = add_in_slot_order<4>(dv.y, term.y);
+      dv.z = add_in_slot_order<4>(dv.z, term.z);
+    }
+  }
+  return dv;
+}
+// and its boundary terms, with the bodies' reactions (one lane per particle)
+__device__ inline vec3 stiffness_boundary(const SimParams& p, const DevArrays& A, unsigned s,
+                                          float k_i, float dt, vec3 dv) {
   if (fabsf(k_i) > p.eps) {
     unsigned mask = A.bmask[s];
     while (mask) {
@@ -1069,6 +1526,26 @@ __device__ inline vec3 viscosity_sum(const SimParams& p, const DevArrays& A, uns
     }
   }
   return da;
+}
+
+// A stiffness pass in mode M: its velocity change, added to v by the
+// particle's first lane.
+template <bool W, bool kDivergenceForm, int M>
+__device__ inline void pass_stiffness(const SimParams& p, DevArrays& A, unsigned s, unsigned q,
+                                      float k_i, float dt, bool tiled, const TileX& tile) {
+  vec3 dv;
+  const bool wraps = wave_wraps<W>(ld3(A.x[s]), p);
+  if constexpr (M == kDeep)
+    dv = wraps ? stiffness_dv_deep<W, kDivergenceForm>(p, A, s, q, k_i, dt)
+               : stiffness_dv_deep<false, kDivergenceForm>(p, A, s, q, k_i, dt);
+  else if constexpr (M == kTile)
+    dv = tiled ? stiffness_dv<W, kDivergenceForm>(p, A, s, k_i, tile, dt)
+               : stiffness_dv<W, kDivergenceForm>(p, A, s, k_i, GlobalX{A.x}, dt);
+  else
+    dv = wraps ? stiffness_dv<W, kDivergenceForm>(p, A, s, k_i, GlobalX{A.x}, dt)
+               : stiffness_dv<false, kDivergenceForm>(p, A, s, k_i, GlobalX{A.x}, dt);
+  if (q != 0u) return;
+  add_v(A, s, stiffness_boundary(p, A, s, k_i, dt, dv));
 }
 
 __device__ inline void orthogonal_vectors(vec3 n, vec3& t1, vec3& t2) {
@@ -1148,7 +1625,7 @@ __device__ inline float viscosity_finish(const SimParams& p, const DevArrays& A,
 // list, the fluid part of the viscosity (viscosity_sum's terms in its order;
 // from an LDS tile, one lane per particle, the two sums walk the list
 // separately).  xi and vi are the particle's position and velocity.
-template <bool W, bool TL>
+template <bool W, int M>
 __device__ inline float pass_density_change_visc(const SimParams& p, const DevArrays& A,
                                                  unsigned s, unsigned q, bool tiled,
                                                  const TileXV& tile, vec3& xi, vec3& vi,
@@ -1157,7 +1634,7 @@ __device__ inline float pass_density_change_visc(const SimParams& p, const DevAr
   vi = ld3(A.v[s]);
   const unsigned nn = A.nnb[s];
   float da;
-  if constexpr (TL) {
+  if constexpr (M == kTile) {
     if (tiled) {
       da = velocity_divergence<W>(p, A, s, xi, vi, nn, tile);
       visc = viscosity_sum<W>(p, A, s, xi, vi, nn, tile);
@@ -1167,7 +1644,7 @@ __device__ inline float pass_density_change_visc(const SimParams& p, const DevAr
       visc = viscosity_sum<W>(p, A, s, xi, vi, nn, g);
     }
   } else {
-    da = velocity_divergence_q<W, true>(p, A, s, q, xi, vi, nn, &visc);
+    da = velocity_divergence_m<W, M, true>(p, A, s, q, xi, vi, nn, &visc);
   }
   da = std_max(da, 0.0f);
   if (nn < 20u) da = 0.0f;
@@ -1176,15 +1653,15 @@ __device__ inline float pass_density_change_visc(const SimParams& p, const DevAr
 
 // warm_start_divergence_solve_0 (runner.hpp:3230-3250)
 // F: also record the warm-start features of the particle
-template <bool W, bool F, bool TL>
-__global__ __launch_bounds__(TL ? kBlock : kLPP * kBlock) void k_ws_div0(SceneTab T, DevArrays A) {
-  ALV_SCENE_PASS(T, A, s, q, TL);
+template <bool W, bool F, int M>
+__global__ __launch_bounds__(pass_threads(M, change_lanes(M))) void k_ws_div0(SceneTab T, DevArrays A) {
+  ALV_SCENE_PASS(T, A, s, q, M, change_lanes(M));
   TileXV tile_;
   bool tiled_ = false;
-  if constexpr (TL) tiled_ = stage_xv(A, s / kBlock, tile_);
+  if constexpr (M == kTile) tiled_ = stage_xv(A, s / kBlock, tile_);
   if (s >= p.first + p.n) return;
   const float dt = A.ctl->dt;
-  const float dadv = pass_density_change<W, TL>(p, A, s, q, tiled_, tile_);
+  const float dadv = pass_density_change<W, M>(p, A, s, q, tiled_, tile_);
   if (q != 0u) return;
   const float kv_prev = A.kappa_v[s];
   const float kv = (dadv > 0.0f) ? 0.5f * std_max(kv_prev, -0.5f) / dt : 0.0f;
@@ -1276,17 +1753,15 @@ __global__ __launch_bounds__(256) void k_ws_div0_learned(SceneTab T, DevArrays A
 }
 
 // warm_start_divergence_solve_1 (runner.hpp:3252-3295)
-template <bool W, bool TL>
-__global__ __launch_bounds__(256) void k_ws_div1(SceneTab T, DevArrays A) {
-  ALV_SCENE(T, A, s);
+template <bool W, int M>
+__global__ __launch_bounds__(pass_threads(M, stiffness_lanes(M))) void k_ws_div1(SceneTab T, DevArrays A) {
+  ALV_SCENE_PASS(T, A, s, q, M, stiffness_lanes(M));
   TileX tk_;
   bool tiled_ = false;
-  if constexpr (TL) tiled_ = stage_x(A, s / kBlock, tk_);
+  if constexpr (M == kTile) tiled_ = stage_x(A, s / kBlock, tk_);
   if (s >= p.first + p.n) return;
   const float dt = A.ctl->dt;
-  vec3 dv = tiled_ ? stiffness_dv<W, true>(p, A, s, A.kappa_v[s], tk_, dt)
-                   : stiffness_dv<W, true>(p, A, s, A.kappa_v[s], GlobalX{A.x}, dt);
-  add_v(A, s, dv);
+  pass_stiffness<W, true, M>(p, A, s, q, A.kappa_v[s], dt, tiled_, tk_);
 }
 // compute_velocity_of_density_change (runner.hpp:3297-3314); also stores the
 // first iteration's stiffness k = rho_adv * alpha.  The density-change passes
@@ -1299,21 +1774,21 @@ __global__ __launch_bounds__(256) void k_ws_div1(SceneTab T, DevArrays A) {
 // the iteration count stays below the minimum and the maximum.  Both passes
 // are bounded to 64 VGPRs (8 waves per SIMD); unbounded, the viscosity terms
 // take 66 (7 waves per SIMD), which measured 2 % slower.
-template <bool W, bool TL>
-__global__ __launch_bounds__(TL ? kBlock : kLPP * kBlock, 8) void k_vel_density_change(SceneTab T, DevArrays A) {
-  __shared__ float lds[kLPP * kBlock / 64];
-  ALV_SCENE_PASS(T, A, s, q, TL);
+template <bool W, int M>
+__global__ __launch_bounds__(pass_threads(M, change_lanes(M)), M == kDeep ? 3 : 8) void k_vel_density_change(SceneTab T, DevArrays A) {
+  __shared__ float lds[pass_threads(M, change_lanes(M)) / 64];
+  ALV_SCENE_PASS(T, A, s, q, M, change_lanes(M));
   TileXV tile_;
   bool tiled_ = false;
-  if constexpr (TL) tiled_ = stage_xv(A, s / kBlock, tile_);
+  if constexpr (M == kTile) tiled_ = stage_xv(A, s / kBlock, tile_);
   const float dt = A.ctl->dt;
   const bool last = A.ctl->div_done != 0u;  // the same for the whole block
   float cfl = -FLT_MAX;
   if (s < p.first + p.n) {
     vec3 xi, vi, visc;
     const float dadv =
-        last ? pass_density_change_visc<W, TL>(p, A, s, q, tiled_, tile_, xi, vi, visc)
-             : pass_density_change<W, TL>(p, A, s, q, tiled_, tile_);
+        last ? pass_density_change_visc<W, M>(p, A, s, q, tiled_, tile_, xi, vi, visc)
+             : pass_density_change<W, M>(p, A, s, q, tiled_, tile_);
     if (q == 0u) {
       A.rho_adv[s] = dadv;
       float inv_dt = 1.0f / dt;
@@ -1331,33 +1806,31 @@ __global__ __launch_bounds__(TL ? kBlock : kLPP * kBlock, 8) void k_vel_density_
   }
 }
 // divergence_solve_iteration (runner.hpp:3316-3363)
-template <bool W, bool TL>
-__global__ __launch_bounds__(256) void k_div_iter(SceneTab T, DevArrays A) {
-  ALV_SCENE(T, A, s);
+template <bool W, int M>
+__global__ __launch_bounds__(pass_threads(M, stiffness_lanes(M))) void k_div_iter(SceneTab T, DevArrays A) {
+  ALV_SCENE_PASS(T, A, s, q, M, stiffness_lanes(M));
   if (A.ctl->div_done) return;
   TileX tk_;
   bool tiled_ = false;
-  if constexpr (TL) tiled_ = stage_x(A, s / kBlock, tk_);
+  if constexpr (M == kTile) tiled_ = stage_x(A, s / kBlock, tk_);
   if (s >= p.first + p.n) return;
   const float dt = A.ctl->dt;
   const float k_i = A.kfac[s];
-  A.kappa_v[s] += k_i;
-  vec3 dv = tiled_ ? stiffness_dv<W, true>(p, A, s, k_i, tk_, dt)
-                   : stiffness_dv<W, true>(p, A, s, k_i, GlobalX{A.x}, dt);
-  add_v(A, s, dv);
+  if (q == 0u) A.kappa_v[s] += k_i;
+  pass_stiffness<W, true, M>(p, A, s, q, k_i, dt, tiled_, tk_);
 }
 // compute_divergence_solve_density_error (runner.hpp:3396-3410) + FP64
 // partial sums of the residual
 // (and the viscosity, as k_vel_density_change)
-template <bool W, bool TL>
-__global__ __launch_bounds__(TL ? kBlock : kLPP * kBlock, 8) void k_div_err(SceneTab T, DevArrays A) {
-  __shared__ double lds[kLPP * kBlock / 64];
-  __shared__ float ldsm[kLPP * kBlock / 64];
-  ALV_SCENE_PASS(T, A, s, q, TL);
+template <bool W, int M>
+__global__ __launch_bounds__(pass_threads(M, change_lanes(M)), M == kDeep ? 3 : 8) void k_div_err(SceneTab T, DevArrays A) {
+  __shared__ double lds[pass_threads(M, change_lanes(M)) / 64];
+  __shared__ float ldsm[pass_threads(M, change_lanes(M)) / 64];
+  ALV_SCENE_PASS(T, A, s, q, M, change_lanes(M));
   if (A.ctl->div_done) return;
   TileXV tile_;
   bool tiled_ = false;
-  if constexpr (TL) tiled_ = stage_xv(A, s / kBlock, tile_);
+  if constexpr (M == kTile) tiled_ = stage_xv(A, s / kBlock, tile_);
   const float dt = A.ctl->dt;
   // k_div_finalize continues while the count it reaches is below both bounds
   const unsigned it = A.ctl->div_iter + 1u;
@@ -1367,8 +1840,8 @@ __global__ __launch_bounds__(TL ? kBlock : kLPP * kBlock, 8) void k_div_err(Scen
   if (s < p.first + p.n) {
     vec3 xi, vi, visc;
     const float dadv =
-        last ? pass_density_change_visc<W, TL>(p, A, s, q, tiled_, tile_, xi, vi, visc)
-             : pass_density_change<W, TL>(p, A, s, q, tiled_, tile_);
+        last ? pass_density_change_visc<W, M>(p, A, s, q, tiled_, tile_, xi, vi, visc)
+             : pass_density_change<W, M>(p, A, s, q, tiled_, tile_);
     if (q == 0u) {
       A.rho_adv[s] = dadv;
       const float k = dadv * A.alpha[s];
@@ -1385,13 +1858,14 @@ __global__ __launch_bounds__(TL ? kBlock : kLPP * kBlock, 8) void k_div_err(Scen
     if (threadIdx.x == 0) A.fpartials[qblk_] = m;
   }
 }
-__global__ __launch_bounds__(kFinBlock) void k_div_finalize(SceneTab T, DevArrays A) {
+__global__ __launch_bounds__(kFinBlock) void k_div_finalize(SceneTab T, DevArrays A, unsigned parts) {
   __shared__ double lds[kFinBlock / 64];
   ALV_SCENE_BLOCK(T, A);
   StepCtl* ctl = A.ctl;
   if (ctl->div_done) return;
   double part = 0.0;
-  for (unsigned b = blk_begin + threadIdx.x; b < blk_end; b += blockDim.x) part += A.partials[b];
+  for (unsigned b = blk_begin * parts + threadIdx.x; b < blk_end * parts; b += blockDim.x)
+    part += A.partials[b];
   double t = block_sum_d(part, lds);
   if (threadIdx.x == 0) {
     float mean = float(t / double(p.n));
@@ -1454,11 +1928,12 @@ __global__ __launch_bounds__(256) void k_viscosity(SceneTab T, DevArrays A) {
 }
 
 // Solver::update_dt (solver.hpp:153-169) on the device.
-__global__ __launch_bounds__(kFinBlock) void k_update_dt(SceneTab T, DevArrays A) {
+__global__ __launch_bounds__(kFinBlock) void k_update_dt(SceneTab T, DevArrays A, unsigned parts) {
   __shared__ float lds[kFinBlock / 64];
   ALV_SCENE_BLOCK(T, A);
   float m = -FLT_MAX;
-  for (unsigned b = blk_begin + threadIdx.x; b < blk_end; b += blockDim.x) m = std_max(m, A.fpartials[b]);
+  for (unsigned b = blk_begin * parts + threadIdx.x; b < blk_end * parts; b += blockDim.x)
+    m = std_max(m, A.fpartials[b]);
   float pm = block_max_f(m, lds);
   if (threadIdx.x == 0) {
     StepCtl* ctl = A.ctl;
@@ -1508,15 +1983,15 @@ __global__ __launch_bounds__(256) void k_integrate_np(SceneTab T, DevArrays A, i
 
 // warm_start_pressure_solve0 (runner.hpp:3430-3450)
 // L: learned warm start (prediction from k_ws_div0_learned)
-template <bool W, bool L, bool TL>
-__global__ __launch_bounds__(TL ? kBlock : kLPP * kBlock) void k_ws_p0(SceneTab T, DevArrays A) {
-  ALV_SCENE_PASS(T, A, s, q, TL);
+template <bool W, bool L, int M>
+__global__ __launch_bounds__(pass_threads(M, change_lanes(M))) void k_ws_p0(SceneTab T, DevArrays A) {
+  ALV_SCENE_PASS(T, A, s, q, M, change_lanes(M));
   TileXV tile_;
   bool tiled_ = false;
-  if constexpr (TL) tiled_ = stage_xv(A, s / kBlock, tile_);
+  if constexpr (M == kTile) tiled_ = stage_xv(A, s / kBlock, tile_);
   if (s >= p.first + p.n) return;
   const float dt = A.ctl->dt;
-  const float dadv = pass_density_adv<W, TL>(p, A, s, q, dt, tiled_, tile_);
+  const float dadv = pass_density_adv<W, M>(p, A, s, q, dt, tiled_, tile_);
   if (q != 0u) return;
   float k = (dadv > 1.0f) ? (0.5f * std_max(A.kappa[s], -0.00025f) / (dt * dt)) : 0.0f;
   if (L && dadv > 1.0f) {
@@ -1527,28 +2002,26 @@ __global__ __launch_bounds__(TL ? kBlock : kLPP * kBlock) void k_ws_p0(SceneTab 
   set_kw(A, s, k);
 }
 // warm_start_pressure_solve1 (runner.hpp:3452-3491)
-template <bool W, bool TL>
-__global__ __launch_bounds__(256) void k_ws_p1(SceneTab T, DevArrays A) {
-  ALV_SCENE(T, A, s);
+template <bool W, int M>
+__global__ __launch_bounds__(pass_threads(M, stiffness_lanes(M))) void k_ws_p1(SceneTab T, DevArrays A) {
+  ALV_SCENE_PASS(T, A, s, q, M, stiffness_lanes(M));
   TileX tk_;
   bool tiled_ = false;
-  if constexpr (TL) tiled_ = stage_x(A, s / kBlock, tk_);
+  if constexpr (M == kTile) tiled_ = stage_x(A, s / kBlock, tk_);
   if (s >= p.first + p.n) return;
   const float dt = A.ctl->dt;
-  vec3 dv = tiled_ ? stiffness_dv<W, false>(p, A, s, A.kappa[s], tk_, dt)
-                   : stiffness_dv<W, false>(p, A, s, A.kappa[s], GlobalX{A.x}, dt);
-  add_v(A, s, dv);
+  pass_stiffness<W, false, M>(p, A, s, q, A.kappa[s], dt, tiled_, tk_);
 }
 // compute_rho_adv (runner.hpp:3525-3541); stores k = (rho_adv - 1) * alpha
-template <bool W, bool TL>
-__global__ __launch_bounds__(TL ? kBlock : kLPP * kBlock) void k_rho_adv(SceneTab T, DevArrays A) {
-  ALV_SCENE_PASS(T, A, s, q, TL);
+template <bool W, int M>
+__global__ __launch_bounds__(pass_threads(M, change_lanes(M))) void k_rho_adv(SceneTab T, DevArrays A) {
+  ALV_SCENE_PASS(T, A, s, q, M, change_lanes(M));
   TileXV tile_;
   bool tiled_ = false;
-  if constexpr (TL) tiled_ = stage_xv(A, s / kBlock, tile_);
+  if constexpr (M == kTile) tiled_ = stage_xv(A, s / kBlock, tile_);
   if (s >= p.first + p.n) return;
   const float dt = A.ctl->dt;
-  const float dadv = pass_density_adv<W, TL>(p, A, s, q, dt, tiled_, tile_);
+  const float dadv = pass_density_adv<W, M>(p, A, s, q, dt, tiled_, tile_);
   if (q != 0u) return;
   A.rho_adv[s] = dadv;
   float alpha = A.alpha[s] * (1.0f / (dt * dt));
@@ -1558,35 +2031,33 @@ __global__ __launch_bounds__(TL ? kBlock : kLPP * kBlock) void k_rho_adv(SceneTa
   set_kw(A, s, k);
 }
 // pressure_solve_iteration (runner.hpp:3543-3588)
-template <bool W, bool TL>
-__global__ __launch_bounds__(256) void k_p_iter(SceneTab T, DevArrays A) {
-  ALV_SCENE(T, A, s);
+template <bool W, int M>
+__global__ __launch_bounds__(pass_threads(M, stiffness_lanes(M))) void k_p_iter(SceneTab T, DevArrays A) {
+  ALV_SCENE_PASS(T, A, s, q, M, stiffness_lanes(M));
   if (A.ctl->dens_done) return;
   TileX tk_;
   bool tiled_ = false;
-  if constexpr (TL) tiled_ = stage_x(A, s / kBlock, tk_);
+  if constexpr (M == kTile) tiled_ = stage_x(A, s / kBlock, tk_);
   if (s >= p.first + p.n) return;
   const float dt = A.ctl->dt;
   const float k_i = A.kfac[s];
-  A.kappa[s] += k_i;
-  vec3 dv = tiled_ ? stiffness_dv<W, false>(p, A, s, k_i, tk_, dt)
-                   : stiffness_dv<W, false>(p, A, s, k_i, GlobalX{A.x}, dt);
-  add_v(A, s, dv);
+  if (q == 0u) A.kappa[s] += k_i;
+  pass_stiffness<W, false, M>(p, A, s, q, k_i, dt, tiled_, tk_);
 }
 // compute_pressure_solve_density_error (runner.hpp:3590-3604) + FP64
 // partial sums of (rho_adv - 1)
-template <bool W, bool TL>
-__global__ __launch_bounds__(TL ? kBlock : kLPP * kBlock) void k_p_err(SceneTab T, DevArrays A) {
-  __shared__ double lds[kLPP * kBlock / 64];
-  ALV_SCENE_PASS(T, A, s, q, TL);
+template <bool W, int M>
+__global__ __launch_bounds__(pass_threads(M, change_lanes(M))) void k_p_err(SceneTab T, DevArrays A) {
+  __shared__ double lds[pass_threads(M, change_lanes(M)) / 64];
+  ALV_SCENE_PASS(T, A, s, q, M, change_lanes(M));
   if (A.ctl->dens_done) return;
   TileXV tile_;
   bool tiled_ = false;
-  if constexpr (TL) tiled_ = stage_xv(A, s / kBlock, tile_);
+  if constexpr (M == kTile) tiled_ = stage_xv(A, s / kBlock, tile_);
   const float dt = A.ctl->dt;
   double part = 0.0;
   if (s < p.first + p.n) {
-    const float dadv = pass_density_adv<W, TL>(p, A, s, q, dt, tiled_, tile_);
+    const float dadv = pass_density_adv<W, M>(p, A, s, q, dt, tiled_, tile_);
     if (q == 0u) {
       A.rho_adv[s] = dadv;
       const float k = (dadv - 1.0f) * A.alpha[s];
@@ -1598,13 +2069,14 @@ __global__ __launch_bounds__(TL ? kBlock : kLPP * kBlock) void k_p_err(SceneTab 
   double t = block_sum_d(part, lds);
   if (threadIdx.x == 0) A.partials[qblk_] = t;
 }
-__global__ __launch_bounds__(kFinBlock) void k_p_finalize(SceneTab T, DevArrays A) {
+__global__ __launch_bounds__(kFinBlock) void k_p_finalize(SceneTab T, DevArrays A, unsigned parts) {
   __shared__ double lds[kFinBlock / 64];
   ALV_SCENE_BLOCK(T, A);
   StepCtl* ctl = A.ctl;
   if (ctl->dens_done) return;
   double part = 0.0;
-  for (unsigned b = blk_begin + threadIdx.x; b < blk_end; b += blockDim.x) part += A.partials[b];
+  for (unsigned b = blk_begin * parts + threadIdx.x; b < blk_end * parts; b += blockDim.x)
+    part += A.partials[b];
   double t = block_sum_d(part, lds);
   if (threadIdx.x == 0) {
     float mean = float(t / double(p.n));
@@ -1637,14 +2109,14 @@ __global__ __launch_bounds__(256) void k_df_finish(SceneTab T, DevArrays A, int 
 
 // compute_velocity_of_density_change (runner.hpp:3297-3314), the density
 // change sum alone (no stiffness factor update): rho_adv <- rho_dot.
-template <bool W, bool TL>
-__global__ __launch_bounds__(TL ? kBlock : kLPP * kBlock) void k_density_change(SceneTab T, DevArrays A) {
-  ALV_SCENE_PASS(T, A, s, q, TL);
+template <bool W, int M>
+__global__ __launch_bounds__(pass_threads(M, change_lanes(M))) void k_density_change(SceneTab T, DevArrays A) {
+  ALV_SCENE_PASS(T, A, s, q, M, change_lanes(M));
   TileXV tile_;
   bool tiled_ = false;
-  if constexpr (TL) tiled_ = stage_xv(A, s / kBlock, tile_);
+  if constexpr (M == kTile) tiled_ = stage_xv(A, s / kBlock, tile_);
   if (s >= p.first + p.n) return;
-  const float dadv = pass_density_change<W, TL>(p, A, s, q, tiled_, tile_);
+  const float dadv = pass_density_change<W, M>(p, A, s, q, tiled_, tile_);
   if (q == 0u) A.rho_adv[s] = dadv;
 }
 
@@ -1704,7 +2176,7 @@ __global__ __launch_bounds__(256) void k_ii_predict0(SceneTab T, DevArrays A) {
     for (int u = 0; u < kNB; ++u) {
       if (t0 + u < nn) {
         vec3 xixj = wrapd<W>(xi - ld3(xj[u]), p);
-        d -= (p.vol / dens2) * (gradW(xixj, p));
+        d -= (p.vol / dens2) * gradW(xixj, p);
       }
     }
   }
@@ -1796,7 +2268,7 @@ __global__ __launch_bounds__(256) void k_ii_iter0(SceneTab T, DevArrays A) {
         vec3 xixj = wrapd<W>(xi - ld3(xj[u]), p);
         float dj = djs[u];
         float dj2 = dj * dj;
-        acc -= (p.vol / dj2 * lpj[u]) * (gradW(xixj, p));
+        acc -= (p.vol / dj2 * lpj[u]) * gradW(xixj, p);
       }
     }
   }
@@ -1915,7 +2387,7 @@ __global__ __launch_bounds__(256) void k_ii_pressure_accel(SceneTab T, DevArrays
         float dj = djs[u];
         float dj2 = dj * dj;
         float dpj = pj[u] / dj2;
-        ai -= (p.mass * (dpi + dpj)) * (gradW(xixj, p));
+        ai -= (p.mass * (dpi + dpj)) * gradW(xixj, p);
       }
     }
   }
@@ -2580,36 +3052,25 @@ KernelProfiler* g_profiler = nullptr;
                          __VA_ARGS__);                                            \
     if (g_profiler) g_profiler->end(#kernel, s);                                  \
   } while (0)
-// density-change passes (ALV_SCENE_PASS): one block per particle block, of
-// 256 threads for the tile instance and kLPP * 256 for the others
-#define ALV_PASS_BLOCK(tiled) dim3((tiled) ? kBlock : kLPP * kBlock)
-#define ALV_LAUNCH_WTP(kernel, L, s, ...)                                         \
+// neighbour passes (ALV_SCENE_PASS) in the form of the launch: LANES is
+// change_lanes or stiffness_lanes; KERNEL(W, M) names the instance
+#define ALV_LAUNCH_FORM(KERNEL, W, M, LANES, L, s, ...)                           \
+  hipLaunchKernelGGL((KERNEL(W, M)), dim3((L).pblocks * ((M) == kDeep ? kBlock / kDeepBlock : 1u)), \
+                     dim3(pass_threads(M, LANES(M))), 0, s, (L).T, __VA_ARGS__)
+#define ALV_LAUNCH_PASS(name, KERNEL, LANES, L, s, ...)                           \
   do {                                                                            \
-    if (g_profiler) g_profiler->begin(#kernel, s);                                \
-    if ((L).p0.wrap_mask)                                                         \
-      hipLaunchKernelGGL((kernel<true, false>), dim3((L).pblocks), ALV_PASS_BLOCK(false), 0, s, \
-                         (L).T, __VA_ARGS__);                                     \
+    if (g_profiler) g_profiler->begin(name, s);                                   \
+    if ((L).deep && (L).p0.wrap_mask)                                             \
+      ALV_LAUNCH_FORM(KERNEL, true, kDeep, LANES, L, s, __VA_ARGS__);             \
+    else if ((L).deep)                                                            \
+      ALV_LAUNCH_FORM(KERNEL, false, kDeep, LANES, L, s, __VA_ARGS__);            \
+    else if ((L).p0.wrap_mask)                                                    \
+      ALV_LAUNCH_FORM(KERNEL, true, kGather, LANES, L, s, __VA_ARGS__);           \
     else if ((L).tiles)                                                           \
-      hipLaunchKernelGGL((kernel<false, true>), dim3((L).pblocks), ALV_PASS_BLOCK(true), 0, s, \
-                         (L).T, __VA_ARGS__);                                     \
+      ALV_LAUNCH_FORM(KERNEL, false, kTile, LANES, L, s, __VA_ARGS__);            \
     else                                                                          \
-      hipLaunchKernelGGL((kernel<false, false>), dim3((L).pblocks), ALV_PASS_BLOCK(false), 0, s, \
-                         (L).T, __VA_ARGS__);                                     \
-    if (g_profiler) g_profiler->end(#kernel, s);                                  \
-  } while (0)
-#define ALV_LAUNCH_W2TP(kernel, flag, L, s, ...)                                  \
-  do {                                                                            \
-    if (g_profiler) g_profiler->begin(#kernel, s);                                \
-    if ((L).p0.wrap_mask)                                                         \
-      hipLaunchKernelGGL((kernel<true, flag, false>), dim3((L).pblocks), ALV_PASS_BLOCK(false), 0, \
-                         s, (L).T, __VA_ARGS__);                                  \
-    else if ((L).tiles)                                                           \
-      hipLaunchKernelGGL((kernel<false, flag, true>), dim3((L).pblocks), ALV_PASS_BLOCK(true), 0, \
-                         s, (L).T, __VA_ARGS__);                                  \
-    else                                                                          \
-      hipLaunchKernelGGL((kernel<false, flag, false>), dim3((L).pblocks), ALV_PASS_BLOCK(false), \
-                         0, s, (L).T, __VA_ARGS__);                               \
-    if (g_profiler) g_profiler->end(#kernel, s);                                  \
+      ALV_LAUNCH_FORM(KERNEL, false, kGather, LANES, L, s, __VA_ARGS__);          \
+    if (g_profiler) g_profiler->end(name, s);                                     \
   } while (0)
 #define ALV_LAUNCH_W2T(kernel, flag, L, s, ...)                                   \
   do {                                                                            \
@@ -2706,8 +3167,39 @@ void launch_gather_boundary(const Launch& L, const DevArrays& A, int kind, hipSt
   ALV_LAUNCH(k_gather_boundary, L, s, A, kind);
 }
 void launch_neighbors(const Launch& L, const DevArrays& A, int with_factor, hipStream_t s) {
-  ALV_LAUNCH_WT(k_neighbors, L, s, A, with_factor);
+  if (g_profiler) g_profiler->begin("k_neighbors", s);
+  if (L.quad && L.p0.wrap_mask)
+    hipLaunchKernelGGL(k_neighbors_quad<true>, dim3(L.pblocks * (kBlock / 16u)), dim3(64), 0, s, L.T,
+                       A, with_factor);
+  else if (L.quad)
+    hipLaunchKernelGGL(k_neighbors_quad<false>, dim3(L.pblocks * (kBlock / 16u)), dim3(64), 0, s,
+                       L.T, A, with_factor);
+  else if (L.p0.wrap_mask)
+    hipLaunchKernelGGL((k_neighbors<true, false>), dim3(L.pblocks * (kBlock / 64u)), dim3(64), 0, s,
+                       L.T, A, with_factor);
+  else if (L.tiles)
+    hipLaunchKernelGGL((k_neighbors<false, true>), dim3(L.pblocks), dim3(kBlock), 0, s, L.T, A,
+                       with_factor);
+  else
+    hipLaunchKernelGGL((k_neighbors<false, false>), dim3(L.pblocks * (kBlock / 64u)), dim3(64), 0, s,
+                       L.T, A, with_factor);
+  if (g_profiler) g_profiler->end("k_neighbors", s);
 }
+// instances of the neighbour passes
+#define K_WS_DIV0_LOG(W, M) k_ws_div0<W, true, M>
+#define K_WS_DIV0(W, M) k_ws_div0<W, false, M>
+#define K_WS_DIV1(W, M) k_ws_div1<W, M>
+#define K_VEL_DENSITY_CHANGE(W, M) k_vel_density_change<W, M>
+#define K_DIV_ITER(W, M) k_div_iter<W, M>
+#define K_DIV_ERR(W, M) k_div_err<W, M>
+#define K_WS_P0_LEARNED(W, M) k_ws_p0<W, true, M>
+#define K_WS_P0(W, M) k_ws_p0<W, false, M>
+#define K_WS_P1(W, M) k_ws_p1<W, M>
+#define K_RHO_ADV(W, M) k_rho_adv<W, M>
+#define K_P_ITER(W, M) k_p_iter<W, M>
+#define K_P_ERR(W, M) k_p_err<W, M>
+#define K_DENSITY_CHANGE(W, M) k_density_change<W, M>
+
 void launch_df_warm_start_div(const Launch& L, const DevArrays& A, hipStream_t s,
                               int features, const MlpDev* net, int net_divergence, int fused) {
   if (!fused) {  // else warm start 0 ran in the neighbour search (mode 2)
@@ -2716,23 +3208,23 @@ void launch_df_warm_start_div(const Launch& L, const DevArrays& A, hipStream_t s
     else if (net)
       ALV_LAUNCH_W2(k_ws_div0_learned, false, L, s, A, *net, net_divergence);
     else if (features)
-      ALV_LAUNCH_W2TP(k_ws_div0, true, L, s, A);
+      ALV_LAUNCH_PASS("k_ws_div0", K_WS_DIV0_LOG, change_lanes, L, s, A);
     else
-      ALV_LAUNCH_W2TP(k_ws_div0, false, L, s, A);
+      ALV_LAUNCH_PASS("k_ws_div0", K_WS_DIV0, change_lanes, L, s, A);
   }
-  ALV_LAUNCH_WT(k_ws_div1, L, s, A);
-  ALV_LAUNCH_WTP(k_vel_density_change, L, s, A);
+  ALV_LAUNCH_PASS("k_ws_div1", K_WS_DIV1, stiffness_lanes, L, s, A);
+  ALV_LAUNCH_PASS("k_vel_density_change", K_VEL_DENSITY_CHANGE, change_lanes, L, s, A);
 }
 void launch_df_div_iteration(const Launch& L, const DevArrays& A, hipStream_t s) {
-  ALV_LAUNCH_WT(k_div_iter, L, s, A);
-  ALV_LAUNCH_WTP(k_div_err, L, s, A);
-  ALV_LAUNCH_FIN(k_div_finalize, L, s, A);
+  ALV_LAUNCH_PASS("k_div_iter", K_DIV_ITER, stiffness_lanes, L, s, A);
+  ALV_LAUNCH_PASS("k_div_err", K_DIV_ERR, change_lanes, L, s, A);
+  ALV_LAUNCH_FIN(k_div_finalize, L, s, A, parts_per_block(L));
 }
 void launch_df_viscosity(const Launch& L, const DevArrays& A, hipStream_t s) {
   ALV_LAUNCH_WT(k_viscosity, L, s, A);
 }
-void launch_update_dt(const Launch& L, const DevArrays& A, hipStream_t s) {
-  ALV_LAUNCH_FIN(k_update_dt, L, s, A);
+void launch_update_dt(const Launch& L, const DevArrays& A, int pass_parts, hipStream_t s) {
+  ALV_LAUNCH_FIN(k_update_dt, L, s, A, pass_parts ? parts_per_block(L) : 1u);
 }
 void launch_df_integrate_np(const Launch& L, const DevArrays& A, int fin, hipStream_t s) {
   ALV_LAUNCH(k_integrate_np, L, s, A, fin);
@@ -2740,16 +3232,16 @@ void launch_df_integrate_np(const Launch& L, const DevArrays& A, int fin, hipStr
 void launch_df_warm_start_dens(const Launch& L, const DevArrays& A, hipStream_t s,
                                int learned) {
   if (learned)
-    ALV_LAUNCH_W2TP(k_ws_p0, true, L, s, A);
+    ALV_LAUNCH_PASS("k_ws_p0", K_WS_P0_LEARNED, change_lanes, L, s, A);
   else
-    ALV_LAUNCH_W2TP(k_ws_p0, false, L, s, A);
-  ALV_LAUNCH_WT(k_ws_p1, L, s, A);
-  ALV_LAUNCH_WTP(k_rho_adv, L, s, A);
+    ALV_LAUNCH_PASS("k_ws_p0", K_WS_P0, change_lanes, L, s, A);
+  ALV_LAUNCH_PASS("k_ws_p1", K_WS_P1, stiffness_lanes, L, s, A);
+  ALV_LAUNCH_PASS("k_rho_adv", K_RHO_ADV, change_lanes, L, s, A);
 }
 void launch_df_dens_iteration(const Launch& L, const DevArrays& A, hipStream_t s) {
-  ALV_LAUNCH_WT(k_p_iter, L, s, A);
-  ALV_LAUNCH_WTP(k_p_err, L, s, A);
-  ALV_LAUNCH_FIN(k_p_finalize, L, s, A);
+  ALV_LAUNCH_PASS("k_p_iter", K_P_ITER, stiffness_lanes, L, s, A);
+  ALV_LAUNCH_PASS("k_p_err", K_P_ERR, change_lanes, L, s, A);
+  ALV_LAUNCH_FIN(k_p_finalize, L, s, A, parts_per_block(L));
 }
 void launch_df_finish(const Launch& L, const DevArrays& A, int dens_finish, hipStream_t s) {
   ALV_LAUNCH_W(k_df_finish, L, s, A, dens_finish);
@@ -2759,7 +3251,7 @@ void launch_export_pairs(const Launch& L, const DevArrays& A, float* x, float* y
   ALV_LAUNCH(k_export_pairs, L, s, A, x, y);
 }
 void launch_density_change(const Launch& L, const DevArrays& A, hipStream_t s) {
-  ALV_LAUNCH_WTP(k_density_change, L, s, A);
+  ALV_LAUNCH_PASS("k_density_change", K_DENSITY_CHANGE, change_lanes, L, s, A);
 }
 void launch_integrate_velocity(const Launch& L, const DevArrays& A, float dt, hipStream_t s) {
   ALV_LAUNCH_W(k_integrate_velocity, L, s, A, dt);
@@ -2835,7 +3327,7 @@ __global__ __launch_bounds__(256) void k_check_math(SimParams p, int op, const f
     case 3: r = W_d2(x, p); break;
     case 4: r = rcp_rn(x); break;
     case 5: r = div_rn(x, b[i]); break;
-    default: break;
+        default: break;
   }
   out[i] = r;
 }

@@ -25,6 +25,8 @@ struct SimParams {
   // periodic wrap (set_wrap_length, constants.hpp:130-136); bit a = axis a
   int wrap_mask;
   float wrap_len[3], wrap_min[3], wrap_max[3];
+  // every periodic axis is filled exactly by five cells or more, from -len/2
+  int wrap_tight;
   // neighbour grid (Consti, constants.hpp:40-49)
   int res[3], off[3];
   unsigned kmax, cell_cap, num_cells;

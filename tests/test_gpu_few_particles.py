@@ -1,0 +1,77 @@
+"""The kernel forms for few particles (deep passes, four-lane search) and the
+staged search where they can go wrong: particle counts around the waves' and
+the blocks' edges, lists at and past their cap and past the slots kept in LDS,
+periodic boxes that the cells fill exactly and ones they do not, and counts on
+both sides of the forms' limits, one step against the oracle from a
+synchronised state.  Lists are compared bit for bit, fields within the
+per-step tolerance (the sums are the oracle's in its order)."""
+import numpy as np
+import pytest
+
+from alluvion_amd import scenes
+from gpu_sync import compare_fields, oracle_for, sync
+
+pytestmark = pytest.mark.gpu
+
+
+def cloud(n, cells, seed, wrap=None, kmax=64, margin=0, density=1.0):
+    """n random particles in a box of cells[a] cells (h = 0.01), optionally
+    periodic on the axes of `wrap`, with `margin` cells of grid around it."""
+    rng = np.random.default_rng(seed)
+    length = np.array(cells) * 0.01
+    x = ((rng.random((n, 3)) - 0.5) * length * 0.999999).astype(np.float32)
+    v = rng.uniform(-0.5, 0.5, (n, 3)).astype(np.float32)
+    w = tuple(float(length[a]) if wrap and wrap[a] else 0.0 for a in range(3))
+    return scenes.Scene(
+        name="cloud", x=x, v=v, gravity=(0.0, -9.81, 0.0), wrap_length=w, max_num_neighbors=kmax,
+        max_num_particles_per_cell=512,
+        grid_offset=tuple(-(c // 2) - margin for c in cells),
+        grid_res=tuple(c + 2 * margin for c in cells), boundaries=[],
+        max_divergence_solve=3, max_density_solve=4)
+
+
+def step_matches(sc, kind="df"):
+    dp, pile, solver, _, _ = scenes.build_solver(sc, kind)
+    orc = oracle_for(sc, dp, [], kind=kind)
+    solver.update_particle_neighbors()
+    orc.update_particle_neighbors()
+    ids, cnt = solver.get_neighbors()
+    oids, ocnt = orc.neighbors()
+    np.testing.assert_array_equal(cnt[:sc.n], ocnt[:sc.n])
+    mask = np.arange(sc.max_num_neighbors)[None, :] < ocnt[:sc.n, None]
+    np.testing.assert_array_equal(np.where(mask, ids[:sc.n], 0), np.where(mask, oids[:sc.n], 0))
+    sync(dp, solver, pile, orc, kind=kind)
+    solver.step()
+    orc.step()
+    assert solver.num_density_solve == orc.report()["num_density_solve"]
+    compare_fields(dp, solver, orc, kind=kind, tag=str((sc.n, kind)))
+
+
+@pytest.mark.parametrize("n", [1, 15, 17, 63, 65, 255, 257, 1000])
+def test_counts_around_waves_and_blocks(n):
+    step_matches(cloud(n, (4, 4, 4), n))
+
+
+@pytest.mark.parametrize("kmax", [7, 30, 40, 64, 90])
+def test_list_caps(kmax):
+    # mean list length about 60: caps below, at and above the slots in LDS
+    step_matches(cloud(900, (4, 4, 4), 3, kmax=kmax))
+
+
+@pytest.mark.parametrize("cells,wrap,margin", [
+    ((6, 8, 5), (True, True, True), 0),
+    ((6, 4, 6), (True, True, True), 0),  # an axis of four cells: the general wrap
+    ((6, 8, 6), (True, False, True), 0),
+    ((8, 6, 6), (False, True, False), 0),
+    ((6, 6, 8), (True, True, True), 1),  # the grid is larger than the box
+])
+@pytest.mark.parametrize("kind", ["df", "ii", "i"])
+def test_periodic_boxes(cells, wrap, margin, kind):
+    n = int(8 * np.prod(cells)) - 3
+    step_matches(cloud(n, cells, 5, wrap=wrap, margin=margin), kind)
+
+
+@pytest.mark.parametrize("wrap", [None, (True, True, True)])
+@pytest.mark.parametrize("n", [81920, 81921, 98304, 98305])
+def test_both_sides_of_the_limits(n, wrap):
+    step_matches(cloud(n, (22, 24, 20), 7, wrap=wrap))
