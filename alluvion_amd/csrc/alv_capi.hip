@@ -2709,7 +2709,7 @@ int alv_node_positions(const float dmin[3], const unsigned res[3], const float c
 
 int alv_check_math(const alv_const* cn, int op, const float* a, const float* b, float* out,
                    size_t n) {
-  if (!cn || op < 0 || op > 6) return fail(ALV_ERR_ARG, "bad argument");
+  if (!cn || op < 0 || op > 10) return fail(ALV_ERR_ARG, "bad argument");
   if (n && (!a || !out || ((op == 1 || op == 5) && !b)))
     return fail(ALV_ERR_ARG, "null argument");
   if (!n) return ALV_OK;

@@ -162,7 +162,54 @@ __device__ inline float gradW_scale(vec3 d, const SimParams& p) {
   return p.l * scale;
 }
 __device__ inline vec3 gradW(vec3 d, const SimParams& p) { return gradW_scale<false>(d, p) * d; }
-__device__ inline vec3 gradW_rn(vec3 d, const SimParams& p) { return gradW_scale<true>(d, p) * d; }
+
+// --- the same for a listed pair (|d|^2 < h^2) --------------------------------
+// Root and reciprocal of a pair's distance, both correctly rounded, from one
+// hardware reciprocal square root y (within one ulp) of x = |d|^2: s = RN(x y)
+// is within two ulp of the root, the remainder x - s^2 is exact with one fused
+// multiply-add and r = RN(s + (x - s^2) y / 2) is the root; y is also within
+// 1.5 ulp of 1/r, and one Newton step gives its reciprocal.  Checked on the
+// CPU for every significand and every estimate within one ulp: the root
+// misses for one (significand, estimate) pair, the reciprocal for nine; of
+// these the hardware gives only the estimate 2^-k for r = 2^k (1 - 2^-24)
+// (checked on the GPU for every significand), where rr is one ulp low; a
+// quotient by that r still rounds correctly unless the dividend is a power of
+// two.  Seven instructions with one transcendental where sqrt_rn and rcp_rn
+// take twelve with two.  x is raised to 2^-96 (a pair at distance 0: q is then
+// 2^-48 / h and the kernel values are those of q = 0).
+struct PairRoot {
+  float r, rr;
+};
+__device__ inline PairRoot pair_root(float x) {
+  x = fmaxf(x, 0x1p-96f);
+  const float y = __builtin_amdgcn_rsqf(x);
+  const float s = x * y;
+  PairRoot o;
+  o.r = __builtin_fmaf(__builtin_fmaf(-s, s, x), 0.5f * y, s);
+  o.rr = __builtin_fmaf(__builtin_fmaf(-o.r, y, 1.0f), y, y);
+  return o;
+}
+// gradW_scale for r = |d| <= h: the branch chooses dividend and divisor
+// before one division ((1 - q)(q - 1) = -(1 - q)^2 exactly).
+__device__ inline float grad_scale_pair(float r2, const SimParams& p) {
+  const PairRoot o = pair_root(r2);
+  const float q = div_known(o.r, p.h, p.inv_h);
+  const float conj = 1.0f - q;
+  const bool in = q <= 0.5f;
+  const float n = in ? q * 3.0f - 2.0f : -(conj * conj);
+  return p.l * div_known(n, in ? p.h : o.r, in ? p.inv_h : o.rr);
+}
+__device__ inline vec3 grad_pair(vec3 d, const SimParams& p) {
+  return grad_scale_pair(length_sqr(d), p) * d;
+}
+// W_d2 for r2 < h^2
+__device__ inline float W_pair(float r2, const SimParams& p) {
+  const float q = div_known(pair_root(r2).r, p.h, p.inv_h);
+  const float conj = 1.0f - q;
+  const float inner = (6.0f * q - 6.0f) * div_known(r2, p.h2, p.inv_h2) + 1.0f;
+  const float outer = 2.0f * conj * conj * conj;
+  return (q <= 0.5f ? inner : outer) * p.k;
+}
 
 // --- quaternion rotation (q = x, y, z, w) -----------------------------------
 __host__ __device__ inline vec3 rotate(vec3 v, float4 q) {

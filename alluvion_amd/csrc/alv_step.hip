@@ -915,10 +915,10 @@ __global__ __launch_bounds__(TL ? 256 : 64, TL ? 8 : 4) void k_neighbors(SceneTa
 #pragma unroll
       for (int u = 0; u < kNB; ++u) {
         vec3 d = wrapd<kWrap>(xi - ld3(xj[u]), p);
-        const float w = W_d2(length_sqr(d), p);
+        const float w = W_pair(length_sqr(d), p);
         dens += p.vol * (t0 + u < nn ? w : 0.0f);
         if (with_factor) {
-          const vec3 g = gradW_rn(d, p);
+          const vec3 g = grad_pair(d, p);
           vec3 gp = (-p.vol) * g;
           sgk += length_sqr(gp);
           gpi -= gp;
@@ -1061,7 +1061,7 @@ __device__ inline float velocity_divergence_q(const SimParams& p, const DevArray
     lane_slots(A, s, q, t0, nn, ja, jb);
     const float4 xa = A.x[ja], va = A.v[ja], xb = A.x[jb], vb = A.v[jb];
     const vec3 da = wrapd<W>(xi - ld3(xa), p), db = wrapd<W>(xi - ld3(xb), p);
-    const vec3 ga = gradW_rn(da, p), gb = gradW_rn(db, p);
+    const vec3 ga = grad_pair(da, p), gb = grad_pair(db, p);
     const vec3 ua = vi - ld3(va), ub = vi - ld3(vb);
     acc = add_in_slot_order(acc, p.vol * dot(ua, ga));
     acc = add_in_slot_order(acc, p.vol * dot(ub, gb));
@@ -1135,7 +1135,7 @@ __device__ inline float velocity_divergence_deep(const SimParams& p, const DevAr
     for (unsigned k = 0; k < kDeepSlots; ++k) {
       if (k >= kDeepSure && __ballot(t0 + 4u * k < nn) == 0ull) break;  // no list of the wave is so long
       const vec3 d = wrapd<W>(xi - ld3(xj[k]), p);
-      const vec3 g = gradW_rn(d, p);
+      const vec3 g = grad_pair(d, p);
       const vec3 u = vi - ld3(vj[k]);
       acc = add_in_slot_order<4>(acc, p.vol * dot(u, g));
       if constexpr (V) {
@@ -1309,10 +1309,10 @@ __global__ __launch_bounds__(64) void k_neighbors_quad(SceneTab T, DevArrays A, 
 #pragma unroll
       for (unsigned k = 0; k < kRound; ++k) {
         const vec3 d = wrapd<kWrap>(xi - ld3(xj[k]), p);
-        const float w = W_d2(length_sqr(d), p);
+        const float w = W_pair(length_sqr(d), p);
         dens = add_in_slot_order<4>(dens, p.vol * (t0 + 4u * k + q < nn ? w : 0.0f));
         if (with_factor) {
-          const vec3 g = gradW_rn(d, p);
+          const vec3 g = grad_pair(d, p);
           const vec3 gp = (-p.vol) * g;
           sgk = add_in_slot_order<4>(sgk, length_sqr(gp));
           gpi.x = add_in_slot_order<4>(gpi.x, -gp.x);
@@ -1434,9 +1434,9 @@ __device__ inline vec3 stiffness_dv(const SimParams& p, const DevArrays& A, unsi
       const bool use = t0 + u < nn && fabsf(k_sum) > p.eps;
       const vec3 d = wrapd<W>(xi - ld3(xj[u]), p);
       if (kDivergenceForm)
-        dv -= (use ? dt * k_sum : 0.0f) * ((-p.vol) * gradW_rn(d, p));
+        dv -= (use ? dt * k_sum : 0.0f) * ((-p.vol) * grad_pair(d, p));
       else
-        dv += (use ? (dt * k_sum) * p.vol : 0.0f) * gradW_rn(d, p);
+        dv += (use ? (dt * k_sum) * p.vol : 0.0f) * grad_pair(d, p);
     }
   }
   return dv;
@@ -1464,9 +1464,9 @@ __device__ inline vec3 stiffness_dv_deep(const SimParams& p, const DevArrays& A,
       const vec3 d = wrapd<W>(xi - ld3(xj[k]), p);
       vec3 term;
       if (kDivergenceForm)
-        term = -((use ? dt * k_sum : 0.0f) * ((-p.vol) * gradW_rn(d, p)));  // dv -= term
+        term = -((use ? dt * k_sum : 0.0f) * ((-p.vol) * grad_pair(d, p)));  // dv -= term
       else
-        term = (use ? (dt * k_sum) * p.vol : 0.0f) * gradW_rn(d, p);
+        term = (use ? (dt * k_sum) * p.vol : 0.0f) * grad_pair(d, p);
       dv.x = add_in_slot_order<4>(dv.x, term.x);
       dv.y = add_in_slot_order<4>(dv.y, term.y);
       dv.z = add_in_slot_order<4>(dv.z, term.z);
@@ -1520,7 +1520,7 @@ __device__ inline vec3 viscosity_sum(const SimParams& p, const DevArrays& A, uns
 #pragma unroll
     for (int u = 0; u < kNB; ++u) {
       vec3 xixj = wrapd<W>(xi - ld3(xj[u]), p);
-      da += div_rn(vj[u].w * dot(xixj, gradW_rn(xixj, p)),
+      da += div_rn(vj[u].w * dot(xixj, grad_pair(xixj, p)),
                    length_sqr(xixj) + 0.01f * p.h2) *
             (vi - ld3(vj[u]));
     }
@@ -2176,7 +2176,7 @@ __global__ __launch_bounds__(256) void k_ii_predict0(SceneTab T, DevArrays A) {
     for (int u = 0; u < kNB; ++u) {
       if (t0 + u < nn) {
         vec3 xixj = wrapd<W>(xi - ld3(xj[u]), p);
-        d -= (p.vol / dens2) * gradW(xixj, p);
+        d -= (p.vol / dens2) * grad_pair(xixj, p);
       }
     }
   }
@@ -2216,7 +2216,7 @@ __global__ __launch_bounds__(256) void k_ii_predict1(SceneTab T, DevArrays A) {
     for (int u = 0; u < kNB; ++u) {
       if (t0 + u < nn) {
         vec3 xixj = wrapd<W>(xi - ld3(xj[u]), p);
-        vec3 gw = gradW(xixj, p);
+        vec3 gw = grad_pair(xixj, p);
         vec3 dji = (dpi * p.rho0) * gw;
         dadv += dt * p.vol * dot(vi - ld3(vj[u]), gw);
         a_ii += p.vol * dot(d_ii - dji, gw);
@@ -2268,7 +2268,7 @@ __global__ __launch_bounds__(256) void k_ii_iter0(SceneTab T, DevArrays A) {
         vec3 xixj = wrapd<W>(xi - ld3(xj[u]), p);
         float dj = djs[u];
         float dj2 = dj * dj;
-        acc -= (p.vol / dj2 * lpj[u]) * gradW(xixj, p);
+        acc -= (p.vol / dj2 * lpj[u]) * grad_pair(xixj, p);
       }
     }
   }
@@ -2315,7 +2315,7 @@ __global__ __launch_bounds__(256) void k_ii_iter1(SceneTab T, DevArrays A) {
         if (t0 + u < nn) {
           vec3 xixj = wrapd<W>(xi - ld3(xj[u]), p);
           vec3 djk_pk = ld3(dpk[u]);
-          vec3 gw = gradW(xixj, p);
+          vec3 gw = grad_pair(xixj, p);
           vec3 dji = (dpi * p.rho0) * gw;
           vec3 dji_pi = dji * lp;
           sum_tmp += p.vol * dot(dpj - ld3(diij[u]) * lpj[u] - (djk_pk - dji_pi), gw);
@@ -2387,7 +2387,7 @@ __global__ __launch_bounds__(256) void k_ii_pressure_accel(SceneTab T, DevArrays
         float dj = djs[u];
         float dj2 = dj * dj;
         float dpj = pj[u] / dj2;
-        ai -= (p.mass * (dpi + dpj)) * gradW(xixj, p);
+        ai -= (p.mass * (dpi + dpj)) * grad_pair(xixj, p);
       }
     }
   }
@@ -2398,7 +2398,7 @@ __global__ __launch_bounds__(256) void k_ii_pressure_accel(SceneTab T, DevArrays
       const unsigned sp = pellet_at(A.pnbr, A, s, t);
       const vec3 xixj = wrapd<W>(xi - ld3(A.px[sp]), p);
       const float dpj = A.pp[sp] / (p.rho0 * p.rho0);
-      const vec3 acc = (p.mass * (dpi + dpj)) * gradW(xixj, p);
+      const vec3 acc = (p.mass * (dpi + dpj)) * grad_pair(xixj, p);
       ai -= acc;
       const unsigned b = A.pbody[sp];
       const BoundaryDev& B = A.bnd[b];
@@ -2489,7 +2489,7 @@ __global__ __launch_bounds__(256) void k_is_diag(SceneTab T, DevArrays A) {
     for (int u = 0; u < kNB; ++u) {
       if (t0 + u < nn) {
         const vec3 xixj = wrapd<W>(xi - ld3(xj[u]), p);
-        const vec3 gw = gradW(xixj, p);
+        const vec3 gw = grad_pair(xixj, p);
         const float dj = djs[u];
         dadv += dt * p.vol * dot(vi - ld3(vj[u]), gw);
         diag += p.vol * (dens + dj) / (dens * dj) / (length_sqr(xixj) + eps) * dot(xixj, gw);
@@ -2502,7 +2502,7 @@ __global__ __launch_bounds__(256) void k_is_diag(SceneTab T, DevArrays A) {
     for (unsigned t = 0; t < npn; ++t) {
       const unsigned sp = pellet_at(A.pnbr, A, s, t);
       const vec3 xixj = wrapd<W>(xi - ld3(A.px[sp]), p);
-      const vec3 g = p.vol * gradW(xixj, p);
+      const vec3 g = p.vol * grad_pair(xixj, p);
       dadv += dt * dot(vi - ld3(A.pv[sp]), g);
       diag += (dens + p.rho0) / (dens * p.rho0) / (length_sqr(xixj) + eps) * dot(xixj, g);
     }
@@ -2562,7 +2562,7 @@ __global__ __launch_bounds__(256) void k_is_iter(SceneTab T, DevArrays A) {
           const vec3 xixj = wrapd<W>(xi - ld3(xj[u]), p);
           const float dj = djs[u];
           off -= p.vol * (dens + dj) / (dens * dj) / (length_sqr(xixj) + eps) *
-                 dot(xixj, gradW(xixj, p)) * lpj[u];
+                 dot(xixj, grad_pair(xixj, p)) * lpj[u];
         }
       }
     }
@@ -2574,7 +2574,7 @@ __global__ __launch_bounds__(256) void k_is_iter(SceneTab T, DevArrays A) {
         const unsigned sp = pellet_at(A.pnbr, A, s, t);
         const vec3 xixj = wrapd<W>(xi - ld3(A.px[sp]), p);
         off -= p.vol * (dens + p.rho0) / (dens * p.rho0) / (length_sqr(xixj) + eps) *
-               dot(xixj, gradW(xixj, p)) * A.pp[sp];
+               dot(xixj, grad_pair(xixj, p)) * A.pp[sp];
       }
     }
     off *= p.rho0;
@@ -2857,9 +2857,9 @@ __global__ __launch_bounds__(256) void k_pellet_fluid_lists(SceneTab T, DevArray
   float dens = p.w0;
   const unsigned nn = A.nnb[s];
   for (unsigned t = 0; t < nn; ++t)
-    dens += W_d2(length_sqr(wrapd<W>(xi - ld3(A.x[pellet_at(A.nbr, A, s, t)]), p)), p);
+    dens += W_pair(length_sqr(wrapd<W>(xi - ld3(A.x[pellet_at(A.nbr, A, s, t)]), p)), p);
   for (unsigned t = 0; t < npn; ++t)
-    dens += W_d2(length_sqr(wrapd<W>(xi - ld3(A.px[pellet_at(A.pnbr, A, s, t)]), p)), p);
+    dens += W_pair(length_sqr(wrapd<W>(xi - ld3(A.px[pellet_at(A.pnbr, A, s, t)]), p)), p);
   const float rho = dens * p.mass;
   A.density[s] = rho;
   reinterpret_cast<float*>(A.v + s)[3] = visc_coefficient(p, rho);
@@ -2894,7 +2894,7 @@ __global__ __launch_bounds__(256) void k_viscosity_pellets(SceneTab T, DevArrays
     for (unsigned t = 0; t < npn; ++t) {
       const unsigned sp = pellet_at(A.pnbr, A, s, t);
       const vec3 xixj = wrapd<W>(xi - ld3(A.px[sp]), p);
-      const vec3 acc = (p.vol * p.bvisc * dot(xixj, gradW(xixj, p)) /
+      const vec3 acc = (p.vol * p.bvisc * dot(xixj, grad_pair(xixj, p)) /
                         (length_sqr(xixj) + 0.01f * p.h2)) *
                        (vi - ld3(A.pv[sp]));
       da += acc;
@@ -2982,7 +2982,7 @@ __global__ __launch_bounds__(256) void k_extrapolate(SceneTab T, DevArrays A, in
   vec3 center = mk(0.f, 0.f, 0.f);
   for (unsigned t = 0; t < nn; ++t) {
     const vec3 xj = ld3(A.x[pellet_at(A.pbnbr, A, s, t)]);
-    const float w = W_d2(length_sqr(wrapd<W>(xi - xj, p)), p) * p.vol;
+    const float w = W_pair(length_sqr(wrapd<W>(xi - xj, p)), p) * p.vol;
     w_sum += w;
     center += w * xj;
   }
@@ -2993,7 +2993,7 @@ __global__ __launch_bounds__(256) void k_extrapolate(SceneTab T, DevArrays A, in
     const unsigned j = pellet_at(A.pbnbr, A, s, t);
     const vec3 xj = ld3(A.x[j]);
     const vec3 xt = xj - center;
-    const float w = W_d2(length_sqr(wrapd<W>(xi - xj, p)), p) * p.vol;
+    const float w = W_pair(length_sqr(wrapd<W>(xi - xj, p)), p) * p.vol;
     const float wp = w * src[j];
     alpha += wp;
     pxs += wp * xt;
@@ -3312,7 +3312,9 @@ void launch_export_iisph(const Launch& L, const DevArrays& A, float* const scala
 }
 // The device arithmetic the kernel functions are built on, element-wise
 // (alv_check_math): 0 sqrt_rn(a), 1 div_known(a, b, RN(1/b)), 2 gradW_scale
-// of the displacement (a, 0, 0), 3 W_d2(a).
+// of the displacement (a, 0, 0), 3 W_d2(a), 4 rcp_rn(a), 5 div_rn(a, b), and
+// for listed pairs 7 the gradient scale at distance a, 8 W at squared distance
+// a, 9 and 10 root and reciprocal root of a.
 __global__ __launch_bounds__(256) void k_check_math(SimParams p, int op, const float* a,
                                                     const float* b, float* out, size_t n) {
   const size_t i = size_t(blockIdx.x) * kBlock + threadIdx.x;
@@ -3327,7 +3329,11 @@ __global__ __launch_bounds__(256) void k_check_math(SimParams p, int op, const f
     case 3: r = W_d2(x, p); break;
     case 4: r = rcp_rn(x); break;
     case 5: r = div_rn(x, b[i]); break;
-        default: break;
+    case 7: r = grad_scale_pair(x * x, p); break;
+    case 8: r = W_pair(x, p); break;
+    case 9: r = pair_root(x).r; break;
+    case 10: r = pair_root(x).rr; break;
+    default: break;
   }
   out[i] = r;
 }

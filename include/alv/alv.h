@@ -487,7 +487,10 @@ int alv_profiling_kernel(unsigned index, const char** name, double* total_ms,
  * spline W of the squared distance a, with the kernel radius of cn; op 4
  * 1 / a, op 5 a / b by the general division (the reciprocal refined to the
  * correctly rounded one); op 6 the gradient scale of op 2 with the
- * compiler's IEEE division in its outer branch. */
+ * compiler's IEEE division in its outer branch.  For listed pairs, with root
+ * and reciprocal from one hardware reciprocal square root: op 7 the gradient
+ * scale at distance a <= h, op 8 W of the squared distance a < h^2, op 9
+ * sqrt(a) and op 10 1 / sqrt(a) rounded twice. */
 int alv_check_math(const alv_const* cn, int op, const float* a, const float* b, float* out,
                    size_t n);
 

@@ -103,3 +103,28 @@ long long check_div_gradient(float h, float* bad) {
   }
   return miss;
 }
+
+/* The sequence of pair_root (root r and reciprocal rr of x's root from one
+ * estimate y of 1 / sqrt(x)), for every x in [1, 4) and every y within one ulp:
+ * counts the (x, y) whose root misses sqrtf and whose reciprocal misses
+ * 1 / sqrtf, and the estimates tried. */
+void check_pair_root(long long* miss_root, long long* miss_rcp, long long* tried) {
+  long long mr = 0, mc = 0, n = 0;
+  for (uint32_t m = 0; m < (1u << 24); ++m) {
+    const float x = from_bits(0x3f800000u + m);
+    const double exact = 1.0 / sqrt((double)x);
+    const float want = sqrtf(x), near = (float)exact;
+    for (int k = -2; k <= 2; ++k) {
+      const float y = from_bits(bits(near) + (uint32_t)k);
+      if (fabs((double)y - exact) >= ldexp(1.0, ilogb(y) - 23)) continue;
+      ++n;
+      const float s = x * y;
+      const float r = fmaf(fmaf(-s, s, x), 0.5f * y, s);
+      mr += bits(r) != bits(want);
+      mc += bits(fmaf(fmaf(-want, y, 1.0f), y, y)) != bits(1.0f / want);
+    }
+  }
+  *miss_root = mr;
+  *miss_rcp = mc;
+  *tried = n;
+}

@@ -126,3 +126,45 @@ def test_known_divisor_division_and_w(h):
     assert_bits(run(L, cn, 1, a * a, d2), (a * a) / F32(cn.kernel_radius_sqr), "x / h^2")
     r2 = (rng.random(1 << 22) * F32(cn.kernel_radius_sqr) * 1.1).astype(F32)
     assert_bits(run(L, cn, 3, r2), numpy_w(r2, h, cn.kernel_radius_sqr, cn.cubic_kernel_k), "W")
+
+
+def test_pair_root_every_significand():
+    """Root and reciprocal of a listed pair's distance from one hardware
+    reciprocal square root: every significand of two binades (the estimate
+    depends on the significand and the exponent's parity only)."""
+    L = alv_ctypes.library()
+    cn = alv_ctypes.const_for(L, 0.01)
+    sig = np.arange(1 << 24, dtype=np.uint32)
+    for e in (127 - 14, 127 - 40):
+        x = ((np.uint32(e) << np.uint32(23)) + sig).view(F32)
+        r = np.sqrt(x)
+        assert_bits(run(L, cn, 9, x), r, "root, exponent %d" % (e - 127))
+        want, got = F32(1.0) / r, run(L, cn, 10, x)
+        # the one exception: r of all ones, where 2^-k is one ulp low
+        ones = (r.view(np.uint32) & np.uint32(0x7fffff)) == 0x7fffff
+        assert_bits(got[~ones], want[~ones], "reciprocal root, exponent %d" % (e - 127))
+        assert np.all(want[ones].view(np.uint32) - got[ones].view(np.uint32) <= 1)
+
+
+@pytest.mark.parametrize("h", [0.01, 2.0 ** -7, 0.037])
+def test_pair_kernels(h):
+    """The listed pairs' gradient scale over every distance of the dividing
+    branch and a dense sample of (0, h], and W over squared distances."""
+    L = alv_ctypes.library()
+    cn = alv_ctypes.const_for(L, h)
+    rs = np.concatenate([gradient_branch(h), (np.arange(1, 1 << 20, dtype=np.float64) /
+                                               (1 << 20) * float(h)).astype(F32)])
+    rs = rs[np.sqrt(rs * rs) <= F32(h)]
+    want = numpy_grad_scale(rs, h, cn.cubic_kernel_l)
+    got = run(L, cn, 7, rs)
+    # one ulp where r is all ones, 2^k (1 - 2^-24), and the dividend a power of
+    # two: the reciprocal there is 2^-k, one ulp low (h = 2^-7: at r = h (1 -
+    # 2^-24) the dividend is -2^-48).  The quotient's ulp is at most two of
+    # the product with l, whose two roundings add one.  At r = h the value is a
+    # zero whose sign is not kept.
+    ones = (np.sqrt(rs * rs).view(np.uint32) & np.uint32(0x7fffff)) == 0x7fffff
+    assert_bits(got[~ones] + F32(0.0), want[~ones] + F32(0.0), "pair gradient scale h=%g" % h)
+    assert np.all(np.abs(got[ones].view(np.int32) - want[ones].view(np.int32)) <= 3)
+    r2 = (np.random.default_rng(6).random(1 << 22) * F32(cn.kernel_radius_sqr)).astype(F32)
+    r2 = r2[r2 < F32(cn.kernel_radius_sqr)]
+    assert_bits(run(L, cn, 8, r2), numpy_w(r2, h, cn.kernel_radius_sqr, cn.cubic_kernel_k), "pair W")

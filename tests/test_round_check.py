@@ -63,3 +63,17 @@ def test_gradient_division_every_distance(tmp_path_factory, h):
     L = lib(tmp_path_factory)
     bad = ctypes.c_float()
     assert L.check_div_gradient(h, ctypes.byref(bad)) == 0, bad.value
+
+
+def test_pair_root_every_estimate(tmp_path_factory):
+    """Root and reciprocal from one reciprocal square root: correctly rounded
+    from every estimate within one ulp but the few counted here, of which the
+    hardware returns only one (tests/test_gpu_math.py)."""
+    L = lib(tmp_path_factory)
+    ll = ctypes.POINTER(ctypes.c_longlong)
+    L.check_pair_root.argtypes = [ll, ll, ll]
+    L.check_pair_root.restype = None
+    root, rcp, tried = ctypes.c_longlong(), ctypes.c_longlong(), ctypes.c_longlong()
+    L.check_pair_root(ctypes.byref(root), ctypes.byref(rcp), ctypes.byref(tried))
+    assert tried.value > 2 * (1 << 24) - 16, tried.value
+    assert (root.value, rcp.value) == (1, 9)
