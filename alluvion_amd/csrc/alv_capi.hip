@@ -1980,19 +1980,17 @@ int pellet_launch(alv_solver* S, const Launch& L, Launch* Lp) {
 // leaves it out, since only a step reads it, after its own neighbour phase.
 int neighbor_phase(alv_solver* S, const Launch& L, int with_factor, bool gather_state = true) {
   DevArrays& A = S->A;
-  launch_clear_grid(L, A, S->stream);
+  launch_clear_grid(L, A, 1, S->stream);
   if (L.active == 0) return ALV_OK;
   launch_cell_count(L, A, S->stream);
-  launch_reserve_padding(L, A, S->stream);
   launch_scan(L.cells, A.cell_count, A.cell_start, A.scan_tmp, S->stream);
   launch_scatter(L, A, S->stream);
-  launch_cell_sort(L, A, S->stream);
-  launch_tiles(L, A, S->stream);
   const int kind = !gather_state            ? ALV_KIND_NONE
                    : S->kind != ALV_SOLVER_DF ? ALV_KIND_II
                    : with_factor             ? ALV_KIND_DF
                                              : ALV_KIND_DF_FACTOR;
-  launch_gather_boundary(L, A, kind, S->stream);
+  launch_sort_gather(L, A, kind, S->stream);
+  launch_tiles(L, A, S->stream);
   launch_neighbors(L, A, with_factor, S->stream);
   ALV_HIP(hipGetLastError());
   S->grid_valid = 1;
@@ -2308,7 +2306,7 @@ int alv_solver_step(alv_solver* S) {
     // factor (solver_df.hpp:81-91): the density solve reads the one each
     // particle ended the last step with.  It goes to user order with the
     // last step's permutation here and comes back in the new one
-    // (k_gather_boundary, ALV_KIND_DF_FACTOR).
+    // (k_sort_gather, ALV_KIND_DF_FACTOR).
     if (!div && L.active && (S->dirty & ALV_F_ALPHA)) {
       launch_unsort_fields(L, A, ALV_F_ALPHA, st);
       ALV_HIP(hipGetLastError());

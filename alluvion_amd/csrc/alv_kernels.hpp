@@ -219,24 +219,26 @@ inline unsigned parts_per_block(const Launch& L) {
 
 // neighbour search (counting sort)
 void launch_fill_u32(unsigned* dst, unsigned value, size_t count, hipStream_t s);
-// zeroes the cell counts (L.cells) and the grid anomaly flags and resets the
-// control blocks for the step's solves
-void launch_clear_grid(const Launch& L, const DevArrays& A, hipStream_t s);
+// clears the cell counts (L.cells; each scene's unused slots are counted into
+// its outside-the-grid bin) and, for a step, the grid anomaly flags, and resets
+// the control blocks for the step's solves
+void launch_clear_grid(const Launch& L, const DevArrays& A, int step, hipStream_t s);
 void launch_cell_count(const Launch& L, const DevArrays& A, hipStream_t s);
-// reserves each scene's unused slots at the end of its outside-the-grid bin
-void launch_reserve_padding(const Launch& L, const DevArrays& A, hipStream_t s);
 // Cells per block of the cell-count scan (1024: four per thread, so a 1 M-cell
 // grid runs 1024 blocks, four per CU); `tmp` holds one sum per block.
 constexpr unsigned kScanPerBlock = 1024;
+// Blocks up to which the scan is one launch (every block adds up the counts
+// before its own, at most 512 KB from L2) or two (it adds up the block sums, 16
+// loads per thread at most); a launch costs a step of few particles 4 us.
+constexpr unsigned kScanOneLaunch = 128, kScanNoTop = 4096;
 void launch_scan(unsigned count, const unsigned* in, unsigned* out, unsigned* tmp,
                  hipStream_t s);
 void launch_scatter(const Launch& L, const DevArrays& A, hipStream_t s);
 void launch_cell_sort(const Launch& L, const DevArrays& A, hipStream_t s);
 // LDS tile ranges of every block (after the sort, before the passes)
 void launch_tiles(const Launch& L, const DevArrays& A, hipStream_t s);
-// gather user -> sorted and compute boundary records
-void launch_gather_boundary(const Launch& L, const DevArrays& A, int solver_kind,
-                            hipStream_t s);
+// sorts every cell, gathers user -> sorted and computes the boundary records
+void launch_sort_gather(const Launch& L, const DevArrays& A, int solver_kind, hipStream_t s);
 // neighbour list + density; mode 1: + DFSPH factor; mode 2: + factor and the
 // divergence solve's warm start 0
 void launch_neighbors(const Launch& L, const DevArrays& A, int with_factor, hipStream_t s);
@@ -388,8 +390,8 @@ enum : unsigned {
   ALV_F_PRESSURE = 1u << 5,
 };
 
-// field codes written by launch_unsort_fields / gathered in gather_boundary
-// solver state gathered into sorted order by k_gather_boundary: DFSPH
+// field codes written by launch_unsort_fields / gathered in k_sort_gather
+// solver state gathered into sorted order by k_sort_gather: DFSPH
 // stiffnesses (with DF_FACTOR also the DFSPH factor, for a step without the
 // divergence solve, which does not compute it), IISPH/ISPH pressure, or none
 // (positions and velocities only)

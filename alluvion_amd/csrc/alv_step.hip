@@ -176,7 +176,9 @@ __global__ __launch_bounds__(256) void k_cell_count(SceneTab T, DevArrays A) {
     A.anomaly[0] = 1u;
   }
   A.key[i] = k;
-  A.slot[i] = atomicAdd(&A.cell_count[k], 1u);
+  // the outside bin's count starts at the scene's unused slots (k_clear_grid)
+  const unsigned first = k == p.cell_base + p.num_cells ? p.span - p.n : 0u;
+  A.slot[i] = atomicAdd(&A.cell_count[k], 1u) - first;
 }
 
 constexpr unsigned kScanPerThread = kScanPerBlock / kBlock;
@@ -213,10 +215,38 @@ __global__ __launch_bounds__(256) void k_scan_top(unsigned nblocks, unsigned* su
   }
 }
 
+// sum of v over the block, in every thread
+__device__ inline unsigned block_sum_u32(unsigned v, unsigned* lds) {
+  unsigned total;
+  block_excl_scan_u32(v, lds, &total);
+  return total;
+}
+
+// Where a block of the scan finds the sum of the cells before its own: the
+// counts themselves (few cells: one launch), the block sums (k_scan_reduce),
+// or their scan (k_scan_top).
+enum { kScanCounts = 0, kScanSums = 1, kScanScanned = 2 };
+
 // out[0..count] = exclusive scan of in[0..count); out[count] = total
+template <int From>
 __global__ __launch_bounds__(256) void k_scan_apply(unsigned count, const unsigned* in,
-                                                    unsigned* out, const unsigned* offsets) {
+                                                    unsigned* out, const unsigned* sums) {
   __shared__ unsigned lds[4];
+  unsigned before = 0;
+  if (From == kScanScanned) {
+    before = sums[blockIdx.x];
+  } else {
+    const uint4* in4 = reinterpret_cast<const uint4*>(in);
+    unsigned v = 0;
+    if (From == kScanCounts)
+      for (unsigned k = threadIdx.x; k < blockIdx.x * (kScanPerBlock / 4u); k += kBlock) {
+        const uint4 q = in4[k];
+        v += q.x + q.y + q.z + q.w;
+      }
+    else
+      for (unsigned k = threadIdx.x; k < blockIdx.x; k += kBlock) v += sums[k];
+    before = block_sum_u32(v, lds);
+  }
   const unsigned base = blockIdx.x * kScanPerBlock + threadIdx.x * kScanPerThread;
   unsigned vals[kScanPerThread];
   unsigned local = 0;
@@ -225,7 +255,7 @@ __global__ __launch_bounds__(256) void k_scan_apply(unsigned count, const unsign
     vals[k] = (base + k < count) ? in[base + k] : 0u;
     local += vals[k];
   }
-  unsigned run = block_excl_scan_u32(local, lds, nullptr) + offsets[blockIdx.x];
+  unsigned run = block_excl_scan_u32(local, lds, nullptr) + before;
 #pragma unroll
   for (unsigned k = 0; k < kScanPerThread; ++k) {
     if (base + k < count) out[base + k] = run;
@@ -250,21 +280,23 @@ __global__ __launch_bounds__(256) void k_scatter(SceneTab T, DevArrays A) {
 // cell when particle order and space are unrelated).  The bin of particles
 // outside the grid keeps the arrival order: nothing depends on it (those
 // particles are in no cell and their own neighbour scans are independent).
-__global__ __launch_bounds__(256) void k_cell_sort(SceneTab T, DevArrays A) {
-  ALV_SCENE_LINEAR(T, A, t);
-  if (t >= p.first + p.n) return;
-  const unsigned i = A.sort_tmp[t];
+__device__ inline unsigned sorted_place(const SimParams& p, const DevArrays& A, unsigned t,
+                                        unsigned i) {
   const unsigned k = A.key[i];
-  if (k == p.cell_base + p.num_cells) {
-    A.sorted_id[t] = i;
-    return;
-  }
+  if (k == p.cell_base + p.num_cells) return t;
   const unsigned b = A.cell_start[k];
   const unsigned e = A.cell_start[k + 1];
   if (e - b > p.cell_cap) A.anomaly[1] = 1u;
   unsigned rank = 0;
   for (unsigned u = b; u < e; ++u) rank += A.sort_tmp[u] < i ? 1u : 0u;
-  A.sorted_id[b + rank] = i;
+  return b + rank;
+}
+// the order alone (the pellets)
+__global__ __launch_bounds__(256) void k_cell_sort(SceneTab T, DevArrays A) {
+  ALV_SCENE_LINEAR(T, A, t);
+  if (t >= p.first + p.n) return;
+  const unsigned i = A.sort_tmp[t];
+  A.sorted_id[sorted_place(p, A, t, i)] = i;
 }
 
 // LDS tile of every particle block.  For a block whose in-grid particles all
@@ -339,10 +371,15 @@ __global__ __launch_bounds__(256) void k_tiles(SceneTab T, DevArrays A, unsigned
 // (compute_particle_boundary_analytic<0>, runner.hpp:1982-2002, with
 // compute_volume_and_boundary_x_analytic, runner.hpp:1738-1771)
 // ---------------------------------------------------------------------------
-__global__ __launch_bounds__(256) void k_gather_boundary(SceneTab T, DevArrays A, int kind) {
-  ALV_SCENE(T, A, s);
-  if (s >= p.first + p.n) return;
-  const unsigned i = A.sorted_id[s];
+// The particle of the scatter's slot t goes to its place in the canonical order
+// (k_cell_sort) on the way: one launch, and the place lies in the same cell, a
+// few slots from t, so the writes stay as coalesced.
+__global__ __launch_bounds__(256) void k_sort_gather(SceneTab T, DevArrays A, int kind) {
+  ALV_SCENE(T, A, t);
+  if (t >= p.first + p.n) return;
+  const unsigned i = A.sort_tmp[t];
+  const unsigned s = sorted_place(p, A, t, i);
+  A.sorted_id[s] = i;
   vec3 x = ld3(A.ux, i);
   vec3 v = ld3(A.uv, i);
   A.x[s] = f4(x, 0.0f);
@@ -3111,36 +3148,30 @@ __global__ __launch_bounds__(256) void k_fill_u32(unsigned* __restrict__ d, unsi
   const size_t i = size_t(blockIdx.x) * kBlock + threadIdx.x;
   if (i < n) d[i] = v;
 }
-// zeroes the cell counts and the three grid anomaly flags and resets every
-// scene's control block (one launch)
-__global__ __launch_bounds__(256) void k_clear_grid(DevArrays A, unsigned cells, unsigned scenes) {
+// Clears the cell counts and the three grid anomaly flags and resets every
+// scene's control block (one launch).  The slots of a scene's range past its
+// particles are counted into its outside-the-grid bin from the start, so that
+// after the scan every scene's sorted range starts where its user range starts.
+// With step 0 (the pellets' grid) only the counts are cleared.
+__global__ __launch_bounds__(256) void k_clear_grid(SceneTab T, DevArrays A, unsigned cells,
+                                                    unsigned scenes, int step) {
   const unsigned i = blockIdx.x * kBlock + threadIdx.x;
-  if (i < cells) A.cell_count[i] = 0u;
+  if (i < cells) {
+    const SimParams& p = T.par[T.cblk_scene[blockIdx.x]];
+    A.cell_count[i] = i == p.cell_base + p.num_cells ? p.span - p.n : 0u;
+  }
+  if (!step) return;
   if (i < 3u) A.anomaly[i] = 0u;
   if (i < scenes) reset_ctl(A, i);
 }
-void launch_clear_grid(const Launch& L, const DevArrays& A, hipStream_t s) {
+void launch_clear_grid(const Launch& L, const DevArrays& A, int step, hipStream_t s) {
   const unsigned nb = std::max(1u, (std::max(L.cells, L.scenes) + kBlock - 1) / kBlock);
-  hipLaunchKernelGGL(k_clear_grid, dim3(nb), dim3(kBlock), 0, s, A, L.cells, L.scenes);
+  hipLaunchKernelGGL(k_clear_grid, dim3(nb), dim3(kBlock), 0, s, L.T, A, L.cells, L.scenes, step);
 }
 void launch_fill_u32(unsigned* dst, unsigned value, size_t count, hipStream_t s) {
   if (!count) return;
   hipLaunchKernelGGL(k_fill_u32, dim3(unsigned((count + kBlock - 1) / kBlock)), dim3(kBlock), 0,
                      s, dst, value, count);
-}
-
-// The slots of a scene's range past its particles are counted into its
-// outside-the-grid bin, so that after the scan every scene's sorted range
-// starts where its user range starts.
-__global__ void k_reserve_padding(SceneTab T, DevArrays A, unsigned scenes) {
-  const unsigned sc = blockIdx.x * blockDim.x + threadIdx.x;
-  if (sc >= scenes) return;
-  const SimParams p = T.par[sc];
-  A.cell_count[p.cell_base + p.num_cells] += p.span - p.n;
-}
-void launch_reserve_padding(const Launch& L, const DevArrays& A, hipStream_t s) {
-  hipLaunchKernelGGL(k_reserve_padding, dim3((L.scenes + 63) / 64), dim3(64), 0, s, L.T, A,
-                     L.scenes);
 }
 
 void launch_cell_count(const Launch& L, const DevArrays& A, hipStream_t s) {
@@ -3149,9 +3180,18 @@ void launch_cell_count(const Launch& L, const DevArrays& A, hipStream_t s) {
 void launch_scan(unsigned count, const unsigned* in, unsigned* out, unsigned* tmp,
                  hipStream_t s) {
   const unsigned nb = (count + kScanPerBlock - 1) / kScanPerBlock;
+  const unsigned* sums = tmp;
+  if (nb <= kScanOneLaunch) {
+    ALV_LAUNCH_GRID(k_scan_apply<kScanCounts>, dim3(nb), s, count, in, out, sums);
+    return;
+  }
   ALV_LAUNCH_GRID(k_scan_reduce, dim3(nb), s, count, in, tmp);
+  if (nb <= kScanNoTop) {
+    ALV_LAUNCH_GRID(k_scan_apply<kScanSums>, dim3(nb), s, count, in, out, sums);
+    return;
+  }
   ALV_LAUNCH1(k_scan_top, s, nb, tmp);
-  ALV_LAUNCH_GRID(k_scan_apply, dim3(nb), s, count, in, out, (const unsigned*)tmp);
+  ALV_LAUNCH_GRID(k_scan_apply<kScanScanned>, dim3(nb), s, count, in, out, sums);
 }
 void launch_scatter(const Launch& L, const DevArrays& A, hipStream_t s) {
   ALV_LAUNCH(k_scatter, L, s, A);
@@ -3163,8 +3203,8 @@ void launch_tiles(const Launch& L, const DevArrays& A, hipStream_t s) {
   if (!A.use_tiles) return;
   ALV_LAUNCH_GRID(k_tiles, dim3(grid_for(L.pblocks)), s, L.T, A, L.pblocks);
 }
-void launch_gather_boundary(const Launch& L, const DevArrays& A, int kind, hipStream_t s) {
-  ALV_LAUNCH(k_gather_boundary, L, s, A, kind);
+void launch_sort_gather(const Launch& L, const DevArrays& A, int kind, hipStream_t s) {
+  ALV_LAUNCH(k_sort_gather, L, s, A, kind);
 }
 void launch_neighbors(const Launch& L, const DevArrays& A, int with_factor, hipStream_t s) {
   if (g_profiler) g_profiler->begin("k_neighbors", s);
@@ -3362,9 +3402,8 @@ void launch_pellet_grid(const Launch& Lp, const DevArrays& A, hipStream_t s) {
   Ap.cell_count = A.pcell_count;
   Ap.cell_start = A.pcell_start;
   Ap.scan_tmp = A.pscan_tmp;
-  launch_fill_u32(A.pcell_count, 0u, Lp.cells, s);
+  launch_clear_grid(Lp, Ap, 0, s);
   if (Lp.active) launch_cell_count(Lp, Ap, s);
-  launch_reserve_padding(Lp, Ap, s);
   launch_scan(Lp.cells, Ap.cell_count, Ap.cell_start, Ap.scan_tmp, s);
   if (Lp.active) {
     launch_scatter(Lp, Ap, s);

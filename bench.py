@@ -71,7 +71,7 @@ def kernel_bytes(name, K, nb, df_fused=False):
         "k_p_iter": nbr + 4 + 12 + 8 + 24 + 4 + 16 * nb,
         "k_p_err": nbr + 12 + 12 + 4 + 4 + 4 + 4 + 4 + 32 * nb,
         "k_df_finish": 4 + 12 + 12 + 8 + 12 + 12 + 8,
-        "k_gather_boundary": 4 + 12 + 12 + 8 + 12 + 12 + 8 + 4,
+        "k_sort_gather": 4 + 4 + 4 + 4 + 12 + 12 + 8 + 12 + 12 + 8 + 4,
         "k_cell_count": 12 + 4 + 4,
         "k_scatter": 4 + 4 + 4,
         "k_density_change": nbr + 12 + 12 + 4 + 32 * nb,
