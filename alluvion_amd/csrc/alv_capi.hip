@@ -1997,23 +1997,47 @@ int neighbor_phase(alv_solver* S, const Launch& L, int with_factor, bool gather_
   return ALV_OK;
 }
 
+bool has_dynamic(const alv_pile* pile) {
+  for (const auto& B : pile->bnd)
+    if (B.dynamic) return true;
+  return false;
+}
+// rigid force sums (solver_df.hpp:347-353) at the end of a step: k_body_sums
+// stores them in body_host, so the control blocks' wait brings back both
+void enqueue_body_sums(alv_solver* S, const Launch& L, const DevArrays& A) {
+  if (!S->batch && L.active && has_dynamic(S->pile)) launch_body_sums(L, A, S->stream);
+}
+
 // Enqueues Jacobi iterations in chunks until every scene's device flag says
-// done.
-template <class LaunchFn>
-int run_loop(alv_solver* S, bool divergence, unsigned max_iter, unsigned* last,
-             LaunchFn launch) {
+// done, then finish(A).  With one scene, finish is enqueued behind the first
+// chunk before the host has seen the flag (its kernels do nothing where the
+// flag is not set) and again only after a solve that took longer; the host
+// waits once per step instead of once per solve and once at the end.
+template <class LaunchFn, class FinishFn>
+int run_loop(alv_solver* S, unsigned max_iter, unsigned* last, LaunchFn launch, FinishFn finish) {
   unsigned issued = 0;
   unsigned chunk = std::max(1u, *last);
-  while (issued < max_iter) {
+  bool ahead = !S->batch;
+  while (issued < max_iter || ahead) {
     unsigned todo = std::min(chunk, max_iter - issued);
     for (unsigned k = 0; k < todo; ++k) launch();
+    if (ahead) {
+      DevArrays A = S->A;
+      A.wait = kWaitDens;
+      finish(A);
+    }
     ALV_HIP(hipGetLastError());
     issued += todo;
     int rc = read_ctl(S);
     if (rc != ALV_OK) return rc;
-    if (all_done(S, divergence)) break;
+    if (all_done(S, false)) {
+      if (ahead) return ALV_OK;
+      break;
+    }
+    ahead = false;
     chunk = std::max(1u, chunk / 2);
   }
+  finish(S->A);
   return ALV_OK;
 }
 
@@ -2037,17 +2061,11 @@ void fill_report(const alv_solver* S, alv_solver_report* r, const StepCtl& c) {
   r->utilized_cfl = c.utilized_cfl;
 }
 
+// The host's part of a step's end, once everything (the body sums included) is
+// enqueued.
 int finish_step(alv_solver* S, const Launch& L) {
-  // rigid force sums (solver_df.hpp:347-353): k_body_sums stores them in
-  // body_host, so the control blocks' wait brings back both
   alv_pile* pile = S->pile;
-  bool any_dynamic = false;
-  for (const auto& B : pile->bnd) any_dynamic |= B.dynamic != 0;
-  const bool body_sums = !S->batch && any_dynamic && L.active;
-  if (body_sums) {
-    launch_body_sums(L, S->A, S->stream);
-    ALV_HIP(hipGetLastError());
-  }
+  const bool body_sums = !S->batch && L.active && has_dynamic(pile);
   int rc = read_ctl(S);
   if (rc != ALV_OK) return rc;
   if (g_event_profiler) g_event_profiler->collect();
@@ -2312,6 +2330,42 @@ int alv_solver_step(alv_solver* S) {
       ALV_HIP(hipGetLastError());
       S->dirty &= ~ALV_F_ALPHA;
     }
+    // The later segments of a solver of one scene are enqueued before the host
+    // has seen whether the solves ended within their chunks (A.wait: their
+    // kernels do nothing where a solve has not), so a step waits once; a solve
+    // that takes longer is finished and its followers are enqueued again.
+    const bool ahead = !S->batch && L.active;
+    auto wait_for = [&](unsigned solves) {
+      DevArrays w = A;
+      w.wait = ahead ? solves : 0u;
+      return w;
+    };
+    const unsigned wait_div = div ? kWaitDiv : 0u, wait_dens = dens ? kWaitDens : 0u;
+    auto density_segment = [&](const DevArrays& Aw) {
+      // with the divergence solve, its density-change passes computed the
+      // viscosity
+      if (L.active && !div) launch_df_viscosity(L, Aw, st);
+      launch_update_dt(L, Aw, div, st);
+      if (L.active) {
+        launch_df_integrate_np(L, Aw, div, st);
+        if (dens) {
+          launch_df_warm_start_dens(L, Aw, st, learned_dens);
+          for (unsigned k = 0; k < cdens; ++k) launch_df_dens_iteration(L, Aw, st);
+        }
+      }
+    };
+    auto end_segment = [&](const DevArrays& Aw) {
+      if (L.active) launch_df_finish(L, Aw, dens, st);
+      enqueue_body_sums(S, L, Aw);
+    };
+    auto finish_divergence = [&] {
+      return finish_loop(S, true, cdiv, S->set.max_divergence_solve,
+                         [&] { launch_df_div_iteration(L, A, st); });
+    };
+    auto finish_density = [&] {
+      return finish_loop(S, false, cdens, S->set.max_density_solve,
+                         [&] { launch_df_dens_iteration(L, A, st); });
+    };
     rc = run_segment(S, 0, keyA, [&] {
       if (neighbor_phase(S, L, fuse_ws ? 2 : div) != ALV_OK) return;
       if (L.active && div) {
@@ -2321,36 +2375,32 @@ int alv_solver_step(alv_solver* S) {
       }
     });
     if (rc != ALV_OK) return rc;
-    if (L.active && div) {
-      rc = finish_loop(S, true, cdiv, S->set.max_divergence_solve,
-                       [&] { launch_df_div_iteration(L, A, st); });
-      if (rc != ALV_OK) return rc;
-    }
+    if (!ahead && L.active && div && (rc = finish_divergence()) != ALV_OK) return rc;
     const unsigned long long keyB = base ^ ((unsigned long long)cdens << 8) ^ (div << 1) ^
                                     (dens << 2) ^ (learned_dens << 3);
-    rc = run_segment(S, 1, keyB, [&] {
-      // with the divergence solve, its density-change passes computed the
-      // viscosity
-      if (L.active && !div) launch_df_viscosity(L, A, st);
-      launch_update_dt(L, A, div, st);
-      if (L.active) {
-        launch_df_integrate_np(L, A, div, st);
-        if (dens) {
-          launch_df_warm_start_dens(L, A, st, learned_dens);
-          for (unsigned k = 0; k < cdens; ++k) launch_df_dens_iteration(L, A, st);
-        }
-      }
-    });
+    rc = run_segment(S, 1, keyB, [&] { density_segment(wait_for(wait_div)); });
     if (rc != ALV_OK) return rc;
-    if (L.active && dens) {
-      rc = finish_loop(S, false, cdens, S->set.max_density_solve,
-                       [&] { launch_df_dens_iteration(L, A, st); });
+    if (!ahead && L.active && dens && (rc = finish_density()) != ALV_OK) return rc;
+    const bool sums = L.active && has_dynamic(S->pile);
+    rc = run_segment(S, 2, base ^ (dens << 1) ^ (div << 2) ^ (sums << 3) ^
+                               ((unsigned long long)L.p0.num_boundaries << 8),
+                     [&] { end_segment(wait_for(wait_div | wait_dens)); });
+    if (rc != ALV_OK) return rc;
+    if (ahead) {
+      rc = read_ctl(S);
       if (rc != ALV_OK) return rc;
+      const bool late_div = div && !S->ctl_host->div_done;
+      const bool late_dens = dens && !S->ctl_host->dens_done;
+      if (late_div) {
+        if ((rc = finish_divergence()) != ALV_OK) return rc;
+        density_segment(A);
+      }
+      if (late_div || late_dens) {
+        if (dens && (rc = finish_density()) != ALV_OK) return rc;
+        end_segment(A);
+        ALV_HIP(hipGetLastError());
+      }
     }
-    rc = run_segment(S, 2, base ^ (dens << 1), [&] {
-      if (L.active) launch_df_finish(L, A, dens, st);
-    });
-    if (rc != ALV_OK) return rc;
   } else if (S->kind == ALV_SOLVER_I && L.p0.pellet_mode) {
     // SolverI::step (solver_i.hpp:79-330) with pellets
     Launch Lp;
@@ -2365,11 +2415,14 @@ int alv_solver_step(alv_solver* S) {
     launch_update_dt(L, A, 0, st);
     if (L.active) {
       launch_is_prepare_pellets(L, A, st);
-      rc = run_loop(S, false, S->set.max_density_solve, &S->last_dens,
-                    [&] { launch_is_iteration_pellets(L, Lp, A, st); });
+      rc = run_loop(S, S->set.max_density_solve, &S->last_dens,
+                    [&] { launch_is_iteration_pellets(L, Lp, A, st); },
+                    [&](const DevArrays& Aw) {
+                      launch_is_settle(L, Aw, st);
+                      launch_is_finish_pellets(L, Lp, Aw, st);
+                      enqueue_body_sums(S, L, Aw);
+                    });
       if (rc != ALV_OK) return rc;
-      launch_is_settle(L, A, st);
-      launch_is_finish_pellets(L, Lp, A, st);
     }
   } else if (S->kind == ALV_SOLVER_I) {
     // SolverI::step (solver_i.hpp:79-330), volume-map boundaries
@@ -2379,11 +2432,14 @@ int alv_solver_step(alv_solver* S) {
     launch_update_dt(L, A, 0, st);
     if (L.active) {
       launch_is_prepare(L, A, st);
-      rc = run_loop(S, false, S->set.max_density_solve, &S->last_dens,
-                    [&] { launch_is_iteration(L, A, st); });
+      rc = run_loop(S, S->set.max_density_solve, &S->last_dens,
+                    [&] { launch_is_iteration(L, A, st); },
+                    [&](const DevArrays& Aw) {
+                      launch_is_settle(L, Aw, st);
+                      launch_ii_finish(L, Aw, st);
+                      enqueue_body_sums(S, L, Aw);
+                    });
       if (rc != ALV_OK) return rc;
-      launch_is_settle(L, A, st);
-      launch_ii_finish(L, A, st);
     }
   } else {
     // SolverIi::step (solver_ii.hpp:76-243)
@@ -2393,10 +2449,13 @@ int alv_solver_step(alv_solver* S) {
     launch_update_dt(L, A, 0, st);
     if (L.active) {
       launch_ii_predict(L, A, st);
-      rc = run_loop(S, false, S->set.max_density_solve, &S->last_dens,
-                    [&] { launch_ii_iteration(L, A, st); });
+      rc = run_loop(S, S->set.max_density_solve, &S->last_dens,
+                    [&] { launch_ii_iteration(L, A, st); },
+                    [&](const DevArrays& Aw) {
+                      launch_ii_finish(L, Aw, st);
+                      enqueue_body_sums(S, L, Aw);
+                    });
       if (rc != ALV_OK) return rc;
-      launch_ii_finish(L, A, st);
     }
   }
   ALV_HIP(hipGetLastError());

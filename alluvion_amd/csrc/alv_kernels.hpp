@@ -113,7 +113,9 @@ struct DevArrays {
   // kernel that changes a block publishes it there (publish_ctl)
   StepCtl* ctl_pub;
   const BoundaryDev* bnd;
+  unsigned wait = 0u;  // solves that must have ended for a launch to do anything
 };
+enum : unsigned { kWaitDiv = 1u, kWaitDens = 2u };
 
 constexpr unsigned kBlock = 256;
 // Lanes per particle of the density-change passes that gather neighbours

@@ -93,6 +93,12 @@ __device__ inline void add_v(DevArrays& A, unsigned s, vec3 dv) {
   A.v[s] = make_float4(v.x + dv.x, v.y + dv.y, v.z + dv.z, v.w);
 }
 __device__ inline float std_min(float a, float b) { return (b < a) ? b : a; }
+// A launch made before the host has seen whether the solve before it ended
+// (kWaitDiv, kWaitDens: a solver of one scene) does nothing until it has; the
+// host then finishes the solve and launches again.
+__device__ inline bool must_wait(const DevArrays& A) {
+  return ((A.wait & kWaitDiv) && !A.ctl->div_done) || ((A.wait & kWaitDens) && !A.ctl->dens_done);
+}
 // The viscosity's coefficient of a neighbour, mu m / rho_j, which
 // compute_viscosity (runner.hpp:2150-2249) divides out for every pair: it is
 // stored with the particle's velocity (v.w) when its density is computed, so
@@ -1968,6 +1974,7 @@ __global__ __launch_bounds__(256) void k_viscosity(SceneTab T, DevArrays A) {
 __global__ __launch_bounds__(kFinBlock) void k_update_dt(SceneTab T, DevArrays A, unsigned parts) {
   __shared__ float lds[kFinBlock / 64];
   ALV_SCENE_BLOCK(T, A);
+  if (must_wait(A)) return;
   float m = -FLT_MAX;
   for (unsigned b = blk_begin * parts + threadIdx.x; b < blk_end * parts; b += blockDim.x)
     m = std_max(m, A.fpartials[b]);
@@ -2006,6 +2013,7 @@ __global__ __launch_bounds__(kFinBlock) void k_update_dt(SceneTab T, DevArrays A
 // which this kernel has not yet changed.
 __global__ __launch_bounds__(256) void k_integrate_np(SceneTab T, DevArrays A, int fin) {
   ALV_SCENE(T, A, s);
+  if (must_wait(A)) return;
   if (s >= p.first + p.n) return;
   const float dt = A.ctl->dt;
   if (fin) {
@@ -2023,6 +2031,7 @@ __global__ __launch_bounds__(256) void k_integrate_np(SceneTab T, DevArrays A, i
 template <bool W, bool L, int M>
 __global__ __launch_bounds__(pass_threads(M, change_lanes(M))) void k_ws_p0(SceneTab T, DevArrays A) {
   ALV_SCENE_PASS(T, A, s, q, M, change_lanes(M));
+  if (must_wait(A)) return;
   TileXV tile_;
   bool tiled_ = false;
   if constexpr (M == kTile) tiled_ = stage_xv(A, s / kBlock, tile_);
@@ -2042,6 +2051,7 @@ __global__ __launch_bounds__(pass_threads(M, change_lanes(M))) void k_ws_p0(Scen
 template <bool W, int M>
 __global__ __launch_bounds__(pass_threads(M, stiffness_lanes(M))) void k_ws_p1(SceneTab T, DevArrays A) {
   ALV_SCENE_PASS(T, A, s, q, M, stiffness_lanes(M));
+  if (must_wait(A)) return;
   TileX tk_;
   bool tiled_ = false;
   if constexpr (M == kTile) tiled_ = stage_x(A, s / kBlock, tk_);
@@ -2053,6 +2063,7 @@ __global__ __launch_bounds__(pass_threads(M, stiffness_lanes(M))) void k_ws_p1(S
 template <bool W, int M>
 __global__ __launch_bounds__(pass_threads(M, change_lanes(M))) void k_rho_adv(SceneTab T, DevArrays A) {
   ALV_SCENE_PASS(T, A, s, q, M, change_lanes(M));
+  if (must_wait(A)) return;
   TileXV tile_;
   bool tiled_ = false;
   if constexpr (M == kTile) tiled_ = stage_xv(A, s / kBlock, tile_);
@@ -2071,6 +2082,7 @@ __global__ __launch_bounds__(pass_threads(M, change_lanes(M))) void k_rho_adv(Sc
 template <bool W, int M>
 __global__ __launch_bounds__(pass_threads(M, stiffness_lanes(M))) void k_p_iter(SceneTab T, DevArrays A) {
   ALV_SCENE_PASS(T, A, s, q, M, stiffness_lanes(M));
+  if (must_wait(A)) return;
   if (A.ctl->dens_done) return;
   TileX tk_;
   bool tiled_ = false;
@@ -2087,6 +2099,7 @@ template <bool W, int M>
 __global__ __launch_bounds__(pass_threads(M, change_lanes(M))) void k_p_err(SceneTab T, DevArrays A) {
   __shared__ double lds[pass_threads(M, change_lanes(M)) / 64];
   ALV_SCENE_PASS(T, A, s, q, M, change_lanes(M));
+  if (must_wait(A)) return;
   if (A.ctl->dens_done) return;
   TileXV tile_;
   bool tiled_ = false;
@@ -2109,6 +2122,7 @@ __global__ __launch_bounds__(pass_threads(M, change_lanes(M))) void k_p_err(Scen
 __global__ __launch_bounds__(kFinBlock) void k_p_finalize(SceneTab T, DevArrays A, unsigned parts) {
   __shared__ double lds[kFinBlock / 64];
   ALV_SCENE_BLOCK(T, A);
+  if (must_wait(A)) return;
   StepCtl* ctl = A.ctl;
   if (ctl->dens_done) return;
   double part = 0.0;
@@ -2131,6 +2145,7 @@ __global__ __launch_bounds__(kFinBlock) void k_p_finalize(SceneTab T, DevArrays 
 template <bool W>
 __global__ __launch_bounds__(256) void k_df_finish(SceneTab T, DevArrays A, int dens_finish) {
   ALV_SCENE(T, A, s);
+  if (must_wait(A)) return;
   if (s >= p.first + p.n) return;
   const float dt = A.ctl->dt;
   const unsigned i = A.sorted_id[s];
@@ -2399,6 +2414,7 @@ __global__ __launch_bounds__(kFinBlock) void k_ii_finalize(SceneTab T, DevArrays
 template <bool W, bool PL>
 __global__ __launch_bounds__(256) void k_ii_pressure_accel(SceneTab T, DevArrays A) {
   ALV_SCENE(T, A, s);
+  if (must_wait(A)) return;
   if (s >= p.first + p.n) return;
   const vec3 xi = ld3(A.x[s]);
   const float dens = A.density[s];
@@ -2472,6 +2488,7 @@ __global__ __launch_bounds__(256) void k_ii_pressure_accel(SceneTab T, DevArrays
 template <bool W>
 __global__ __launch_bounds__(256) void k_ii_finish(SceneTab T, DevArrays A) {
   ALV_SCENE(T, A, s);
+  if (must_wait(A)) return;
   if (s >= p.first + p.n) return;
   const float dt = A.ctl->dt;
   const unsigned i = A.sorted_id[s];
@@ -2631,6 +2648,7 @@ __global__ __launch_bounds__(256) void k_is_iter(SceneTab T, DevArrays A) {
 // in the reference.
 __global__ __launch_bounds__(256) void k_is_settle(SceneTab T, DevArrays A) {
   ALV_SCENE(T, A, s);
+  if (must_wait(A)) return;
   if (s >= p.first + p.n) return;
   const unsigned it = A.ctl->dens_iter;
   if (it != 0u && (it & 1u) == 0u) A.pressure[s] = A.last_pressure[s];
@@ -2644,6 +2662,7 @@ __global__ __launch_bounds__(256) void k_is_settle(SceneTab T, DevArrays A) {
 constexpr unsigned kBodyBlocks = 256;
 
 __global__ __launch_bounds__(256) void k_body_partials(SceneTab T, DevArrays A) {
+  if (must_wait(A)) return;
   __shared__ double lds[4];
   const SimParams p = T.par[0];
   const unsigned b = blockIdx.y;
@@ -2670,6 +2689,7 @@ __global__ __launch_bounds__(256) void k_body_partials(SceneTab T, DevArrays A) 
 }
 
 __global__ __launch_bounds__(256) void k_body_sums(SceneTab T, DevArrays A, unsigned nblk) {
+  if (must_wait(A)) return;
   __shared__ double lds[4];
   const SimParams p = T.par[0];
   const unsigned b = blockIdx.x;
@@ -3011,6 +3031,7 @@ __global__ __launch_bounds__(256) void k_extrapolate(SceneTab T, DevArrays A, in
   ALV_SCENE_LINEAR(T, A, s);
   if (s >= p.n) return;
   if (!final_pressure && A.ctl->dens_done) return;
+  if (must_wait(A)) return;
   const float* src = (final_pressure || (A.ctl->dens_iter & 1u) != 0u) ? A.pressure
                                                                         : A.last_pressure;
   const vec3 xi = ld3(A.px[s]);
