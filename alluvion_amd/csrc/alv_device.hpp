@@ -617,6 +617,24 @@ __device__ inline vec3 wrap_disp(vec3 d, const SimParams& p) {
   return d;
 }
 
+// --- four lanes per item (a DPP quad) ----------------------------------------
+// bit q set when lane q of the quad hits
+__device__ inline unsigned quad_bits(bool hit, unsigned q) {
+  int b = hit ? int(1u << q) : 0;
+  b |= __builtin_amdgcn_mov_dpp(b, 0xB1, 0xf, 0xf, true);  // lanes 1 0 3 2
+  b |= __builtin_amdgcn_mov_dpp(b, 0x4E, 0xf, 0xf, true);  // lanes 2 3 0 1
+  return unsigned(b);
+}
+// acc + (the quad's lanes' t, in lane order); every lane holds the sum
+__device__ inline float quad_add(float acc, float t) {
+  const int b = __float_as_int(t);
+  acc += __int_as_float(__builtin_amdgcn_mov_dpp(b, 0x00, 0xf, 0xf, true));
+  acc += __int_as_float(__builtin_amdgcn_mov_dpp(b, 0x55, 0xf, 0xf, true));
+  acc += __int_as_float(__builtin_amdgcn_mov_dpp(b, 0xAA, 0xf, 0xf, true));
+  acc += __int_as_float(__builtin_amdgcn_mov_dpp(b, 0xFF, 0xf, 0xf, true));
+  return acc;
+}
+
 // Block index remapped so that each of the 8 XCDs (which receive blocks
 // round-robin) works on one contiguous range of particles: neighbouring
 // particles then share an XCD's L2.

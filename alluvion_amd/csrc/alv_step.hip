@@ -1204,13 +1204,6 @@ __device__ inline float velocity_divergence_deep(const SimParams& p, const DevAr
 // the terms in slot order.
 // ---------------------------------------------------------------------------
 constexpr unsigned kQuadList = 64;  // list slots kept in LDS; later ones go to the list at once
-// bit q set when lane q of the quad hits
-__device__ inline unsigned quad_bits(bool hit, unsigned q) {
-  int b = hit ? int(1u << q) : 0;
-  b |= __builtin_amdgcn_mov_dpp(b, 0xB1, 0xf, 0xf, true);  // lanes 1 0 3 2
-  b |= __builtin_amdgcn_mov_dpp(b, 0x4E, 0xf, 0xf, true);  // lanes 2 3 0 1
-  return unsigned(b);
-}
 template <bool W>
 __global__ __launch_bounds__(64) void k_neighbors_quad(SceneTab T, DevArrays A, int with_factor) {
   __shared__ unsigned list_[kQuadList][16];

@@ -75,3 +75,34 @@ def test_periodic_boxes(cells, wrap, margin, kind):
 @pytest.mark.parametrize("n", [81920, 81921, 98304, 98305])
 def test_both_sides_of_the_limits(n, wrap):
     step_matches(cloud(n, (22, 24, 20), 7, wrap=wrap))
+
+
+@pytest.mark.parametrize("ns", [1, 15, 65, 300])
+@pytest.mark.parametrize("kmax,wrap", [(7, None), (64, None), (40, (True, True, True)),
+                                       (64, (True, False, True))])
+def test_sample_lists(ns, kmax, wrap):
+    sc = cloud(900, (6, 5 if wrap is None else 6, 6), 9, wrap=wrap, kmax=kmax)
+    dp, pile, solver, _, _ = scenes.build_solver(sc)
+    solver.update_particle_neighbors()
+    orc = oracle_for(sc, dp, [])
+    orc.update_particle_neighbors()
+    rng = np.random.default_rng(ns)
+    pts = ((rng.random((ns, 3)) - 0.5) * 0.07).astype(np.float32)  # some outside the grid
+    pts[:ns // 3] = sc.x[:ns // 3]  # the particle of the sample's own index is left out
+    sx = dp.create_coated((ns,), 3)
+    sx.set(pts)
+    nbr, cnt = dp.create((ns, kmax), 4), dp.create((ns,), 1, np.uint32)
+    runner = dp.Runner()
+    runner.launch_make_neighbor_list(sx, solver.pid, solver.pid_length, nbr, cnt, solver.grid_anomaly,
+                                     ns)
+    ids, xixj, counts = orc.sample_neighbors(pts)
+    np.testing.assert_array_equal(dp.coat(cnt).get(), counts)
+    got = dp.coat(nbr).get().reshape(ns, kmax, 4)
+    for k in range(ns):
+        c = counts[k]
+        np.testing.assert_array_equal(got[k, :c, 3].view(np.uint32), ids[k, :c])
+        np.testing.assert_array_equal(got[k, :c, :3], xixj[k, :c].astype(np.float32))
+    out = dp.create((ns,), 1)
+    runner.launch_sample_fluid_density(nbr, cnt, out, ns)
+    want = orc.sample_density(xixj, counts)
+    assert np.abs(dp.coat(out).get() - want).max() <= 1e-5 * max(np.abs(want).max(), 1e-30)
