@@ -39,6 +39,9 @@ namespace {
 
 constexpr unsigned kChunk = 2048;  // samples per weight-gradient partial
 constexpr unsigned kWgradJobs = 53;
+// steps whose losses stay on the device before they are fetched (512 KB at a
+// batch of 65,536)
+constexpr unsigned kLossSteps = 64;
 
 __global__ __launch_bounds__(256) void k_mlp_pack(const float* __restrict__ P,
                                                   bf16x8* __restrict__ ops) {
@@ -93,48 +96,79 @@ __device__ inline uint64_t mix64(uint64_t z) {
   return z ^ (z >> 31);
 }
 
-__global__ __launch_bounds__(256) void k_mlp_gather(const float* __restrict__ X,
-                                                    const float* __restrict__ Y, uint64_t n_data,
-                                                    const float* __restrict__ norm, uint64_t seed,
-                                                    unsigned step, unsigned B,
-                                                    float* __restrict__ xn,
-                                                    float* __restrict__ tn) {
-  const unsigned i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= B) return;
-  const uint64_t idx = mix64(seed ^ mix64((uint64_t(step) << 32) | i)) % n_data;
+// Where a batch comes from: normalised samples, or a random draw from raw
+// data, normalised on the way.
+struct Batch {
+  const float* x;
+  const float* y;
+  uint64_t n_data;  // 0: x, y are the normalised batch itself
+  const float* norm;
+  uint64_t seed;
+  unsigned step;
+};
+__device__ inline void batch_sample(const Batch& D, unsigned i, float (&x)[kMlpIn],
+                                    float (&y)[kMlpOut]) {
+  if (D.n_data == 0) {
+#pragma unroll
+    for (int k = 0; k < kMlpIn; ++k) x[k] = D.x[size_t(i) * kMlpIn + k];
+#pragma unroll
+    for (int o = 0; o < kMlpOut; ++o) y[o] = D.y[size_t(i) * kMlpOut + o];
+    return;
+  }
+  const uint64_t idx = mix64(D.seed ^ mix64((uint64_t(D.step) << 32) | i)) % D.n_data;
 #pragma unroll
   for (int k = 0; k < kMlpIn; ++k)
-    xn[size_t(i) * kMlpIn + k] = (X[idx * kMlpIn + k] - norm[k]) * norm[kMlpIn + k];
+    x[k] = (D.x[idx * kMlpIn + k] - D.norm[k]) * D.norm[kMlpIn + k];
 #pragma unroll
   for (int o = 0; o < kMlpOut; ++o)
-    tn[size_t(i) * kMlpOut + o] =
-        (Y[idx * kMlpOut + o] - norm[2 * kMlpIn + o]) / norm[2 * kMlpIn + 2 + o];
+    y[o] = (D.y[idx * kMlpOut + o] - D.norm[2 * kMlpIn + o]) / D.norm[2 * kMlpIn + 2 + o];
 }
 
+// Activations and deltas of a batch, in tiles of 16 samples: [B/16][rows][16],
+// so a wave writes its tile of 64 rows as 2 KB in a piece and the weight
+// gradients read eight samples of a row as 16 bytes, 32 lanes to 512 bytes.
 struct TrainBufs {
-  __bf16* U;    // [8][B]
-  __bf16* A1;   // [64][B]
+  __bf16* U;    // 8 rows
+  __bf16* A1;   // 64 rows
   __bf16* A2;
   __bf16* A3;
-  __bf16* DY;   // [2][B]
-  __bf16* DZ3;  // [64][B]
+  __bf16* DY;   // 2 rows
+  __bf16* DZ3;  // 64 rows
   __bf16* DZ2;
   __bf16* DZ1;
 };
 
-__device__ inline void store_operands(__bf16* dst, const bf16x8 (&op)[2], int g, unsigned p,
-                                      unsigned B) {
+// The wave's 64 rows x 16 samples go through its LDS tile: the registers hold
+// one sample per lane (2-byte stores to 64 lines each), the tile is stored
+// with two 16-byte stores per lane.
+constexpr int kTileHalfs = kMlpHid * 16;
+__device__ inline void store_tile(__bf16* dst, const __bf16* tile, unsigned tile_index, int lane) {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  const uint4* src = reinterpret_cast<const uint4*>(tile);
+  uint4* out = reinterpret_cast<uint4*>(dst + size_t(tile_index) * kTileHalfs);
+  out[lane] = src[lane];
+  out[64 + lane] = src[64 + lane];
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+__device__ inline void store_operands(__bf16* dst, const bf16x8 (&op)[2], int g, int c,
+                                      __bf16* tile, unsigned tile_index, int lane) {
 #pragma unroll
   for (int s = 0; s < 2; ++s)
 #pragma unroll
-    for (int j = 0; j < 8; ++j) dst[size_t(hperm(s, g, j)) * B + p] = op[s][j];
+    for (int j = 0; j < 8; ++j) tile[hperm(s, g, j) * 16 + c] = op[s][j];
+  store_tile(dst, tile, tile_index, lane);
 }
-__device__ inline void store_tiles(__bf16* dst, const f32x4 (&t)[4], int g, unsigned p,
-                                   unsigned B) {
+__device__ inline void store_tiles(__bf16* dst, const f32x4 (&t)[4], int g, int c, __bf16* tile,
+                                   unsigned tile_index, int lane) {
 #pragma unroll
   for (int m = 0; m < 4; ++m)
 #pragma unroll
-    for (int r = 0; r < 4; ++r) dst[size_t(m * 16 + 4 * g + r) * B + p] = (__bf16)t[m][r];
+    for (int r = 0; r < 4; ++r) tile[(m * 16 + 4 * g + r) * 16 + c] = (__bf16)t[m][r];
+  store_tile(dst, tile, tile_index, lane);
 }
 // delta tiles: round to bf16 once, so that the stored value and the operand
 // of the next product are the same number
@@ -145,81 +179,91 @@ __device__ inline void round_tiles(f32x4 (&t)[4]) {
     for (int r = 0; r < 4; ++r) t[m][r] = float((__bf16)t[m][r]);
 }
 
-// Forward + backward of tiles of 16 samples (B a multiple of 16).  Every
-// lane of every wave reaches the MFMAs; there is no early return.
-__global__ __launch_bounds__(256) void k_mlp_fwd_bwd(MlpDev M, const float* __restrict__ xn,
-                                                     const float* __restrict__ tn, unsigned B,
-                                                     TrainBufs T, double* __restrict__ loss_part) {
+// Forward + backward, one tile of 16 samples per wave (B a multiple of 64).
+// Every lane of every wave reaches the MFMAs; there is no early return.  Bound
+// by the latency of a chain of seven layers at two waves per SIMD (189 VGPRs);
+// 65,536 samples write 51 MB of activations and deltas.  It takes 30 us with
+// the draw of the batch, against 43 and a 6 us gather before: a loop over
+// tiles kept all weight operands in registers (256 VGPRs, one wave per SIMD),
+// and bounds of three or four waves spill (64 and 39 us).
+__global__ __launch_bounds__(256) void k_mlp_fwd_bwd(MlpDev M, Batch D, unsigned B, TrainBufs T,
+                                                     double* __restrict__ loss_part) {
+  __shared__ __align__(16) __bf16 tiles_[4][kTileHalfs];
   const int lane = threadIdx.x & 63, g = lane >> 4, c = lane & 15;
-  const unsigned wave = (blockIdx.x * blockDim.x + threadIdx.x) >> 6;
-  const unsigned n_waves = (gridDim.x * blockDim.x) >> 6;
-  const unsigned n_tiles = B / 16;
+  __bf16* lt = tiles_[threadIdx.x >> 6];
+  const unsigned tile = (blockIdx.x * blockDim.x + threadIdx.x) >> 6;  // the wave's (B / 64 blocks)
   const bf16x8* ops = M.ops;
   const float scale = 2.0f / float(B);
   float loss = 0.0f;
-  for (unsigned tile = wave; tile < n_tiles; tile += n_waves) {
-    const unsigned p = tile * 16 + c;
-    bf16x8 u;
+  float xs[kMlpIn], ts[kMlpOut];
+  if (g == 0) {
+    batch_sample(D, tile * 16 + c, xs, ts);
+  } else {
 #pragma unroll
-    for (int k = 0; k < kMlpIn; ++k) u[k] = (__bf16)(g == 0 ? xn[size_t(p) * kMlpIn + k] : 0.0f);
-    MlpTileState S;
-    mlp_forward_tile(M, u, lane, S);
-    // output delta (rows 0, 1 live in lanes of group 0)
-    bf16x8 dyop;
+    for (int k = 0; k < kMlpIn; ++k) xs[k] = 0.0f;
 #pragma unroll
-    for (int j = 0; j < 8; ++j) dyop[j] = (__bf16)0.0f;
-    if (g == 0) {
-#pragma unroll
-      for (int o = 0; o < kMlpOut; ++o) {
-        const float e = S.y[o] - tn[size_t(p) * kMlpOut + o];
-        loss += e * e;
-        const __bf16 d = (__bf16)(scale * e);
-        dyop[o] = d;
-        T.DY[size_t(o) * B + p] = d;
-      }
-#pragma unroll
-      for (int k = 0; k < kMlpIn; ++k) T.U[size_t(k) * B + p] = u[k];
-    }
-    store_operands(T.A1, S.a1, g, p, B);
-    store_operands(T.A2, S.a2, g, p, B);
-    store_operands(T.A3, S.a3, g, p, B);
-    // layer 4 -> 3
-    f32x4 d[4];
-    const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int m = 0; m < 4; ++m) {
-      d[m] = mfma16x16x32(ops[kOpsT4 + m * 64 + lane], dyop, zero);
-#pragma unroll
-      for (int r = 0; r < 4; ++r) d[m][r] *= mlp_silu_grad(S.z3[m][r]);
-    }
-    round_tiles(d);
-    store_tiles(T.DZ3, d, g, p, B);
-    bf16x8 dop[2];
-    tiles_to_operands(d, dop);
-    // layer 3 -> 2
-#pragma unroll
-    for (int m = 0; m < 4; ++m) {
-      f32x4 acc = mfma16x16x32(ops[kOpsT3 + (m * 2 + 0) * 64 + lane], dop[0], zero);
-      acc = mfma16x16x32(ops[kOpsT3 + (m * 2 + 1) * 64 + lane], dop[1], acc);
-#pragma unroll
-      for (int r = 0; r < 4; ++r) acc[r] *= mlp_silu_grad(S.z2[m][r]);
-      d[m] = acc;
-    }
-    round_tiles(d);
-    store_tiles(T.DZ2, d, g, p, B);
-    tiles_to_operands(d, dop);
-    // layer 2 -> 1
-#pragma unroll
-    for (int m = 0; m < 4; ++m) {
-      f32x4 acc = mfma16x16x32(ops[kOpsT2 + (m * 2 + 0) * 64 + lane], dop[0], zero);
-      acc = mfma16x16x32(ops[kOpsT2 + (m * 2 + 1) * 64 + lane], dop[1], acc);
-#pragma unroll
-      for (int r = 0; r < 4; ++r) acc[r] *= mlp_silu_grad(S.z1[m][r]);
-      d[m] = acc;
-    }
-    round_tiles(d);
-    store_tiles(T.DZ1, d, g, p, B);
+    for (int o = 0; o < kMlpOut; ++o) ts[o] = 0.0f;
   }
+  bf16x8 u;
+#pragma unroll
+  for (int k = 0; k < kMlpIn; ++k) u[k] = (__bf16)xs[k];
+  MlpTileState S;
+  mlp_forward_tile(M, u, lane, S);
+  // output delta (rows 0, 1 live in lanes of group 0)
+  bf16x8 dyop;
+#pragma unroll
+  for (int j = 0; j < 8; ++j) dyop[j] = (__bf16)0.0f;
+  if (g == 0) {
+#pragma unroll
+    for (int o = 0; o < kMlpOut; ++o) {
+      const float e = S.y[o] - ts[o];
+      loss += e * e;
+      const __bf16 d = (__bf16)(scale * e);
+      dyop[o] = d;
+      T.DY[(size_t(tile) * kMlpOut + o) * 16 + c] = d;
+    }
+#pragma unroll
+    for (int k = 0; k < kMlpIn; ++k) T.U[(size_t(tile) * kMlpIn + k) * 16 + c] = u[k];
+  }
+  store_operands(T.A1, S.a1, g, c, lt, tile, lane);
+  store_operands(T.A2, S.a2, g, c, lt, tile, lane);
+  store_operands(T.A3, S.a3, g, c, lt, tile, lane);
+  // layer 4 -> 3
+  f32x4 d[4];
+  const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int m = 0; m < 4; ++m) {
+    d[m] = mfma16x16x32(ops[kOpsT4 + m * 64 + lane], dyop, zero);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) d[m][r] *= mlp_silu_grad(S.z3[m][r]);
+  }
+  round_tiles(d);
+  store_tiles(T.DZ3, d, g, c, lt, tile, lane);
+  bf16x8 dop[2];
+  tiles_to_operands(d, dop);
+  // layer 3 -> 2
+#pragma unroll
+  for (int m = 0; m < 4; ++m) {
+    f32x4 acc = mfma16x16x32(ops[kOpsT3 + (m * 2 + 0) * 64 + lane], dop[0], zero);
+    acc = mfma16x16x32(ops[kOpsT3 + (m * 2 + 1) * 64 + lane], dop[1], acc);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) acc[r] *= mlp_silu_grad(S.z2[m][r]);
+    d[m] = acc;
+  }
+  round_tiles(d);
+  store_tiles(T.DZ2, d, g, c, lt, tile, lane);
+  tiles_to_operands(d, dop);
+  // layer 2 -> 1
+#pragma unroll
+  for (int m = 0; m < 4; ++m) {
+    f32x4 acc = mfma16x16x32(ops[kOpsT2 + (m * 2 + 0) * 64 + lane], dop[0], zero);
+    acc = mfma16x16x32(ops[kOpsT2 + (m * 2 + 1) * 64 + lane], dop[1], acc);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) acc[r] *= mlp_silu_grad(S.z1[m][r]);
+    d[m] = acc;
+  }
+  round_tiles(d);
+  store_tiles(T.DZ1, d, g, c, lt, tile, lane);
   // block sum of the squared errors
   __shared__ float red[256];
   red[threadIdx.x] = loss;
@@ -232,6 +276,9 @@ __global__ __launch_bounds__(256) void k_mlp_fwd_bwd(MlpDev M, const float* __re
 }
 
 // One wave per (job, chunk).  Jobs 0-39: weight tiles; 40-52: bias tiles.
+// Bound by the latency of its loads: 32 lanes read 512 contiguous bytes of a
+// tile and eight steps are in flight, 20 us for 65,536 samples (27 with one
+// step in flight and rows a batch apart).
 struct WgradJob {
   int layer;   // 1..4
   int mt, nt;  // output-unit tile, input-unit tile (nt < 0: bias)
@@ -271,13 +318,23 @@ __global__ __launch_bounds__(64) void k_mlp_wgrad(TrainBufs T, unsigned B,
     zeros[j] = (__bf16)0.0f;
   }
   f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-  for (unsigned p0 = p_begin; p0 < p_begin + kChunk; p0 += 32) {
-    const unsigned p = p0 + 8 * g;
-    const bf16x8 a = a_ok ? *reinterpret_cast<const bf16x8*>(dz + size_t(arow) * B + p) : zeros;
-    const bf16x8 b = J.nt < 0 ? ones
-                     : (b_ok ? *reinterpret_cast<const bf16x8*>(ain + size_t(brow) * B + p)
-                             : zeros);
-    acc = mfma16x16x32(a, b, acc);
+  // eight steps' operands are loaded together (rows past the layer's from row
+  // 0, then zeroed): one latency for eight products
+  constexpr unsigned kDepth = 8;
+  static_assert(kChunk % (32u * kDepth) == 0u, "whole groups of steps");
+  const int arow_l = a_ok ? arow : 0, brow_l = b_ok ? brow : 0;
+  for (unsigned p0 = p_begin; p0 < p_begin + kChunk; p0 += 32u * kDepth) {
+    bf16x8 a[kDepth], b[kDepth];
+#pragma unroll
+    for (unsigned k = 0; k < kDepth; ++k) {
+      const unsigned p = p0 + 32u * k + 8 * g, tile = p >> 4, half = p & 8u;
+      a[k] = *reinterpret_cast<const bf16x8*>(dz + (size_t(tile) * n_out + arow_l) * 16 + half);
+      if (J.nt >= 0)
+        b[k] = *reinterpret_cast<const bf16x8*>(ain + (size_t(tile) * n_in + brow_l) * 16 + half);
+    }
+#pragma unroll
+    for (unsigned k = 0; k < kDepth; ++k)
+      acc = mfma16x16x32(a_ok ? a[k] : zeros, J.nt < 0 ? ones : (b_ok ? b[k] : zeros), acc);
   }
   float* out = partials + size_t(chunk) * kMlpParams;
 #pragma unroll
@@ -302,14 +359,20 @@ __global__ __launch_bounds__(256) void k_mlp_reduce(const float* __restrict__ pa
   grad[k] = float(s);
 }
 
-__global__ __launch_bounds__(256) void k_mlp_adam(float* __restrict__ P, float* __restrict__ m1,
-                                                  float* __restrict__ m2,
-                                                  const float* __restrict__ grad, float lr,
-                                                  float c1, float c2) {
+// The reduction and Adam in one pass over the parameters; 64-thread blocks
+// put the 9,026 parameters on 142 CUs (5 us; a reduction of 256-thread blocks
+// and a pass of its own took 14 and 4).
+__global__ __launch_bounds__(64) void k_mlp_adam(const float* __restrict__ partials,
+                                                 unsigned n_chunks, float* __restrict__ P,
+                                                 float* __restrict__ m1, float* __restrict__ m2,
+                                                 float lr, float c1, float c2) {
   const unsigned k = blockIdx.x * blockDim.x + threadIdx.x;
   if (k >= unsigned(kMlpParams)) return;
+  double s = 0.0;
+#pragma unroll 8
+  for (unsigned ch = 0; ch < n_chunks; ++ch) s += partials[size_t(ch) * kMlpParams + k];
   const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
-  const float gk = grad[k];
+  const float gk = float(s);
   const float a = b1 * m1[k] + (1.0f - b1) * gk;
   const float b = b2 * m2[k] + (1.0f - b2) * gk * gk;
   m1[k] = a;
@@ -375,14 +438,15 @@ struct DevBuf {
   }
 };
 
-int alloc_train(alv_mlp* m, unsigned B, DevBuf& blob, TrainBufs& T, float** xn, float** tn,
+// loss_steps: steps whose block losses are kept on the device at a time
+int alloc_train(alv_mlp* m, unsigned B, unsigned loss_steps, DevBuf& blob, TrainBufs& T,
                 float** partials, double** loss_part, unsigned* fb_blocks) {
   const size_t per = size_t(B) * sizeof(__bf16);
   const unsigned n_chunks = B / kChunk;
-  *fb_blocks = std::min(1024u, (B / 16 + 3) / 4);
-  const size_t bytes = per * (8 + 64 * 3 + 2 + 64 * 3) + size_t(B) * (8 + 2) * sizeof(float) +
+  *fb_blocks = B / 64u;
+  const size_t bytes = per * (8 + 64 * 3 + 2 + 64 * 3) +
                        size_t(n_chunks) * kMlpParams * sizeof(float) +
-                       size_t(*fb_blocks) * sizeof(double) + 16 * 256;
+                       size_t(loss_steps) * *fb_blocks * sizeof(double) + 16 * 256;
   MLP_HIP(hipMalloc(&blob.p, bytes));
   char* q = static_cast<char*>(blob.p);
   auto take = [&](size_t n) {
@@ -398,22 +462,18 @@ int alloc_train(alv_mlp* m, unsigned B, DevBuf& blob, TrainBufs& T, float** xn, 
   T.DZ3 = reinterpret_cast<__bf16*>(take(per * 64));
   T.DZ2 = reinterpret_cast<__bf16*>(take(per * 64));
   T.DZ1 = reinterpret_cast<__bf16*>(take(per * 64));
-  *xn = reinterpret_cast<float*>(take(size_t(B) * 8 * sizeof(float)));
-  *tn = reinterpret_cast<float*>(take(size_t(B) * 2 * sizeof(float)));
   *partials = reinterpret_cast<float*>(take(size_t(n_chunks) * kMlpParams * sizeof(float)));
-  *loss_part = reinterpret_cast<double*>(take(size_t(*fb_blocks) * sizeof(double)));
+  *loss_part = reinterpret_cast<double*>(take(size_t(loss_steps) * *fb_blocks * sizeof(double)));
   return ALV_OK;
 }
 
-// gradient of the normalised batch (xn, tn already on the device)
-int grad_batch(alv_mlp* m, const float* xn, const float* tn, unsigned B, TrainBufs& T,
-               float* partials, double* loss_part, unsigned fb_blocks) {
-  hipLaunchKernelGGL(k_mlp_fwd_bwd, dim3(fb_blocks), dim3(256), 0, m->stream, m->dev(), xn, tn,
-                     B, T, loss_part);
+// forward, backward and the weight gradients' partial sums of a batch
+int grad_batch(alv_mlp* m, const Batch& D, unsigned B, TrainBufs& T, float* partials,
+               double* loss_part, unsigned fb_blocks) {
+  hipLaunchKernelGGL(k_mlp_fwd_bwd, dim3(fb_blocks), dim3(256), 0, m->stream, m->dev(), D, B, T,
+                     loss_part);
   hipLaunchKernelGGL(k_mlp_wgrad, dim3(kWgradJobs, B / kChunk), dim3(64), 0, m->stream, T, B,
                      partials);
-  hipLaunchKernelGGL(k_mlp_reduce, dim3((kMlpParams + 255) / 256), dim3(256), 0, m->stream,
-                     partials, B / kChunk, m->grad);
   MLP_HIP(hipGetLastError());
   return ALV_OK;
 }
@@ -577,13 +637,16 @@ int alv_mlp_loss_grad(alv_mlp* m, const float* dev_xn, const float* dev_tn, size
   const unsigned B = unsigned(n);
   DevBuf blob;
   TrainBufs T;
-  float *xn, *tn, *partials;
+  float* partials;
   double* loss_part;
   unsigned fb;
-  rc = alloc_train(m, B, blob, T, &xn, &tn, &partials, &loss_part, &fb);
+  rc = alloc_train(m, B, 1, blob, T, &partials, &loss_part, &fb);
   if (rc != ALV_OK) return rc;
-  rc = grad_batch(m, dev_xn, dev_tn, B, T, partials, loss_part, fb);
+  rc = grad_batch(m, Batch{dev_xn, dev_tn, 0, nullptr, 0, 0}, B, T, partials, loss_part, fb);
   if (rc != ALV_OK) return rc;
+  hipLaunchKernelGGL(k_mlp_reduce, dim3((kMlpParams + 255) / 256), dim3(256), 0, m->stream,
+                     partials, B / kChunk, m->grad);
+  MLP_HIP(hipGetLastError());
   std::vector<double> lp(fb);
   MLP_HIP(hipMemcpyAsync(host_grad, m->grad, kMlpParams * sizeof(float), hipMemcpyDeviceToHost,
                          m->stream));
@@ -604,31 +667,34 @@ int alv_mlp_train(alv_mlp* m, const float* dev_x, const float* dev_y, size_t n,
   if (rc != ALV_OK) return rc;
   DevBuf blob;
   TrainBufs T;
-  float *xn, *tn, *partials;
+  float* partials;
   double* loss_part;
   unsigned fb;
-  rc = alloc_train(m, batch, blob, T, &xn, &tn, &partials, &loss_part, &fb);
+  const unsigned keep = std::max(1u, std::min(steps, kLossSteps));
+  rc = alloc_train(m, batch, keep, blob, T, &partials, &loss_part, &fb);
   if (rc != ALV_OK) return rc;
-  std::vector<double> lp(fb);
+  std::vector<double> lp(size_t(keep) * fb);
   for (unsigned st = 0; st < steps; ++st) {
-    hipLaunchKernelGGL(k_mlp_gather, dim3((batch + 255) / 256), dim3(256), 0, m->stream, dev_x,
-                       dev_y, uint64_t(n), m->norm, uint64_t(seed), st, batch, xn, tn);
-    rc = grad_batch(m, xn, tn, batch, T, partials, loss_part, fb);
+    const Batch D{dev_x, dev_y, uint64_t(n), m->norm, uint64_t(seed), st};
+    rc = grad_batch(m, D, batch, T, partials, loss_part + size_t(st % keep) * fb, fb);
     if (rc != ALV_OK) return rc;
     ++m->adam_t;
     const float c1 = 1.0f - std::pow(0.9f, float(m->adam_t));
     const float c2 = 1.0f - std::pow(0.999f, float(m->adam_t));
-    hipLaunchKernelGGL(k_mlp_adam, dim3((kMlpParams + 255) / 256), dim3(256), 0, m->stream,
-                       m->params, m->adam_m, m->adam_v, m->grad, lr, c1, c2);
+    hipLaunchKernelGGL(k_mlp_adam, dim3((kMlpParams + 63) / 64), dim3(64), 0, m->stream, partials,
+                       batch / kChunk, m->params, m->adam_m, m->adam_v, lr, c1, c2);
     rc = pack(m);
     if (rc != ALV_OK) return rc;
-    if (host_loss) {
-      MLP_HIP(hipMemcpyAsync(lp.data(), loss_part, fb * sizeof(double), hipMemcpyDeviceToHost,
-                             m->stream));
+    const unsigned held = st % keep + 1u;
+    if (host_loss && (held == keep || st + 1u == steps)) {
+      MLP_HIP(hipMemcpyAsync(lp.data(), loss_part, size_t(held) * fb * sizeof(double),
+                             hipMemcpyDeviceToHost, m->stream));
       MLP_HIP(hipStreamSynchronize(m->stream));
-      double L = 0;
-      for (double v : lp) L += v;
-      host_loss[st] = float(L / double(batch));
+      for (unsigned k = 0; k < held; ++k) {
+        double L = 0;
+        for (unsigned b = 0; b < fb; ++b) L += lp[size_t(k) * fb + b];
+        host_loss[st + 1u - held + k] = float(L / double(batch));
+      }
     }
   }
   MLP_HIP(hipStreamSynchronize(m->stream));

@@ -87,6 +87,49 @@ def test_gradient_matches_oracle():
     assert np.linalg.norm(g - eg) > np.linalg.norm(g - og)
 
 
+@pytest.mark.parametrize("steps", [1, 63, 64, 65, 130])
+def test_drawn_batches_and_losses(steps):
+    """Training's first step against the gradient of the batch it draws, and
+    the losses of runs that end before, at and after a fetch of 64 steps."""
+    import alluvion_amd._alluvion as al
+    dp = Depot(np.float32)
+    rng = np.random.default_rng(41)
+    n, batch, seed = 5003, 2048, 9
+    x = rng.standard_normal((n, 8)).astype(np.float32)
+    t = rng.standard_normal((n, 2)).astype(np.float32)
+    p = random_params(42)
+    X, T = device_array(dp, x), device_array(dp, t)
+
+    def trained(k):
+        net = al.WarmStartNet(0)
+        net.set_params(p)
+        return net.train(X, T, n, batch, k, 1e-3, seed), net
+
+    losses, net = trained(steps)
+    assert len(losses) == steps
+    if steps > 1:  # the steps of a run do not depend on its length
+        assert np.array_equal(losses, trained(150)[0][:steps])
+        return
+    mask = (1 << 64) - 1
+
+    def mix(z):
+        z = (z + 0x9E3779B97F4A7C15) & mask
+        z = ((z ^ (z >> 30)) * 0xBF58476D1CE4E5B9) & mask
+        z = ((z ^ (z >> 27)) * 0x94D049BB133111EB) & mask
+        return z ^ (z >> 31)
+
+    idx = [mix(seed ^ mix(i)) % n for i in range(batch)]
+    plain = al.WarmStartNet(0)
+    plain.set_params(p)
+    loss, g = plain.loss_grad(device_array(dp, x[idx]), device_array(dp, t[idx]), batch)
+    assert np.float32(loss) == np.float32(losses[0])
+    # Adam's first step is lr * g / (|g| + eps'), of sign(g) and size lr; the
+    # parameters (below 8) are rounded to 2^-22 at most
+    moved = p - net.get_params()
+    big = np.abs(g) > 1e-4
+    assert np.all(np.abs(moved[big] - 1e-3 * np.sign(g[big])) <= 1e-3 * 1e-3 + 2.0 ** -22)
+
+
 def test_training_fits_a_smooth_map():
     import alluvion_amd._alluvion as al
     dp = Depot(np.float32)
