@@ -304,6 +304,8 @@ struct alv_pile {
   size_t inertia_cap = 0;
   alv_contact* contacts_dev = nullptr;
   unsigned* count_dev = nullptr;
+  unsigned long long* hits_dev = nullptr;  // a bit per contact candidate
+  size_t hits_cap = 0;
   std::vector<alv_contact> contacts;  // host copy of the kept contacts
   unsigned num_found = 0;
   // device kinematics (x, v, q, omega of every body) as of the last copy:
@@ -330,6 +332,7 @@ struct alv_pile {
     if (inertia_dev) (void)hipFree(inertia_dev);
     if (contacts_dev) (void)hipFree(contacts_dev);
     if (count_dev) (void)hipFree(count_dev);
+    if (hits_dev) (void)hipFree(hits_dev);
     if (kin_dev) (void)hipFree(kin_dev);
   }
   // x [B][3], v [B][3], q [B][4], omega [B][3]
@@ -1143,6 +1146,7 @@ int run_collision(alv_pile* P, const std::vector<ContactJob>& jobs, unsigned can
   ALV_HIP(reserve_dev(&P->bodies_dev, &P->bodies_cap, nb));
   ALV_HIP(reserve_dev(&P->inertia_dev, &P->inertia_cap, size_t(nb) * 5));
   ALV_HIP(reserve_dev(&P->jobs_dev, &P->jobs_cap, jobs.size()));
+  ALV_HIP(reserve_dev(&P->hits_dev, &P->hits_cap, collision_hit_words(candidates)));
   if (!P->count_dev) ALV_HIP(hipMalloc(&P->count_dev, sizeof(unsigned)));
   if (!P->contacts_dev && P->max_num_contacts)
     ALV_HIP(hipMalloc(&P->contacts_dev, size_t(P->max_num_contacts) * sizeof(alv_contact)));
@@ -1159,8 +1163,8 @@ int run_collision(alv_pile* P, const std::vector<ContactJob>& jobs, unsigned can
   ALV_HIP(hipMemcpyAsync(P->jobs_dev, jobs.data(), jobs.size() * sizeof(ContactJob),
                          hipMemcpyHostToDevice, stream));
   launch_collision(P->jobs_dev, unsigned(jobs.size()), candidates, nb, P->bodies_dev,
-                   P->inertia_dev, verts, tolerance, P->max_num_contacts, P->contacts_dev,
-                   P->count_dev, stream);
+                   P->inertia_dev, verts, tolerance, P->max_num_contacts, P->hits_dev,
+                   P->contacts_dev, P->count_dev, stream);
   ALV_HIP(hipGetLastError());
   unsigned found = 0;
   ALV_HIP(hipMemcpyAsync(&found, P->count_dev, sizeof(unsigned), hipMemcpyDeviceToHost, stream));

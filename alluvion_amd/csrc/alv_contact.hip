@@ -6,11 +6,10 @@
 // body j (box or sphere, in j's frame).  The reference appends contacts with
 // an atomic counter, so their order -- and the result of the sequential
 // Gauss-Seidel contact solve that follows -- depends on thread timing.  Here
-// the candidates are numbered (pair in (i, j) order, then vertex) and one
-// workgroup compacts them with a wave-ballot scan, so contacts come out in
-// that order on every run.  Contact counts are small (the vertices of a few
-// collision meshes), so a single workgroup is enough; the kernel is far from
-// any hardware bound and is not on the fluid's hot path.
+// the candidates are numbered (pair in (i, j) order, then vertex), one pass
+// over all of them leaves a bit per candidate, and a second one places each
+// hit at the number of bits before its own, so contacts come out in that
+// order on every run.
 #include <hip/hip_runtime.h>
 
 #include "alv_contact.hpp"
@@ -19,7 +18,7 @@
 namespace alv {
 namespace {
 
-constexpr unsigned kContactThreads = 1024;
+constexpr unsigned kContactThreads = 256;
 constexpr unsigned kContactWaves = kContactThreads / 64;
 
 // R diag(v) R^T for the rotation of q, stored as diagonal and (01, 02, 12)
@@ -65,11 +64,12 @@ __device__ inline void put3(float* dst, vec3 v) {
   dst[2] = v.z;
 }
 
-// Tests vertex `vert` of body i against body j; true and a filled record
-// when the vertex is inside body j (dist < 0).  World vertices (pellets,
+// Tests vertex `vert` of body i against body j: whether it is inside body j
+// (dist < 0) or, with `Record`, the record of a vertex known to be.  World vertices (pellets,
 // collision_test_with_pellets, runner.hpp:3627-3727) are already placed;
 // body-frame vertices are placed with body i's kinematics.  `inertia`
 // holds [B][3] principal inertia, then [B][2] (restitution, friction).
+template <bool Record>
 __device__ bool test_vertex(unsigned i, unsigned j, unsigned flags, unsigned nb,
                             const BoundaryDev* bodies, const float* inertia, const float* verts,
                             unsigned vert, float tolerance, alv_contact* out) {
@@ -103,7 +103,7 @@ __device__ bool test_vertex(unsigned i, unsigned j, unsigned flags, unsigned nb,
     dist = sdf_eval(Bj, wrt_j) * Bj.sign - tolerance;
     n = sdf_gradient(Bj, wrt_j, 1e-3f) * Bj.sign;
   }
-  if (!(dist < 0)) return false;
+  if (!Record) return dist < 0;
   n = n * (1.0f / sqrtf(length_sqr(n)));
   const vec3 cp_j = rotate(wrt_j - dist * n, qj) + xj;
   const vec3 nw = rotate(n, qj);
@@ -142,54 +142,90 @@ __device__ bool test_vertex(unsigned i, unsigned j, unsigned flags, unsigned nb,
   return true;
 }
 
-__global__ __launch_bounds__(kContactThreads) void k_collision(
+// Candidate c: the last job whose first candidate is not past it.
+template <bool Record>
+__device__ bool test_candidate(unsigned c, const ContactJob* jobs, unsigned num_jobs, unsigned nb,
+                               const BoundaryDev* bodies, const float* inertia,
+                               const float* verts, float tolerance, alv_contact* out) {
+  unsigned lo = 0, hi = num_jobs;
+  while (hi - lo > 1) {
+    const unsigned mid = (lo + hi) / 2;
+    if (jobs[mid].cbase <= c)
+      lo = mid;
+    else
+      hi = mid;
+  }
+  const ContactJob J = jobs[lo];
+  const unsigned local = c - J.cbase;
+  return test_vertex<Record>(J.i, J.j + local % J.nj, J.flags, nb, bodies, inertia, verts,
+                             J.vbase + local / J.nj, tolerance, out);
+}
+
+// One candidate per thread; hits[w]: the candidates 64 w ... that are inside.
+// Bound by the latency of a candidate's chain of loads (job, bodies, vertex),
+// which one workgroup walking the list paid once per 1,024 candidates: 45,000
+// took 90 us; this pass takes 4 and the records 7.
+__global__ __launch_bounds__(kContactThreads) void k_collision_hits(
     const ContactJob* jobs, unsigned num_jobs, unsigned num_candidates, unsigned nb,
     const BoundaryDev* bodies, const float* inertia, const float* verts, float tolerance,
-    unsigned max_contacts, alv_contact* contacts, unsigned* count) {
+    unsigned long long* hits) {
+  const unsigned c = blockIdx.x * kContactThreads + threadIdx.x;
+  const bool hit = c < num_candidates && test_candidate<false>(c, jobs, num_jobs, nb, bodies,
+                                                               inertia, verts, tolerance, nullptr);
+  const unsigned long long mask = __ballot(hit);
+  if ((threadIdx.x & 63) == 0) hits[c / 64] = mask;
+}
+
+// A contact's slot is the number of hits before it: each block counts the
+// bits before its own (8 bytes per 64 candidates, from L2); a block without
+// hits does nothing but the last one, which leaves the total.
+__global__ __launch_bounds__(kContactThreads) void k_collision_records(
+    const ContactJob* jobs, unsigned num_jobs, unsigned num_candidates, unsigned nb,
+    const BoundaryDev* bodies, const float* inertia, const float* verts, float tolerance,
+    const unsigned long long* hits, unsigned max_contacts, alv_contact* contacts,
+    unsigned* count) {
   __shared__ unsigned wave_sum[kContactWaves];
-  __shared__ unsigned base;
+  const unsigned first = blockIdx.x * kContactWaves;  // the block's first word
   const unsigned lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  if (threadIdx.x == 0) base = 0;
+  const bool last = blockIdx.x + 1 == gridDim.x;
+  unsigned long long own = 0;
+  for (unsigned w = 0; w < kContactWaves; ++w) own |= hits[first + w];
+  if (own == 0 && !last) return;
+  unsigned before = 0;
+  for (unsigned w = threadIdx.x; w < first; w += kContactThreads) before += __popcll(hits[w]);
+  for (int m = 32; m > 0; m >>= 1) before += __shfl_xor(before, m);
+  if (lane == 0) wave_sum[wave] = before;
   __syncthreads();
-  for (unsigned c0 = 0; c0 < num_candidates; c0 += kContactThreads) {
-    const unsigned c = c0 + threadIdx.x;
+  before = 0;
+  for (unsigned w = 0; w < kContactWaves; ++w) before += wave_sum[w];
+  for (unsigned w = 0; w < wave; ++w) before += __popcll(hits[first + w]);
+  const unsigned long long mask = hits[first + wave];
+  const unsigned slot = before + __popcll(mask & ((1ull << lane) - 1ull));
+  if (((mask >> lane) & 1ull) && slot < max_contacts) {
     alv_contact rec;
-    bool hit = false;
-    if (c < num_candidates) {
-      unsigned k = 0;
-      while (k + 1 < num_jobs && jobs[k + 1].cbase <= c) ++k;
-      const ContactJob J = jobs[k];
-      const unsigned local = c - J.cbase;
-      hit = test_vertex(J.i, J.j + local % J.nj, J.flags, nb, bodies, inertia, verts,
-                        J.vbase + local / J.nj, tolerance, &rec);
-    }
-    const unsigned long long mask = __ballot(hit);
-    const unsigned before = __popcll(mask & ((1ull << lane) - 1ull));
-    if (lane == 0) wave_sum[wave] = unsigned(__popcll(mask));
-    __syncthreads();
-    unsigned offset = base;
-    for (unsigned w = 0; w < wave; ++w) offset += wave_sum[w];
-    const unsigned slot = offset + before;
-    if (hit && slot < max_contacts) contacts[slot] = rec;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-      unsigned total = 0;
-      for (unsigned w = 0; w < kContactWaves; ++w) total += wave_sum[w];
-      base += total;
-    }
-    __syncthreads();
+    test_candidate<true>(blockIdx.x * kContactThreads + threadIdx.x, jobs, num_jobs, nb, bodies,
+                         inertia, verts, tolerance, &rec);
+    contacts[slot] = rec;
   }
-  if (threadIdx.x == 0) count[0] = base;
+  if (last && threadIdx.x == kContactThreads - 1) count[0] = before + __popcll(mask);
 }
 
 }  // namespace
 
+size_t collision_hit_words(unsigned num_candidates) {
+  return (size_t(num_candidates) + kContactThreads - 1) / kContactThreads * kContactWaves;
+}
+
 void launch_collision(const ContactJob* jobs, unsigned num_jobs, unsigned num_candidates,
                       unsigned nb, const BoundaryDev* bodies, const float* inertia,
                       const float* verts, float tolerance, unsigned max_contacts,
-                      alv_contact* contacts, unsigned* count, hipStream_t s) {
-  hipLaunchKernelGGL(k_collision, dim3(1), dim3(kContactThreads), 0, s, jobs, num_jobs,
-                     num_candidates, nb, bodies, inertia, verts, tolerance, max_contacts,
+                      unsigned long long* hits, alv_contact* contacts, unsigned* count,
+                      hipStream_t s) {
+  const dim3 blocks(unsigned(collision_hit_words(num_candidates) / kContactWaves));
+  hipLaunchKernelGGL(k_collision_hits, blocks, dim3(kContactThreads), 0, s, jobs, num_jobs,
+                     num_candidates, nb, bodies, inertia, verts, tolerance, hits);
+  hipLaunchKernelGGL(k_collision_records, blocks, dim3(kContactThreads), 0, s, jobs, num_jobs,
+                     num_candidates, nb, bodies, inertia, verts, tolerance, hits, max_contacts,
                      contacts, count);
 }
 

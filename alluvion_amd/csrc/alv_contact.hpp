@@ -24,10 +24,14 @@ struct ContactJob {
   unsigned pad;
 };
 
+// Words of `hits`, one bit per candidate in whole blocks.
+size_t collision_hit_words(unsigned num_candidates);
+
 // inertia: [B][3] principal inertia, then [B][2] (restitution, friction)
 void launch_collision(const ContactJob* jobs, unsigned num_jobs, unsigned num_candidates,
                       unsigned nb, const BoundaryDev* bodies, const float* inertia,
                       const float* verts, float tolerance, unsigned max_contacts,
-                      alv_contact* contacts, unsigned* count, hipStream_t s);
+                      unsigned long long* hits, alv_contact* contacts, unsigned* count,
+                      hipStream_t s);
 
 }  // namespace alv

@@ -59,6 +59,24 @@ def test_contacts_and_solve_match_oracle():
     np.testing.assert_allclose(w, rb["omega"], rtol=1e-5, atol=1e-5)
 
 
+@pytest.mark.parametrize("nv", [1, 63, 64, 65, 255, 256, 257, 1025])
+@pytest.mark.parametrize("kept", [512, 40])
+def test_candidates_over_waves_and_blocks(nv, kept):
+    """Contacts numbered over the ends of waves and blocks, with runs of
+    candidates without a hit and a cap inside a block."""
+    rng = np.random.default_rng(nv)
+    verts = f32(rng.uniform(-0.04, 0.04, (nv, 3)))
+    verts[300:600, 1] = 0.04  # a whole block of misses
+    verts[-1, 1] = -0.04
+    sc = contact_scene(verts, (0.05, TOP + 0.01, -0.02), restitution=0.5, friction=0.2)
+    sc.max_num_contacts = kept
+    dp, pile, solver, _, _ = scenes.build_solver(sc)
+    orc = of.Oracle(sc, precision=4)
+    total = orc.find_contacts()
+    assert pile.find_contacts() == total > 0
+    compare_contacts(pile.get_contacts(), of.contact_dicts(orc.contacts()))
+
+
 def test_pair_overloads_and_capacity():
     sc = rotated_sphere_scene()
     sc.max_num_contacts = 7
