@@ -635,6 +635,12 @@ __device__ inline float quad_add(float acc, float t) {
   return acc;
 }
 
+// the same for a vector; lanes whose term is not `ok` add nothing
+__device__ inline vec3 quad_add3(vec3 acc, vec3 t, bool ok) {
+  return mk(quad_add(acc.x, ok ? t.x : 0.0f), quad_add(acc.y, ok ? t.y : 0.0f),
+            quad_add(acc.z, ok ? t.z : 0.0f));
+}
+
 // Block index remapped so that each of the 8 XCDs (which receive blocks
 // round-robin) works on one contiguous range of particles: neighbouring
 // particles then share an XCD's L2.

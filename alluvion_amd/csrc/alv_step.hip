@@ -2837,33 +2837,83 @@ __global__ __launch_bounds__(256) void k_node_positions(GridGeomDev g, float* ou
 // fluid and pellets, where pellet ids follow every fluid id, so each list
 // in (cell, id) order is the same.
 // ---------------------------------------------------------------------------
+// Four lanes per particle, in blocks of 64 threads (16 particles): lane q of
+// a particle looks at every fourth entry, so the lists come out as one lane
+// would write them.
+#define ALV_SCENE_QUAD(T, A, s, q, blk)                                \
+  const unsigned blk_ = (blk);                                         \
+  const unsigned q = threadIdx.x & 3u;                                 \
+  const unsigned s = blk_ * 16u + (threadIdx.x >> 2);                  \
+  const SimParams p = (T).par[(T).blk_scene[blk_ / (kBlock / 16u)]]
 // The 27 cells around x in the reference order (dx outer, dz inner; periodic
-// axes wrapped), each in ascending sorted index: f(j, x - x_j) for every j
-// of `xs` closer than the kernel radius.
-template <bool W, class F>
-__device__ inline void scan_cells(const SimParams& p, const unsigned* cell_start,
-                                  const float4* xs, vec3 x, F&& f) {
+// axes wrapped), each in ascending sorted index: every entry of `xs` closer
+// than the kernel radius goes to `list`, at most kmax, the last slot keeping
+// the latest one.  Returns the number found, the same in the four lanes.
+template <bool W>
+__device__ inline unsigned list_cells(const SimParams& p, const DevArrays& A,
+                                      const unsigned* cell_start, const float4* xs, vec3 x,
+                                      uint4* list, unsigned s, unsigned q) {
   int ip[3];
   cell_ipos(x, p, ip);
-  for (int t = 0; t < 27; ++t) {
-    int q[3] = {ip[0] + t / 9 - 1, ip[1] + (t / 3) % 3 - 1, ip[2] + t % 3 - 1};
-    if constexpr (W) {
+  const unsigned K = p.kmax, below = (1u << q) - 1u;
+  unsigned* row = reinterpret_cast<unsigned*>(list + nbr_group(A, 0u, s));
+  unsigned cnt = 0;
+  // entries [b, e), 16 per round: all loads of a round first
+  auto scan = [&](unsigned b, unsigned e) {
+    for (unsigned j0 = b; j0 < e; j0 += 16u) {
+      float4 xc[4];
+#pragma unroll
+      for (unsigned u = 0; u < 4u; ++u) xc[u] = xs[min(j0 + 4u * u + q, e - 1u)];
+#pragma unroll
+      for (unsigned u = 0; u < 4u; ++u) {
+        const unsigned j = j0 + 4u * u + q;
+        const bool hit = length_sqr(wrapd<W>(x - ld3(xc[u]), p)) < p.h2 && j < e;
+        const unsigned bits = quad_bits(hit, q);
+        const unsigned at = cnt + unsigned(__builtin_popcount(bits & below));
+        cnt += unsigned(__builtin_popcount(bits));
+        if (hit && (at + 1u < K || (bits >> q) == 1u)) {
+          const unsigned slot = min(at, K - 1u);
+          row[(slot >> 2) * 256u + (slot & 3u)] = j;
+        }
+      }
+    }
+  };
+  if (!W || !(p.wrap_mask & 4)) {
+    // the three cells of a column are one span; all spans are found first
+    const int z0 = max(ip[2] - 1, 0), z1 = min(ip[2] + 1, p.res[2] - 1);
+    unsigned jb[9], je[9];
+#pragma unroll
+    for (int r = 0; r < 9; ++r) {
+      int nx = ip[0] + r / 3 - 1, ny = ip[1] + r % 3 - 1;
+      if (W && (p.wrap_mask & 1)) nx = nx >= p.res[0] ? nx - p.res[0] : (nx < 0 ? nx + p.res[0] : nx);
+      if (W && (p.wrap_mask & 2)) ny = ny >= p.res[1] ? ny - p.res[1] : (ny < 0 ? ny + p.res[1] : ny);
+      const bool ok = z0 <= z1 && nx >= 0 && nx < p.res[0] && ny >= 0 && ny < p.res[1];
+      const unsigned c = p.cell_base + (unsigned(ok ? nx : 0) * unsigned(p.res[1]) +
+                                        unsigned(ok ? ny : 0)) * unsigned(p.res[2]);
+      jb[r] = cell_start[c + unsigned(ok ? z0 : 0)];
+      je[r] = cell_start[c + unsigned(ok ? z1 : 0) + 1u];
+      if (!ok) jb[r] = je[r] = 0u;
+    }
+#pragma unroll
+    for (int r = 0; r < 9; ++r) scan(jb[r], je[r]);
+  } else {
+    for (int t = 0; t < 27; ++t) {
+      int c3[3] = {ip[0] + t / 9 - 1, ip[1] + (t / 3) % 3 - 1, ip[2] + t % 3 - 1};
       for (int a = 0; a < 3; ++a)
         if (p.wrap_mask & (1 << a))
-          q[a] = q[a] >= p.res[a] ? q[a] - p.res[a] : (q[a] < 0 ? q[a] + p.res[a] : q[a]);
-    }
-    if (!within_grid(q, p)) continue;
-    const unsigned c = p.cell_base + cell_linear(q, p);
-    const unsigned e = cell_start[c + 1];
-    for (unsigned j = cell_start[c]; j < e; ++j) {
-      const vec3 d = wrapd<W>(x - ld3(xs[j]), p);
-      if (length_sqr(d) < p.h2) f(j, d);
+          c3[a] = c3[a] >= p.res[a] ? c3[a] - p.res[a] : (c3[a] < 0 ? c3[a] + p.res[a] : c3[a]);
+      if (!within_grid(c3, p)) continue;
+      const unsigned c = p.cell_base + cell_linear(c3, p);
+      scan(cell_start[c], cell_start[c + 1]);
     }
   }
+  return cnt;
 }
-__device__ inline void list_put(uint4* list, const DevArrays& A, unsigned s, unsigned t,
-                                unsigned v) {
-  reinterpret_cast<unsigned*>(list + nbr_group(A, t >> 2, s))[t & 3u] = v;
+// Entry 4 k + q of a list for the quad's round k (a lane past the end gets
+// the last entry, which the caller drops).
+__device__ inline unsigned quad_entry(const uint4* list, const DevArrays& A, unsigned s, unsigned t,
+                                      unsigned n) {
+  return pellet_at(list, A, s, min(t, n - 1u));
 }
 
 // transform_pellets (runner.hpp:4071-4085) with the step-start kinematics:
@@ -2890,44 +2940,52 @@ __global__ __launch_bounds__(256) void k_pellet_gather(SceneTab T, DevArrays A) 
 // runner.hpp:1913-1971; the fluid lists are k_neighbors') and the density
 // with pellets (compute_density_with_pellets, runner.hpp:2074-2098):
 // rho = m (W(0) + sum_fluid W + sum_pellets W), both sums over the lists.
+// Bound by the latency of the cells' and entries' loads: four lanes per
+// particle with 16 entries in flight (13 us for 16,384 fluid particles; one
+// lane, an entry at a time, took 43).  The density's terms are evaluated four
+// at a time and added in list order.
+constexpr unsigned kQuadInFlight = 4;  // entries per lane whose loads are in flight together
 template <bool W>
-__global__ __launch_bounds__(256) void k_pellet_fluid_lists(SceneTab T, DevArrays A) {
-  ALV_SCENE(T, A, s);
-  if (s >= p.first + p.n) return;
-  const unsigned K = p.kmax;
+__global__ __launch_bounds__(64) void k_pellet_fluid_lists(SceneTab T, DevArrays A) {
+  ALV_SCENE_QUAD(T, A, s, q, xcd_block());
+  if (s >= p.first + p.n) return;  // whole quads
   const vec3 xi = ld3(A.x[s]);
-  unsigned cnt = 0;
-  scan_cells<W>(p, A.pcell_start, A.px, xi, [&](unsigned j, vec3) {
-    list_put(A.pnbr, A, s, min(cnt, K - 1), j);
-    ++cnt;
-  });
-  const unsigned npn = min(cnt, K);
-  A.pnnb[s] = npn;
-  if (cnt > K) A.anomaly[2] = 1u;
+  const unsigned cnt = list_cells<W>(p, A, A.pcell_start, A.px, xi, A.pnbr, s, q);
+  const unsigned npn = min(cnt, p.kmax);
+  if (q == 0u) A.pnnb[s] = npn;
+  if (cnt > p.kmax) A.anomaly[2] = 1u;
+  __threadfence_block();  // the lanes' list writes
   float dens = p.w0;
-  const unsigned nn = A.nnb[s];
-  for (unsigned t = 0; t < nn; ++t)
-    dens += W_pair(length_sqr(wrapd<W>(xi - ld3(A.x[pellet_at(A.nbr, A, s, t)]), p)), p);
-  for (unsigned t = 0; t < npn; ++t)
-    dens += W_pair(length_sqr(wrapd<W>(xi - ld3(A.px[pellet_at(A.pnbr, A, s, t)]), p)), p);
+  auto add = [&](const uint4* list, unsigned n, const float4* xs) {
+    for (unsigned t0 = 0; t0 < n; t0 += 4u * kQuadInFlight) {
+      float4 xj[kQuadInFlight];
+#pragma unroll
+      for (unsigned k = 0; k < kQuadInFlight; ++k)
+        xj[k] = xs[quad_entry(list, A, s, t0 + 4u * k + q, n)];
+#pragma unroll
+      for (unsigned k = 0; k < kQuadInFlight; ++k) {
+        const float w = W_pair(length_sqr(wrapd<W>(xi - ld3(xj[k]), p)), p);
+        dens = quad_add(dens, t0 + 4u * k + q < n ? w : 0.0f);
+      }
+    }
+  };
+  add(A.nbr, A.nnb[s], A.x);
+  add(A.pnbr, npn, A.px);
+  if (q != 0u) return;
   const float rho = dens * p.mass;
   A.density[s] = rho;
   reinterpret_cast<float*>(A.v + s)[3] = visc_coefficient(p, rho);
 }
 // The fluid lists of the pellets (the bead lists of the same search), which
-// the MLS extrapolation reads.  One thread per pellet.
+// the MLS extrapolation reads.  Four lanes per pellet as above (9 us for
+// 21,385 pellets; 25 with one lane).
 template <bool W>
-__global__ __launch_bounds__(256) void k_pellet_bead_lists(SceneTab T, DevArrays A) {
-  ALV_SCENE_LINEAR(T, A, s);
-  if (s >= p.n) return;
-  const unsigned K = p.kmax;
-  unsigned cnt = 0;
-  scan_cells<W>(p, A.cell_start, A.x, ld3(A.px[s]), [&](unsigned j, vec3) {
-    list_put(A.pbnbr, A, s, min(cnt, K - 1), j);
-    ++cnt;
-  });
-  A.pbnnb[s] = min(cnt, K);
-  if (cnt > K) A.anomaly[2] = 1u;
+__global__ __launch_bounds__(64) void k_pellet_bead_lists(SceneTab T, DevArrays A) {
+  ALV_SCENE_QUAD(T, A, s, q, blockIdx.x);
+  if (s >= p.n) return;  // whole quads
+  const unsigned cnt = list_cells<W>(p, A, A.cell_start, A.x, ld3(A.px[s]), A.pbnbr, s, q);
+  if (q == 0u) A.pbnnb[s] = min(cnt, p.kmax);
+  if (cnt > p.kmax) A.anomaly[2] = 1u;
 }
 // compute_viscosity_with_pellets (runner.hpp:2251-2297) with
 // clear_acceleration and the per-block CFL maxima, as k_viscosity
@@ -3019,10 +3077,13 @@ __device__ inline void sym_pinv(vec3 d, vec3 o, float inv[3][3]) {
 // a pellet without fluid neighbours gets 0).  Inside the Jacobi loop it
 // reads the buffer the next iteration reads; final_pressure reads the
 // solved pressure and also stores the pellets' pressure in user order.
+// Four lanes per pellet, terms added in list order (8 us for 21,385 pellets,
+// bound by the latency of one pellet's list and plane fit; 13 with one lane).
 template <bool W>
-__global__ __launch_bounds__(256) void k_extrapolate(SceneTab T, DevArrays A, int final_pressure) {
-  ALV_SCENE_LINEAR(T, A, s);
-  if (s >= p.n) return;
+__global__ __launch_bounds__(64) void k_extrapolate(SceneTab T, DevArrays A, int final_pressure) {
+  ALV_SCENE_QUAD(T, A, s, q, blockIdx.x);
+  A.ctl += T.blk_scene[blk_ / (kBlock / 16u)];
+  if (s >= p.n) return;  // whole quads
   if (!final_pressure && A.ctl->dens_done) return;
   if (must_wait(A)) return;
   const float* src = (final_pressure || (A.ctl->dens_iter & 1u) != 0u) ? A.pressure
@@ -3031,25 +3092,43 @@ __global__ __launch_bounds__(256) void k_extrapolate(SceneTab T, DevArrays A, in
   const unsigned nn = A.pbnnb[s];
   float w_sum = 0.f;
   vec3 center = mk(0.f, 0.f, 0.f);
-  for (unsigned t = 0; t < nn; ++t) {
-    const vec3 xj = ld3(A.x[pellet_at(A.pbnbr, A, s, t)]);
-    const float w = W_pair(length_sqr(wrapd<W>(xi - xj, p)), p) * p.vol;
-    w_sum += w;
-    center += w * xj;
+  for (unsigned t0 = 0; t0 < nn; t0 += 4u * kQuadInFlight) {
+    float4 x4[kQuadInFlight];
+#pragma unroll
+    for (unsigned k = 0; k < kQuadInFlight; ++k)
+      x4[k] = A.x[quad_entry(A.pbnbr, A, s, t0 + 4u * k + q, nn)];
+#pragma unroll
+    for (unsigned k = 0; k < kQuadInFlight; ++k) {
+      const bool ok = t0 + 4u * k + q < nn;
+      const vec3 xj = ld3(x4[k]);
+      const float w = W_pair(length_sqr(wrapd<W>(xi - xj, p)), p) * p.vol;
+      w_sum = quad_add(w_sum, ok ? w : 0.f);
+      center = quad_add3(center, w * xj, ok);
+    }
   }
   center = mk(center.x / w_sum, center.y / w_sum, center.z / w_sum);
   float alpha = 0.f;
   vec3 dg = mk(0.f, 0.f, 0.f), od = mk(0.f, 0.f, 0.f), pxs = mk(0.f, 0.f, 0.f);
-  for (unsigned t = 0; t < nn; ++t) {
-    const unsigned j = pellet_at(A.pbnbr, A, s, t);
-    const vec3 xj = ld3(A.x[j]);
-    const vec3 xt = xj - center;
-    const float w = W_pair(length_sqr(wrapd<W>(xi - xj, p)), p) * p.vol;
-    const float wp = w * src[j];
-    alpha += wp;
-    pxs += wp * xt;
-    dg += w * mk(xt.x * xt.x, xt.y * xt.y, xt.z * xt.z);
-    od += w * mk(xt.x * xt.y, xt.x * xt.z, xt.y * xt.z);
+  for (unsigned t0 = 0; t0 < nn; t0 += 4u * kQuadInFlight) {
+    float4 x4[kQuadInFlight];
+    float pj[kQuadInFlight];
+#pragma unroll
+    for (unsigned k = 0; k < kQuadInFlight; ++k) {
+      const unsigned j = quad_entry(A.pbnbr, A, s, t0 + 4u * k + q, nn);
+      x4[k] = A.x[j];
+      pj[k] = src[j];
+    }
+#pragma unroll
+    for (unsigned k = 0; k < kQuadInFlight; ++k) {
+      const bool ok = t0 + 4u * k + q < nn;
+      const vec3 xj = ld3(x4[k]), xt = xj - center;
+      const float w = W_pair(length_sqr(wrapd<W>(xi - xj, p)), p) * p.vol;
+      const float wp = w * pj[k];
+      alpha = quad_add(alpha, ok ? wp : 0.f);
+      pxs = quad_add3(pxs, wp * xt, ok);
+      dg = quad_add3(dg, w * mk(xt.x * xt.x, xt.y * xt.y, xt.z * xt.z), ok);
+      od = quad_add3(od, w * mk(xt.x * xt.y, xt.x * xt.z, xt.y * xt.z), ok);
+    }
   }
   alpha /= w_sum;
   float inv[3][3];
@@ -3058,6 +3137,7 @@ __global__ __launch_bounds__(256) void k_extrapolate(SceneTab T, DevArrays A, in
                         inv[1][0] * pxs.x + inv[1][1] * pxs.y + inv[1][2] * pxs.z,
                         inv[2][0] * pxs.x + inv[2][1] * pxs.y + inv[2][2] * pxs.z);
   const float pr = fmaxf(alpha + dot(plane, xi - center), 0.f);
+  if (q != 0u) return;
   A.pp[s] = pr;
   if (final_pressure) A.upressure[A.cap + A.psorted_id[s]] = pr;
 }
@@ -3145,6 +3225,17 @@ KernelProfiler* g_profiler = nullptr;
       hipLaunchKernelGGL(kernel<true>, dim3((L).pblocks), dim3(kBlock), 0, s, (L).T, __VA_ARGS__); \
     else                                                                          \
       hipLaunchKernelGGL(kernel<false>, dim3((L).pblocks), dim3(kBlock), 0, s, (L).T, __VA_ARGS__); \
+    if (g_profiler) g_profiler->end(#kernel, s);                                  \
+  } while (0)
+// four lanes per particle, blocks of 16
+#define ALV_LAUNCH_QUAD(kernel, L, s, ...)                                        \
+  do {                                                                            \
+    if (g_profiler) g_profiler->begin(#kernel, s);                                \
+    const dim3 grid_((L).pblocks * (kBlock / 16u));                               \
+    if ((L).p0.wrap_mask)                                                         \
+      hipLaunchKernelGGL(kernel<true>, grid_, dim3(64), 0, s, (L).T, __VA_ARGS__); \
+    else                                                                          \
+      hipLaunchKernelGGL(kernel<false>, grid_, dim3(64), 0, s, (L).T, __VA_ARGS__); \
     if (g_profiler) g_profiler->end(#kernel, s);                                  \
   } while (0)
 // one block per scene
@@ -3426,8 +3517,8 @@ void launch_pellet_grid(const Launch& Lp, const DevArrays& A, hipStream_t s) {
   }
 }
 void launch_pellet_lists(const Launch& L, const Launch& Lp, const DevArrays& A, hipStream_t s) {
-  if (L.active) ALV_LAUNCH_W(k_pellet_fluid_lists, L, s, A);
-  if (Lp.active) ALV_LAUNCH_W(k_pellet_bead_lists, Lp, s, A);
+  if (L.active) ALV_LAUNCH_QUAD(k_pellet_fluid_lists, L, s, A);
+  if (Lp.active) ALV_LAUNCH_QUAD(k_pellet_bead_lists, Lp, s, A);
 }
 void launch_pellet_viscosity(const Launch& L, const DevArrays& A, hipStream_t s) {
   ALV_LAUNCH_W(k_viscosity_pellets, L, s, A);
@@ -3438,13 +3529,13 @@ void launch_is_prepare_pellets(const Launch& L, const DevArrays& A, hipStream_t 
 }
 void launch_is_iteration_pellets(const Launch& L, const Launch& Lp, const DevArrays& A,
                                  hipStream_t s) {
-  if (Lp.active) ALV_LAUNCH_W(k_extrapolate, Lp, s, A, 0);
+  if (Lp.active) ALV_LAUNCH_QUAD(k_extrapolate, Lp, s, A, 0);
   ALV_LAUNCH_W2(k_is_iter, true, L, s, A);
   ALV_LAUNCH_FIN(k_ii_finalize, L, s, A);
 }
 void launch_is_finish_pellets(const Launch& L, const Launch& Lp, const DevArrays& A,
                               hipStream_t s) {
-  if (Lp.active) ALV_LAUNCH_W(k_extrapolate, Lp, s, A, 1);
+  if (Lp.active) ALV_LAUNCH_QUAD(k_extrapolate, Lp, s, A, 1);
   ALV_LAUNCH_W2(k_ii_pressure_accel, true, L, s, A);
   ALV_LAUNCH_W(k_ii_finish, L, s, A);
 }

@@ -58,6 +58,51 @@ def test_pellet_lists_and_density_match_oracle():
     assert np.all(dp.coat(solver.grid_anomaly).get() == 0)
 
 
+@pytest.mark.parametrize("n,npel", [(1, 17), (15, 1), (17, 63), (300, 257)])
+@pytest.mark.parametrize("kmax,wrap", [(7, None), (64, None), (40, (True, False, True)),
+                                       (64, (True, True, False)), (64, (True, True, True))])
+def test_list_edges_match_oracle(n, npel, kmax, wrap):
+    """Counts around a wave's 16 particles, list caps below and above the
+    lengths, and periodic axes with and without the cells' third one."""
+    from alluvion_amd import scenes
+    rng = np.random.default_rng(n + kmax)
+    cells = (3, 3, 4)
+    length = np.array(cells) * 0.01
+
+    def points(k):
+        return ((rng.random((k, 3)) - 0.5) * length * 0.999999).astype(np.float32)
+
+    body = scenes.BoundarySpec("sphere", (0.01,), 1.0, (4, 4, 4),
+                               collision_vertices=points(npel).astype(np.float64))
+    x = points(n)
+    sc = scenes.Scene(
+        name="pellet_cloud", x=x, v=np.zeros_like(x), boundaries=[body], volume_method="pellets",
+        wrap_length=tuple(float(length[a]) if wrap and wrap[a] else 0.0 for a in range(3)),
+        grid_offset=(-2, -2, -2), grid_res=(4, 4, 4) if wrap is None else cells,
+        max_num_neighbors=kmax, max_num_pellets=npel + 5, max_num_particles_per_cell=512)
+    if wrap is not None:  # the grid's cells fill the box
+        sc.wrap_length = tuple(w and 0.01 * sc.grid_res[a] for a, w in enumerate(sc.wrap_length))
+    dp, pile, solver, _, _ = scenes.build_solver(sc, kind="i")
+    solver.transform_all_pellets()
+    solver.update_particle_neighbors()
+    orc = of.Oracle(sc, precision=4, kind="i")
+    orc.transform_pellets()
+    orc.update_particle_neighbors()
+    mx = orc.max_n
+    for got, want_pellets, rows in ((solver.get_neighbors(), False, slice(0, n)),
+                                    (solver.get_pellet_neighbors(0, mx), True, slice(0, n)),
+                                    (solver.get_pellet_neighbors(1, sc.max_num_pellets), False,
+                                     slice(mx, mx + npel))):
+        oids, ocnt = pellet_lists_orc(orc, want_pellets, rows)
+        ids, cnt = got[0][:len(ocnt)], got[1][:len(ocnt)]
+        np.testing.assert_array_equal(cnt, ocnt)
+        mask = np.arange(ids.shape[1])[None, :] < ocnt[:, None]
+        np.testing.assert_array_equal(np.where(mask, ids, 0),
+                                      np.where(mask, oids[:, :ids.shape[1]], 0))
+    dens = dp.coat(solver.particle_density).get()[:n]
+    assert rel(dens, orc.get("density")[:n]) < 1e-6
+
+
 def body_state(pile, b):
     q = pile.get_q(b)
     return (np.array(list(pile.get_x(b))), np.array(list(pile.get_v(b))),
