@@ -2349,7 +2349,7 @@ int alv_solver_step(alv_solver* S) {
       // with the divergence solve, its density-change passes computed the
       // viscosity
       if (L.active && !div) launch_df_viscosity(L, Aw, st);
-      launch_update_dt(L, Aw, div, st);
+      launch_update_dt(L, Aw, st);
       if (L.active) {
         launch_df_integrate_np(L, Aw, div, st);
         if (dens) {
@@ -2416,7 +2416,7 @@ int alv_solver_step(alv_solver* S) {
     if (rc != ALV_OK) return rc;
     launch_pellet_lists(L, Lp, A, st);
     if (L.active) launch_pellet_viscosity(L, A, st);
-    launch_update_dt(L, A, 0, st);
+    launch_update_dt(L, A, st);
     if (L.active) {
       launch_is_prepare_pellets(L, A, st);
       rc = run_loop(S, S->set.max_density_solve, &S->last_dens,
@@ -2433,7 +2433,7 @@ int alv_solver_step(alv_solver* S) {
     rc = neighbor_phase(S, L, 0);
     if (rc != ALV_OK) return rc;
     if (L.active) launch_ii_viscosity_predict(L, A, st);
-    launch_update_dt(L, A, 0, st);
+    launch_update_dt(L, A, st);
     if (L.active) {
       launch_is_prepare(L, A, st);
       rc = run_loop(S, S->set.max_density_solve, &S->last_dens,
@@ -2450,7 +2450,7 @@ int alv_solver_step(alv_solver* S) {
     rc = neighbor_phase(S, L, 0);
     if (rc != ALV_OK) return rc;
     if (L.active) launch_ii_viscosity_predict(L, A, st);
-    launch_update_dt(L, A, 0, st);
+    launch_update_dt(L, A, st);
     if (L.active) {
       launch_ii_predict(L, A, st);
       rc = run_loop(S, S->set.max_density_solve, &S->last_dens,

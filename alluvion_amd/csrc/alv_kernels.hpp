@@ -256,9 +256,7 @@ void launch_df_div_iteration(const Launch& L, const DevArrays& A, hipStream_t s)
 // the viscosity of a step without a divergence solve (with one, that solve's
 // density-change passes compute it)
 void launch_df_viscosity(const Launch& L, const DevArrays& A, hipStream_t s);
-// pass_parts: the maxima come from a density-change pass (in its form's
-// blocks), else from k_viscosity
-void launch_update_dt(const Launch& L, const DevArrays& A, int pass_parts, hipStream_t s);
+void launch_update_dt(const Launch& L, const DevArrays& A, hipStream_t s);
 // fin: the divergence solve ran (and computed the viscosity): also finish it
 // and add the bodies' viscous reactions
 void launch_df_integrate_np(const Launch& L, const DevArrays& A, int fin, hipStream_t s);

@@ -1535,6 +1535,89 @@ __device__ inline vec3 stiffness_boundary(const SimParams& p, const DevArrays& A
   return dv;
 }
 
+// acc[c] += the c-th component of term(load(j)) over a list of nn entries, in
+// list order.  One lane per particle takes four entries at a time; in the deep
+// form (D, see velocity_divergence_deep) lane q of four takes entries 4 k + q,
+// NS of them in flight, and every lane of the particle ends with the sums.
+// `self` is an index that may be loaded from in place of an entry past the
+// count, whose term is dropped.  Up to kDeepMaxBlocks a pass is bound by these
+// latencies: 16,384 particles with pellets 16 -> 7 us (k_is_iter), 16 -> 8
+// (k_is_diag, k_ii_pressure_accel), whole steps 344 -> 300; IISPH steps of 4,096
+// particles 193 -> 111 us and of 95,220 240 -> 208 (the search's share
+// included), of 101,568 on the one-lane side 242 -> 225.
+template <bool D, unsigned NS, unsigned N, class Load, class Term>
+__device__ inline void list_sum(const uint4* list, const DevArrays& A, unsigned s, unsigned q,
+                                unsigned nn, unsigned self, float (&acc)[N], Load load,
+                                Term term) {
+  if constexpr (D) {
+    const unsigned* row = reinterpret_cast<const unsigned*>(list + nbr_group(A, 0u, s)) + q;
+    const unsigned last = nbr_groups(A.kmax) - 1u;
+    for (unsigned t0 = 0; t0 < nn; t0 += 4u * NS) {
+      unsigned j[NS];
+#pragma unroll
+      for (unsigned k = 0; k < NS; ++k) j[k] = row[min((t0 >> 2) + k, last) * 256u];
+#pragma unroll
+      for (unsigned k = 0; k < NS; ++k) asm volatile("" : "+v"(j[k]));
+      decltype(load(0u)) d[NS];
+#pragma unroll
+      for (unsigned k = 0; k < NS; ++k) d[k] = load(t0 + 4u * k + q < nn ? j[k] : self);
+#pragma unroll
+      for (unsigned k = 0; k < NS; ++k) {
+        float t[N];
+        term(d[k], t);
+        const bool ok = t0 + 4u * k + q < nn;
+#pragma unroll
+        for (unsigned c = 0; c < N; ++c)
+          acc[c] = add_in_slot_order<4>(acc[c], ok ? t[c] : 0.0f);
+      }
+    }
+  } else {
+    for (unsigned t0 = 0; t0 < nn; t0 += kNB) {
+      uint4 g = list[nbr_group(A, t0 >> 2, s)];
+      asm volatile("" : "+v"(g.x), "+v"(g.y), "+v"(g.z), "+v"(g.w));  // see batch_ids
+      const unsigned j[kNB] = {g.x, t0 + 1 < nn ? g.y : self, t0 + 2 < nn ? g.z : self,
+                               t0 + 3 < nn ? g.w : self};
+      decltype(load(0u)) d[kNB];
+#pragma unroll
+      for (int u = 0; u < kNB; ++u) d[u] = load(j[u]);
+#pragma unroll
+      for (int u = 0; u < kNB; ++u) {
+        if (t0 + u < nn) {
+          float t[N];
+          term(d[u], t);
+#pragma unroll
+          for (unsigned c = 0; c < N; ++c) acc[c] += t[c];
+        }
+      }
+    }
+  }
+}
+// entries in flight per lane: most lists whole, or half of one where an entry
+// is three or four vectors
+constexpr unsigned kListDeep = 9, kListDeepWide = 5;
+struct EntryX {
+  vec3 x;
+};
+struct EntryXV {
+  vec3 x, v;
+};
+struct EntryXVS {
+  vec3 x, v;
+  float a;
+};
+struct EntryXS {
+  vec3 x;
+  float a;
+};
+struct EntryXSS {
+  vec3 x;
+  float a, b;
+};
+struct EntryIter1 {
+  vec3 x, dij_pj, dii;
+  float lp;
+};
+
 // sum_j mu m / rho_j (x_ij . gradW_ij) / (|x_ij|^2 + 0.01 h^2) (v_i - v_j)
 template <bool W, class Src>
 __device__ inline vec3 viscosity_sum(const SimParams& p, const DevArrays& A, unsigned s,
@@ -1940,27 +2023,33 @@ __device__ inline void reset_ctl(const DevArrays& A, unsigned scene) {
 // k_integrate_np; k_viscosity serves the step without a divergence solve and
 // IISPH.
 // ---------------------------------------------------------------------------
-template <bool W, bool TL>
+template <bool W, int M>
 __global__ __launch_bounds__(256) void k_viscosity(SceneTab T, DevArrays A) {
   __shared__ float lds[4];
-  ALV_SCENE(T, A, s);
+  ALV_SCENE_PASS(T, A, s, q, M, stiffness_lanes(M));
   TileXV tile_;
   bool tiled_ = false;
-  if constexpr (TL) tiled_ = stage_xv(A, s / kBlock, tile_);
+  if constexpr (M == kTile) tiled_ = stage_xv(A, s / kBlock, tile_);
   const float dt = A.ctl->dt;
   float cfl = -FLT_MAX;
   if (s < p.first + p.n) {
     const vec3 xi = ld3(A.x[s]), vi = ld3(A.v[s]);
     const unsigned nn = A.nnb[s];
-    vec3 da = tiled_ ? viscosity_sum<W>(p, A, s, xi, vi, nn, tile_)
-                     : viscosity_sum<W>(p, A, s, xi, vi, nn, GlobalXV{A.x, A.v});
-    da = boundary_viscosity<true>(p, A, s, xi, vi, da);
-    vec3 a = mk(p.g[0], p.g[1], p.g[2]) + da;
-    A.a[s] = f4(a, 0.f);
-    cfl = length_sqr(vi + a * dt);
+    vec3 da;
+    if constexpr (M == kDeep)
+      velocity_divergence_deep<W, true>(p, A, s, q, xi, vi, nn, &da);
+    else
+      da = tiled_ ? viscosity_sum<W>(p, A, s, xi, vi, nn, tile_)
+                  : viscosity_sum<W>(p, A, s, xi, vi, nn, GlobalXV{A.x, A.v});
+    if (q == 0u) {
+      da = boundary_viscosity<true>(p, A, s, xi, vi, da);
+      vec3 a = mk(p.g[0], p.g[1], p.g[2]) + da;
+      A.a[s] = f4(a, 0.f);
+      cfl = length_sqr(vi + a * dt);
+    }
   }
   float m = block_max_f(cfl, lds);
-  if (threadIdx.x == 0) A.fpartials[xcd_block()] = m;
+  if (threadIdx.x == 0) A.fpartials[qblk_] = m;
 }
 
 // Solver::update_dt (solver.hpp:153-169) on the device.
@@ -2199,32 +2288,29 @@ __global__ __launch_bounds__(256) void k_integrate_velocity(SceneTab T, DevArray
 // IISPH (runner.hpp:2609-2887)
 // ---------------------------------------------------------------------------
 // predict_advection0 (runner.hpp:2609-2639)
-template <bool W>
+template <bool W, bool D>
 __global__ __launch_bounds__(256) void k_ii_predict0(SceneTab T, DevArrays A) {
-  ALV_SCENE(T, A, s);
+  ALV_SCENE_PASS(T, A, s, q, D ? kDeep : kGather, D ? kDeepLanes : 1u);
   if (s >= p.first + p.n) return;
   const float dt = A.ctl->dt;
-  add_v(A, s, dt * ld3(A.a[s]));
-  A.last_pressure[s] = A.pressure[s] * 0.5f;
+  if (q == 0u) {
+    add_v(A, s, dt * ld3(A.a[s]));
+    A.last_pressure[s] = A.pressure[s] * 0.5f;
+  }
   const vec3 xi = ld3(A.x[s]);
   const float dens = A.density[s];
   const float dens2 = dens * dens;
-  vec3 d = mk(0.f, 0.f, 0.f);
-  const unsigned nn = A.nnb[s];
-  for (unsigned t0 = 0; t0 < nn; t0 += kNB) {
-    unsigned j[kNB];
-    batch_ids(A, s, nn, t0, j);
-    float4 xj[kNB];
-#pragma unroll
-    for (int u = 0; u < kNB; ++u) xj[u] = A.x[j[u]];
-#pragma unroll
-    for (int u = 0; u < kNB; ++u) {
-      if (t0 + u < nn) {
-        vec3 xixj = wrapd<W>(xi - ld3(xj[u]), p);
-        d -= (p.vol / dens2) * grad_pair(xixj, p);
-      }
-    }
-  }
+  float sum[3] = {0.f, 0.f, 0.f};
+  list_sum<D, kListDeep>(
+      A.nbr, A, s, q, A.nnb[s], s, sum, [&](unsigned j) { return EntryX{ld3(A.x[j])}; },
+      [&](const EntryX& e, float (&t)[3]) {
+        const vec3 g = (p.vol / dens2) * grad_pair(wrapd<W>(xi - e.x, p), p);
+        t[0] = -g.x;
+        t[1] = -g.y;
+        t[2] = -g.z;
+      });
+  if (q != 0u) return;
+  vec3 d = mk(sum[0], sum[1], sum[2]);
   unsigned mask = A.bmask[s];
   while (mask) {
     const unsigned b = __builtin_ctz(mask);
@@ -2235,9 +2321,9 @@ __global__ __launch_bounds__(256) void k_ii_predict0(SceneTab T, DevArrays A) {
   A.dii[s] = f4(d * p.rho0, 0.f);
 }
 // predict_advection1 (runner.hpp:2640-2690)
-template <bool W>
+template <bool W, bool D>
 __global__ __launch_bounds__(256) void k_ii_predict1(SceneTab T, DevArrays A) {
-  ALV_SCENE(T, A, s);
+  ALV_SCENE_PASS(T, A, s, q, D ? kDeep : kGather, D ? kDeepLanes : 1u);
   if (s >= p.first + p.n) return;
   const float dt = A.ctl->dt;
   const vec3 xi = ld3(A.x[s]), vi = ld3(A.v[s]), d_ii = ld3(A.dii[s]);
@@ -2245,29 +2331,18 @@ __global__ __launch_bounds__(256) void k_ii_predict1(SceneTab T, DevArrays A) {
   const float dens2 = dens * dens;
   const float inv_dens2 = 1.0f / dens2;
   const float dpi = p.vol * inv_dens2;
-  float dadv = dens / p.rho0;
-  float a_ii = 0.f;
-  const unsigned nn = A.nnb[s];
-  for (unsigned t0 = 0; t0 < nn; t0 += kNB) {
-    unsigned j[kNB];
-    batch_ids(A, s, nn, t0, j);
-    float4 xj[kNB], vj[kNB];
-#pragma unroll
-    for (int u = 0; u < kNB; ++u) {
-      xj[u] = A.x[j[u]];
-      vj[u] = A.v[j[u]];
-    }
-#pragma unroll
-    for (int u = 0; u < kNB; ++u) {
-      if (t0 + u < nn) {
-        vec3 xixj = wrapd<W>(xi - ld3(xj[u]), p);
-        vec3 gw = grad_pair(xixj, p);
-        vec3 dji = (dpi * p.rho0) * gw;
-        dadv += dt * p.vol * dot(vi - ld3(vj[u]), gw);
-        a_ii += p.vol * dot(d_ii - dji, gw);
-      }
-    }
-  }
+  float sum[2] = {dens / p.rho0, 0.f};
+  list_sum<D, kListDeep>(
+      A.nbr, A, s, q, A.nnb[s], s, sum,
+      [&](unsigned j) { return EntryXV{ld3(A.x[j]), ld3(A.v[j])}; },
+      [&](const EntryXV& e, float (&t)[2]) {
+        const vec3 gw = grad_pair(wrapd<W>(xi - e.x, p), p);
+        const vec3 dji = (dpi * p.rho0) * gw;
+        t[0] = dt * p.vol * dot(vi - e.v, gw);
+        t[1] = p.vol * dot(d_ii - dji, gw);
+      });
+  if (q != 0u) return;
+  float dadv = sum[0], a_ii = sum[1];
   unsigned mask = A.bmask[s];
   while (mask) {
     const unsigned b = __builtin_ctz(mask);
@@ -2287,44 +2362,33 @@ __global__ __launch_bounds__(256) void k_ii_predict1(SceneTab T, DevArrays A) {
 // iteration's copy last_pressure <- pressure (solver_ii.hpp:204) is folded in:
 // from the second iteration on, neighbour values are read from `pressure`
 // and each particle refreshes its own last_pressure.
-template <bool W>
+template <bool W, bool D>
 __global__ __launch_bounds__(256) void k_ii_iter0(SceneTab T, DevArrays A) {
-  ALV_SCENE(T, A, s);
+  ALV_SCENE_PASS(T, A, s, q, D ? kDeep : kGather, D ? kDeepLanes : 1u);
   if (A.ctl->dens_done) return;
   if (s >= p.first + p.n) return;
   const float* lp = (A.ctl->dens_iter == 0u) ? A.last_pressure : A.pressure;
   const vec3 xi = ld3(A.x[s]);
-  vec3 acc = mk(0.f, 0.f, 0.f);
-  const unsigned nn = A.nnb[s];
-  for (unsigned t0 = 0; t0 < nn; t0 += kNB) {
-    unsigned j[kNB];
-    batch_ids(A, s, nn, t0, j);
-    float4 xj[kNB];
-    float djs[kNB], lpj[kNB];
-#pragma unroll
-    for (int u = 0; u < kNB; ++u) {
-      xj[u] = A.x[j[u]];
-      djs[u] = A.density[j[u]];
-      lpj[u] = lp[j[u]];
-    }
-#pragma unroll
-    for (int u = 0; u < kNB; ++u) {
-      if (t0 + u < nn) {
-        vec3 xixj = wrapd<W>(xi - ld3(xj[u]), p);
-        float dj = djs[u];
-        float dj2 = dj * dj;
-        acc -= (p.vol / dj2 * lpj[u]) * grad_pair(xixj, p);
-      }
-    }
-  }
-  A.dij_pj[s] = f4(acc * p.rho0, 0.f);
+  float sum[3] = {0.f, 0.f, 0.f};
+  list_sum<D, kListDeep>(
+      A.nbr, A, s, q, A.nnb[s], s, sum,
+      [&](unsigned j) { return EntryXSS{ld3(A.x[j]), A.density[j], lp[j]}; },
+      [&](const EntryXSS& e, float (&t)[3]) {
+        const float dj2 = e.a * e.a;
+        const vec3 g = (p.vol / dj2 * e.b) * grad_pair(wrapd<W>(xi - e.x, p), p);
+        t[0] = -g.x;
+        t[1] = -g.y;
+        t[2] = -g.z;
+      });
+  if (q != 0u) return;
+  A.dij_pj[s] = f4(mk(sum[0], sum[1], sum[2]) * p.rho0, 0.f);
   A.last_pressure[s] = lp[s];
 }
 // pressure_solve_iteration1 (runner.hpp:2716-2772) + FP64 partial sums
-template <bool W>
+template <bool W, bool D>
 __global__ __launch_bounds__(256) void k_ii_iter1(SceneTab T, DevArrays A) {
   __shared__ double lds[4];
-  ALV_SCENE(T, A, s);
+  ALV_SCENE_PASS(T, A, s, q, D ? kDeep : kGather, D ? kDeepLanes : 1u);
   if (A.ctl->dens_done) return;
   const float dt = A.ctl->dt;
   double part = 0.0;
@@ -2341,57 +2405,47 @@ __global__ __launch_bounds__(256) void k_ii_iter1(SceneTab T, DevArrays A) {
     const float denom = a_ii * dt2;
     const float w = 2.0f / 3.0f;
     float pr = 0.f;
-    float sum_tmp = 0.f;
-    const unsigned nn = A.nnb[s];
-    for (unsigned t0 = 0; t0 < nn; t0 += kNB) {
-      unsigned j[kNB];
-      batch_ids(A, s, nn, t0, j);
-      float4 xj[kNB], dpk[kNB], diij[kNB];
-      float lpj[kNB];
-#pragma unroll
-      for (int u = 0; u < kNB; ++u) {
-        xj[u] = A.x[j[u]];
-        dpk[u] = A.dij_pj[j[u]];
-        diij[u] = A.dii[j[u]];
-        lpj[u] = A.last_pressure[j[u]];
+    float sum[1] = {0.f};
+    list_sum<D, kListDeepWide>(
+        A.nbr, A, s, q, A.nnb[s], s, sum,
+        [&](unsigned j) {
+          return EntryIter1{ld3(A.x[j]), ld3(A.dij_pj[j]), ld3(A.dii[j]), A.last_pressure[j]};
+        },
+        [&](const EntryIter1& e, float (&t)[1]) {
+          const vec3 gw = grad_pair(wrapd<W>(xi - e.x, p), p);
+          const vec3 dji = (dpi * p.rho0) * gw;
+          const vec3 dji_pi = dji * lp;
+          t[0] = p.vol * dot(dpj - e.dii * e.lp - (e.dij_pj - dji_pi), gw);
+        });
+    if (q == 0u) {
+      float sum_tmp = sum[0];
+      unsigned mask = A.bmask[s];
+      while (mask) {
+        const unsigned b = __builtin_ctz(mask);
+        mask &= mask - 1u;
+        float4 k = A.bker[size_t(b) * A.cap + s];
+        sum_tmp += dot(dpj, mk(k.x, k.y, k.z));
       }
-#pragma unroll
-      for (int u = 0; u < kNB; ++u) {
-        if (t0 + u < nn) {
-          vec3 xixj = wrapd<W>(xi - ld3(xj[u]), p);
-          vec3 djk_pk = ld3(dpk[u]);
-          vec3 gw = grad_pair(xixj, p);
-          vec3 dji = (dpi * p.rho0) * gw;
-          vec3 dji_pi = dji * lp;
-          sum_tmp += p.vol * dot(dpj - ld3(diij[u]) * lpj[u] - (djk_pk - dji_pi), gw);
-        }
-      }
+      sum_tmp *= p.rho0;
+      if (fabsf(denom) > 1.0e-9f)
+        pr = std_max((1.0f - w) * lp + w / denom * (bb - dt2 * sum_tmp), 0.0f);
+      float err = pr == 0.f ? 0.f : (denom * pr + sum_tmp * dt2 - bb);
+      A.density_err[s] = err;
+      A.pressure[s] = pr;
+      part = double(err);
     }
-    unsigned mask = A.bmask[s];
-    while (mask) {
-      const unsigned b = __builtin_ctz(mask);
-      mask &= mask - 1u;
-      float4 k = A.bker[size_t(b) * A.cap + s];
-      sum_tmp += dot(dpj, mk(k.x, k.y, k.z));
-    }
-    sum_tmp *= p.rho0;
-    if (fabsf(denom) > 1.0e-9f)
-      pr = std_max((1.0f - w) * lp + w / denom * (bb - dt2 * sum_tmp), 0.0f);
-    float err = pr == 0.f ? 0.f : (denom * pr + sum_tmp * dt2 - bb);
-    A.density_err[s] = err;
-    A.pressure[s] = pr;
-    part = double(err);
   }
   double t = block_sum_d(part, lds);
-  if (threadIdx.x == 0) A.partials[xcd_block()] = t;
+  if (threadIdx.x == 0) A.partials[qblk_] = t;
 }
-__global__ __launch_bounds__(kFinBlock) void k_ii_finalize(SceneTab T, DevArrays A) {
+__global__ __launch_bounds__(kFinBlock) void k_ii_finalize(SceneTab T, DevArrays A, unsigned parts) {
   __shared__ double lds[kFinBlock / 64];
   ALV_SCENE_BLOCK(T, A);
   StepCtl* ctl = A.ctl;
   if (ctl->dens_done) return;
   double part = 0.0;
-  for (unsigned b = blk_begin + threadIdx.x; b < blk_end; b += blockDim.x) part += A.partials[b];
+  for (unsigned b = blk_begin * parts + threadIdx.x; b < blk_end * parts; b += blockDim.x)
+    part += A.partials[b];
   double t = block_sum_d(part, lds);
   if (threadIdx.x == 0) {
     float mean = float(t / double(p.n));
@@ -2403,61 +2457,78 @@ __global__ __launch_bounds__(kFinBlock) void k_ii_finalize(SceneTab T, DevArrays
     publish_ctl(A, ctl, scene_);
   }
 }
+// sum += term(sp, x_j, f) over the pellet list of particle s, in list order,
+// with the reaction f at x_j added to the force and torque of the pellet's
+// body.  In the deep form the four lanes evaluate four entries; their reactions
+// follow one after the other, for a body's sums are read and written back.
+template <bool D, class Term>
+__device__ inline void pellet_forces(const SimParams& p, const DevArrays& A, unsigned s, unsigned q,
+                                     vec3& sum, Term term) {
+  const unsigned npn = A.pnnb[s];
+  for (unsigned t0 = 0; t0 < npn; t0 += D ? 4u : 1u) {
+    const unsigned t = D ? t0 + q : t0;
+    const bool ok = t < npn;
+    const unsigned sp = pellet_at(A.pnbr, A, s, ok ? t : npn - 1u);
+    vec3 xj, f;
+    const vec3 a = term(sp, xj, f);
+    sum = D ? quad_add3(sum, a, ok) : sum + a;
+    const unsigned b = A.pbody[sp];
+    const BoundaryDev& B = A.bnd[b];
+    auto react = [&] {
+      const size_t o = size_t(b) * A.cap + s;
+      const vec3 tq = cross(xj - mk(B.x[0], B.x[1], B.x[2]), f);
+      const float4 F = A.bforce[o], Tq = A.btorque[o];
+      A.bforce[o] = f4(ld3(F) + f, 0.f);
+      A.btorque[o] = f4(ld3(Tq) + tq, 0.f);
+    };
+    const bool hit = ok && B.accum;
+    if constexpr (D) {
+      if (__ballot(hit) != 0ull) {
+        for (unsigned l = 0; l < 4u; ++l) {
+          if (hit && q == l) react();
+          __threadfence_block();  // the next lane reads what this one wrote
+        }
+      }
+    } else if (hit) {
+      react();
+    }
+  }
+}
 // compute_pressure_accels (runner.hpp:2774-2817)
-template <bool W, bool PL>
+template <bool W, bool PL, bool D>
 __global__ __launch_bounds__(256) void k_ii_pressure_accel(SceneTab T, DevArrays A) {
-  ALV_SCENE(T, A, s);
+  ALV_SCENE_PASS(T, A, s, q, D ? kDeep : kGather, D ? kDeepLanes : 1u);
   if (must_wait(A)) return;
   if (s >= p.first + p.n) return;
   const vec3 xi = ld3(A.x[s]);
   const float dens = A.density[s];
   const float dens2 = dens * dens;
   const float dpi = A.pressure[s] / dens2;
-  vec3 ai = mk(0.f, 0.f, 0.f);
-  const unsigned nn = A.nnb[s];
-  for (unsigned t0 = 0; t0 < nn; t0 += kNB) {
-    unsigned j[kNB];
-    batch_ids(A, s, nn, t0, j);
-    float4 xj[kNB];
-    float djs[kNB], pj[kNB];
-#pragma unroll
-    for (int u = 0; u < kNB; ++u) {
-      xj[u] = A.x[j[u]];
-      djs[u] = A.density[j[u]];
-      pj[u] = A.pressure[j[u]];
-    }
-#pragma unroll
-    for (int u = 0; u < kNB; ++u) {
-      if (t0 + u < nn) {
-        vec3 xixj = wrapd<W>(xi - ld3(xj[u]), p);
-        float dj = djs[u];
-        float dj2 = dj * dj;
-        float dpj = pj[u] / dj2;
-        ai -= (p.mass * (dpi + dpj)) * grad_pair(xixj, p);
-      }
-    }
-  }
+  float sum[3] = {0.f, 0.f, 0.f};
+  list_sum<D, kListDeep>(
+      A.nbr, A, s, q, A.nnb[s], s, sum,
+      [&](unsigned j) { return EntryXSS{ld3(A.x[j]), A.density[j], A.pressure[j]}; },
+      [&](const EntryXSS& e, float (&t)[3]) {
+        const float dj2 = e.a * e.a;
+        const float dpj = e.b / dj2;
+        const vec3 g = (p.mass * (dpi + dpj)) * grad_pair(wrapd<W>(xi - e.x, p), p);
+        t[0] = -g.x;
+        t[1] = -g.y;
+        t[2] = -g.z;
+      });
+  vec3 ai = mk(sum[0], sum[1], sum[2]);
   if constexpr (PL) {
     // compute_pressure_accels_with_pellets (runner.hpp:2819-2870)
-    const unsigned npn = A.pnnb[s];
-    for (unsigned t = 0; t < npn; ++t) {
-      const unsigned sp = pellet_at(A.pnbr, A, s, t);
+    pellet_forces<D>(p, A, s, q, ai, [&](unsigned sp, vec3& xj, vec3& f) {
       const vec3 xixj = wrapd<W>(xi - ld3(A.px[sp]), p);
       const float dpj = A.pp[sp] / (p.rho0 * p.rho0);
       const vec3 acc = (p.mass * (dpi + dpj)) * grad_pair(xixj, p);
-      ai -= acc;
-      const unsigned b = A.pbody[sp];
-      const BoundaryDev& B = A.bnd[b];
-      if (B.accum) {
-        const size_t o = size_t(b) * A.cap + s;
-        const vec3 f = p.mass * acc;
-        const vec3 tq = cross((xi - xixj) - mk(B.x[0], B.x[1], B.x[2]), f);
-        float4 F = A.bforce[o], T = A.btorque[o];
-        A.bforce[o] = f4(ld3(F) + f, 0.f);
-        A.btorque[o] = f4(ld3(T) + tq, 0.f);
-      }
-    }
+      xj = xi - xixj;
+      f = p.mass * acc;
+      return mk(-acc.x, -acc.y, -acc.z);
+    });
   }
+  if (q != 0u) return;
   unsigned mask = PL ? 0u : A.bmask[s];
   while (mask) {
     const unsigned b = __builtin_ctz(mask);
@@ -2510,50 +2581,39 @@ __global__ __launch_bounds__(256) void k_is_advect(SceneTab T, DevArrays A) {
 }
 // calculate_isph_diagonal_adv_density (runner.hpp:2901-2949): the Jacobi
 // diagonal (times rho0) into aii, the advected density into adv_density
-template <bool W, bool PL>
+template <bool W, bool PL, bool D>
 __global__ __launch_bounds__(256) void k_is_diag(SceneTab T, DevArrays A) {
-  ALV_SCENE(T, A, s);
+  ALV_SCENE_PASS(T, A, s, q, D ? kDeep : kGather, D ? kDeepLanes : 1u);
   if (s >= p.first + p.n) return;
   const float dt = A.ctl->dt;
   const vec3 xi = ld3(A.x[s]), vi = ld3(A.v[s]);
   const float dens = A.density[s];
   const float eps = 0.01f * p.h2;
-  float dadv = dens / p.rho0;
-  float diag = 0.f;
-  const unsigned nn = A.nnb[s];
-  for (unsigned t0 = 0; t0 < nn; t0 += kNB) {
-    unsigned j[kNB];
-    batch_ids(A, s, nn, t0, j);
-    float4 xj[kNB], vj[kNB];
-    float djs[kNB];
-#pragma unroll
-    for (int u = 0; u < kNB; ++u) {
-      xj[u] = A.x[j[u]];
-      vj[u] = A.v[j[u]];
-      djs[u] = A.density[j[u]];
-    }
-#pragma unroll
-    for (int u = 0; u < kNB; ++u) {
-      if (t0 + u < nn) {
-        const vec3 xixj = wrapd<W>(xi - ld3(xj[u]), p);
+  float sum[2] = {dens / p.rho0, 0.f};
+  list_sum<D, kListDeep>(
+      A.nbr, A, s, q, A.nnb[s], s, sum,
+      [&](unsigned j) { return EntryXVS{ld3(A.x[j]), ld3(A.v[j]), A.density[j]}; },
+      [&](const EntryXVS& e, float (&t)[2]) {
+        const vec3 xixj = wrapd<W>(xi - e.x, p);
         const vec3 gw = grad_pair(xixj, p);
-        const float dj = djs[u];
-        dadv += dt * p.vol * dot(vi - ld3(vj[u]), gw);
-        diag += p.vol * (dens + dj) / (dens * dj) / (length_sqr(xixj) + eps) * dot(xixj, gw);
-      }
-    }
-  }
+        t[0] = dt * p.vol * dot(vi - e.v, gw);
+        t[1] = p.vol * (dens + e.a) / (dens * e.a) / (length_sqr(xixj) + eps) * dot(xixj, gw);
+      });
   if constexpr (PL) {
     // calculate_isph_diagonal_adv_density_with_pellets (runner.hpp:2951-3001)
-    const unsigned npn = A.pnnb[s];
-    for (unsigned t = 0; t < npn; ++t) {
-      const unsigned sp = pellet_at(A.pnbr, A, s, t);
-      const vec3 xixj = wrapd<W>(xi - ld3(A.px[sp]), p);
-      const vec3 g = p.vol * grad_pair(xixj, p);
-      dadv += dt * dot(vi - ld3(A.pv[sp]), g);
-      diag += (dens + p.rho0) / (dens * p.rho0) / (length_sqr(xixj) + eps) * dot(xixj, g);
-    }
-  } else {
+    list_sum<D, kListDeepWide>(
+        A.pnbr, A, s, q, A.pnnb[s], 0u, sum,
+        [&](unsigned j) { return EntryXV{ld3(A.px[j]), ld3(A.pv[j])}; },
+        [&](const EntryXV& e, float (&t)[2]) {
+          const vec3 xixj = wrapd<W>(xi - e.x, p);
+          const vec3 g = p.vol * grad_pair(xixj, p);
+          t[0] = dt * dot(vi - e.v, g);
+          t[1] = (dens + p.rho0) / (dens * p.rho0) / (length_sqr(xixj) + eps) * dot(xixj, g);
+        });
+  }
+  if (q != 0u) return;
+  float dadv = sum[0], diag = sum[1];
+  if constexpr (!PL) {
     unsigned mask = A.bmask[s];
     while (mask) {
       const unsigned b = __builtin_ctz(mask);
@@ -2571,10 +2631,10 @@ __global__ __launch_bounds__(256) void k_is_diag(SceneTab T, DevArrays A) {
   A.adv_density[s] = dadv;
 }
 // isph_solve_iteration (runner.hpp:2996-3042) + FP64 partial sums
-template <bool W, bool PL>
+template <bool W, bool PL, bool D>
 __global__ __launch_bounds__(256) void k_is_iter(SceneTab T, DevArrays A) {
   __shared__ double lds[4];
-  ALV_SCENE(T, A, s);
+  ALV_SCENE_PASS(T, A, s, q, D ? kDeep : kGather, D ? kDeepLanes : 1u);
   if (A.ctl->dens_done) return;
   const float dt = A.ctl->dt;
   const bool odd = (A.ctl->dens_iter & 1u) != 0u;
@@ -2590,51 +2650,40 @@ __global__ __launch_bounds__(256) void k_is_iter(SceneTab T, DevArrays A) {
     const float denom = diag * dt2;
     const float eps = 0.01f * p.h2;
     const float w = 2.0f / 3.0f;
-    float off = 0.f;
-    const unsigned nn = A.nnb[s];
-    for (unsigned t0 = 0; t0 < nn; t0 += kNB) {
-      unsigned j[kNB];
-      batch_ids(A, s, nn, t0, j);
-      float4 xj[kNB];
-      float djs[kNB], lpj[kNB];
-#pragma unroll
-      for (int u = 0; u < kNB; ++u) {
-        xj[u] = A.x[j[u]];
-        djs[u] = A.density[j[u]];
-        lpj[u] = lp[j[u]];
-      }
-#pragma unroll
-      for (int u = 0; u < kNB; ++u) {
-        if (t0 + u < nn) {
-          const vec3 xixj = wrapd<W>(xi - ld3(xj[u]), p);
-          const float dj = djs[u];
-          off -= p.vol * (dens + dj) / (dens * dj) / (length_sqr(xixj) + eps) *
-                 dot(xixj, grad_pair(xixj, p)) * lpj[u];
-        }
-      }
-    }
+    float sum[1] = {0.f};
+    list_sum<D, kListDeep>(
+        A.nbr, A, s, q, A.nnb[s], s, sum,
+        [&](unsigned j) { return EntryXSS{ld3(A.x[j]), A.density[j], lp[j]}; },
+        [&](const EntryXSS& e, float (&t)[1]) {
+          const vec3 xixj = wrapd<W>(xi - e.x, p);
+          t[0] = -(p.vol * (dens + e.a) / (dens * e.a) / (length_sqr(xixj) + eps) *
+                   dot(xixj, grad_pair(xixj, p)) * e.b);
+        });
     if constexpr (PL) {
       // isph_solve_iteration_with_pellets (runner.hpp:3055-3118): pellets
       // at rest density with the extrapolated pressure
-      const unsigned npn = A.pnnb[s];
-      for (unsigned t = 0; t < npn; ++t) {
-        const unsigned sp = pellet_at(A.pnbr, A, s, t);
-        const vec3 xixj = wrapd<W>(xi - ld3(A.px[sp]), p);
-        off -= p.vol * (dens + p.rho0) / (dens * p.rho0) / (length_sqr(xixj) + eps) *
-               dot(xixj, grad_pair(xixj, p)) * A.pp[sp];
-      }
+      list_sum<D, kListDeepWide>(
+          A.pnbr, A, s, q, A.pnnb[s], 0u, sum,
+          [&](unsigned j) { return EntryXS{ld3(A.px[j]), A.pp[j]}; },
+          [&](const EntryXS& e, float (&t)[1]) {
+            const vec3 xixj = wrapd<W>(xi - e.x, p);
+            t[0] = -(p.vol * (dens + p.rho0) / (dens * p.rho0) / (length_sqr(xixj) + eps) *
+                     dot(xixj, grad_pair(xixj, p)) * e.a);
+          });
     }
-    off *= p.rho0;
-    float pr = 0.f;
-    if (fabsf(denom) > 1.0e-9f)
-      pr = std_max((1.0f - w) * lp[s] + w * (bb / denom - off / diag), 0.0f);
-    const float err = pr == 0.f ? 0.f : (denom * pr + off * dt2 - bb);
-    A.density_err[s] = err;
-    out[s] = pr;
-    part = double(err);
+    if (q == 0u) {
+      const float off = sum[0] * p.rho0;
+      float pr = 0.f;
+      if (fabsf(denom) > 1.0e-9f)
+        pr = std_max((1.0f - w) * lp[s] + w * (bb / denom - off / diag), 0.0f);
+      const float err = pr == 0.f ? 0.f : (denom * pr + off * dt2 - bb);
+      A.density_err[s] = err;
+      out[s] = pr;
+      part = double(err);
+    }
   }
   double t = block_sum_d(part, lds);
-  if (threadIdx.x == 0) A.partials[xcd_block()] = t;
+  if (threadIdx.x == 0) A.partials[qblk_] = t;
 }
 // After an even, non-zero number of iterations the result is in
 // last_pressure; with none, `pressure` keeps the previous step's values, as
@@ -2989,40 +3038,36 @@ __global__ __launch_bounds__(64) void k_pellet_bead_lists(SceneTab T, DevArrays 
 }
 // compute_viscosity_with_pellets (runner.hpp:2251-2297) with
 // clear_acceleration and the per-block CFL maxima, as k_viscosity
-template <bool W>
+template <bool W, bool D>
 __global__ __launch_bounds__(256) void k_viscosity_pellets(SceneTab T, DevArrays A) {
   __shared__ float lds[4];
-  ALV_SCENE(T, A, s);
+  ALV_SCENE_PASS(T, A, s, q, D ? kDeep : kGather, D ? kDeepLanes : 1u);
   const float dt = A.ctl->dt;
   float cfl = -FLT_MAX;
   if (s < p.first + p.n) {
     const vec3 xi = ld3(A.x[s]), vi = ld3(A.v[s]);
-    vec3 da = viscosity_sum<W>(p, A, s, xi, vi, A.nnb[s], GlobalXV{A.x, A.v});
-    const unsigned npn = A.pnnb[s];
-    for (unsigned t = 0; t < npn; ++t) {
-      const unsigned sp = pellet_at(A.pnbr, A, s, t);
+    vec3 da;
+    if constexpr (D)
+      velocity_divergence_deep<W, true>(p, A, s, q, xi, vi, A.nnb[s], &da);
+    else
+      da = viscosity_sum<W>(p, A, s, xi, vi, A.nnb[s], GlobalXV{A.x, A.v});
+    pellet_forces<D>(p, A, s, q, da, [&](unsigned sp, vec3& xj, vec3& f) {
       const vec3 xixj = wrapd<W>(xi - ld3(A.px[sp]), p);
       const vec3 acc = (p.vol * p.bvisc * dot(xixj, grad_pair(xixj, p)) /
                         (length_sqr(xixj) + 0.01f * p.h2)) *
                        (vi - ld3(A.pv[sp]));
-      da += acc;
-      const unsigned b = A.pbody[sp];
-      const BoundaryDev& B = A.bnd[b];
-      if (B.accum) {
-        const size_t o = size_t(b) * A.cap + s;
-        const vec3 f = (-p.mass) * acc;
-        const vec3 tq = cross((xi - xixj) - mk(B.x[0], B.x[1], B.x[2]), f);
-        float4 F = A.bforce[o], Tq = A.btorque[o];
-        A.bforce[o] = f4(ld3(F) + f, 0.f);
-        A.btorque[o] = f4(ld3(Tq) + tq, 0.f);
-      }
+      xj = xi - xixj;
+      f = (-p.mass) * acc;
+      return acc;
+    });
+    if (q == 0u) {
+      const vec3 a = mk(p.g[0], p.g[1], p.g[2]) + da;
+      A.a[s] = f4(a, 0.f);
+      cfl = length_sqr(vi + a * dt);
     }
-    const vec3 a = mk(p.g[0], p.g[1], p.g[2]) + da;
-    A.a[s] = f4(a, 0.f);
-    cfl = length_sqr(vi + a * dt);
   }
   float m = block_max_f(cfl, lds);
-  if (threadIdx.x == 0) A.fpartials[xcd_block()] = m;
+  if (threadIdx.x == 0) A.fpartials[qblk_] = m;
 }
 
 // Pseudo-inverse of the symmetric 3x3 moment matrix of the MLS plane fit
@@ -3167,24 +3212,10 @@ KernelProfiler* g_profiler = nullptr;
                          __VA_ARGS__);                                            \
     if (g_profiler) g_profiler->end(#kernel, s);                                  \
   } while (0)
-// neighbour passes with an LDS-tile instance (never with the periodic wrap):
-// the gather instances reserve no LDS, so they keep their occupancy
-#define ALV_LAUNCH_WT(kernel, L, s, ...)                                          \
-  do {                                                                            \
-    if (g_profiler) g_profiler->begin(#kernel, s);                                \
-    if ((L).p0.wrap_mask)                                                         \
-      hipLaunchKernelGGL((kernel<true, false>), dim3((L).pblocks), dim3(kBlock), 0, s, (L).T, \
-                         __VA_ARGS__);                                            \
-    else if ((L).tiles)                                                           \
-      hipLaunchKernelGGL((kernel<false, true>), dim3((L).pblocks), dim3(kBlock), 0, s, (L).T, \
-                         __VA_ARGS__);                                            \
-    else                                                                          \
-      hipLaunchKernelGGL((kernel<false, false>), dim3((L).pblocks), dim3(kBlock), 0, s, (L).T, \
-                         __VA_ARGS__);                                            \
-    if (g_profiler) g_profiler->end(#kernel, s);                                  \
-  } while (0)
 // neighbour passes (ALV_SCENE_PASS) in the form of the launch: LANES is
-// change_lanes or stiffness_lanes; KERNEL(W, M) names the instance
+// change_lanes or stiffness_lanes; KERNEL(W, M) names the instance.  Only the
+// tile instances (never with the periodic wrap) reserve LDS for the tile, so
+// the gather instances keep their occupancy.
 #define ALV_LAUNCH_FORM(KERNEL, W, M, LANES, L, s, ...)                           \
   hipLaunchKernelGGL((KERNEL(W, M)), dim3((L).pblocks * ((M) == kDeep ? kBlock / kDeepBlock : 1u)), \
                      dim3(pass_threads(M, LANES(M))), 0, s, (L).T, __VA_ARGS__)
@@ -3202,20 +3233,6 @@ KernelProfiler* g_profiler = nullptr;
     else                                                                          \
       ALV_LAUNCH_FORM(KERNEL, false, kGather, LANES, L, s, __VA_ARGS__);          \
     if (g_profiler) g_profiler->end(name, s);                                     \
-  } while (0)
-#define ALV_LAUNCH_W2T(kernel, flag, L, s, ...)                                   \
-  do {                                                                            \
-    if (g_profiler) g_profiler->begin(#kernel, s);                                \
-    if ((L).p0.wrap_mask)                                                         \
-      hipLaunchKernelGGL((kernel<true, flag, false>), dim3((L).pblocks), dim3(kBlock), 0, s, \
-                         (L).T, __VA_ARGS__);                                     \
-    else if ((L).tiles)                                                           \
-      hipLaunchKernelGGL((kernel<false, flag, true>), dim3((L).pblocks), dim3(kBlock), 0, s, \
-                         (L).T, __VA_ARGS__);                                     \
-    else                                                                          \
-      hipLaunchKernelGGL((kernel<false, flag, false>), dim3((L).pblocks), dim3(kBlock), 0, s, \
-                         (L).T, __VA_ARGS__);                                     \
-    if (g_profiler) g_profiler->end(#kernel, s);                                  \
   } while (0)
 // kernels templated on the periodic wrap: one name for both instances
 #define ALV_LAUNCH_W(kernel, L, s, ...)                                           \
@@ -3344,6 +3361,18 @@ void launch_neighbors(const Launch& L, const DevArrays& A, int with_factor, hipS
 #define K_P_ITER(W, M) k_p_iter<W, M>
 #define K_P_ERR(W, M) k_p_err<W, M>
 #define K_DENSITY_CHANGE(W, M) k_density_change<W, M>
+#define K_VISCOSITY(W, M) k_viscosity<W, M>
+#define K_VISCOSITY_PELLETS(W, M) k_viscosity_pellets<W, (M) == kDeep>
+#define K_II_PREDICT0(W, M) k_ii_predict0<W, (M) == kDeep>
+#define K_II_PREDICT1(W, M) k_ii_predict1<W, (M) == kDeep>
+#define K_II_ITER0(W, M) k_ii_iter0<W, (M) == kDeep>
+#define K_II_ITER1(W, M) k_ii_iter1<W, (M) == kDeep>
+#define K_II_PRESSURE_ACCEL(W, M) k_ii_pressure_accel<W, false, (M) == kDeep>
+#define K_II_PRESSURE_ACCEL_PL(W, M) k_ii_pressure_accel<W, true, (M) == kDeep>
+#define K_IS_DIAG(W, M) k_is_diag<W, false, (M) == kDeep>
+#define K_IS_DIAG_PL(W, M) k_is_diag<W, true, (M) == kDeep>
+#define K_IS_ITER(W, M) k_is_iter<W, false, (M) == kDeep>
+#define K_IS_ITER_PL(W, M) k_is_iter<W, true, (M) == kDeep>
 
 void launch_df_warm_start_div(const Launch& L, const DevArrays& A, hipStream_t s,
                               int features, const MlpDev* net, int net_divergence, int fused) {
@@ -3366,10 +3395,10 @@ void launch_df_div_iteration(const Launch& L, const DevArrays& A, hipStream_t s)
   ALV_LAUNCH_FIN(k_div_finalize, L, s, A, parts_per_block(L));
 }
 void launch_df_viscosity(const Launch& L, const DevArrays& A, hipStream_t s) {
-  ALV_LAUNCH_WT(k_viscosity, L, s, A);
+  ALV_LAUNCH_PASS("k_viscosity", K_VISCOSITY, stiffness_lanes, L, s, A);
 }
-void launch_update_dt(const Launch& L, const DevArrays& A, int pass_parts, hipStream_t s) {
-  ALV_LAUNCH_FIN(k_update_dt, L, s, A, pass_parts ? parts_per_block(L) : 1u);
+void launch_update_dt(const Launch& L, const DevArrays& A, hipStream_t s) {
+  ALV_LAUNCH_FIN(k_update_dt, L, s, A, parts_per_block(L));
 }
 void launch_df_integrate_np(const Launch& L, const DevArrays& A, int fin, hipStream_t s) {
   ALV_LAUNCH(k_integrate_np, L, s, A, fin);
@@ -3402,30 +3431,30 @@ void launch_integrate_velocity(const Launch& L, const DevArrays& A, float dt, hi
   ALV_LAUNCH_W(k_integrate_velocity, L, s, A, dt);
 }
 void launch_ii_viscosity_predict(const Launch& L, const DevArrays& A, hipStream_t s) {
-  ALV_LAUNCH_WT(k_viscosity, L, s, A);
+  ALV_LAUNCH_PASS("k_viscosity", K_VISCOSITY, stiffness_lanes, L, s, A);
 }
 void launch_ii_predict(const Launch& L, const DevArrays& A, hipStream_t s) {
-  ALV_LAUNCH_W(k_ii_predict0, L, s, A);
-  ALV_LAUNCH_W(k_ii_predict1, L, s, A);
+  ALV_LAUNCH_PASS("k_ii_predict0", K_II_PREDICT0, stiffness_lanes, L, s, A);
+  ALV_LAUNCH_PASS("k_ii_predict1", K_II_PREDICT1, stiffness_lanes, L, s, A);
 }
 void launch_ii_iteration(const Launch& L, const DevArrays& A, hipStream_t s) {
-  ALV_LAUNCH_W(k_ii_iter0, L, s, A);
-  ALV_LAUNCH_W(k_ii_iter1, L, s, A);
-  ALV_LAUNCH_FIN(k_ii_finalize, L, s, A);
+  ALV_LAUNCH_PASS("k_ii_iter0", K_II_ITER0, stiffness_lanes, L, s, A);
+  ALV_LAUNCH_PASS("k_ii_iter1", K_II_ITER1, stiffness_lanes, L, s, A);
+  ALV_LAUNCH_FIN(k_ii_finalize, L, s, A, parts_per_block(L));
 }
 void launch_is_prepare(const Launch& L, const DevArrays& A, hipStream_t s) {
   ALV_LAUNCH(k_is_advect, L, s, A);
-  ALV_LAUNCH_W2(k_is_diag, false, L, s, A);
+  ALV_LAUNCH_PASS("k_is_diag", K_IS_DIAG, stiffness_lanes, L, s, A);
 }
 void launch_is_iteration(const Launch& L, const DevArrays& A, hipStream_t s) {
-  ALV_LAUNCH_W2(k_is_iter, false, L, s, A);
-  ALV_LAUNCH_FIN(k_ii_finalize, L, s, A);
+  ALV_LAUNCH_PASS("k_is_iter", K_IS_ITER, stiffness_lanes, L, s, A);
+  ALV_LAUNCH_FIN(k_ii_finalize, L, s, A, parts_per_block(L));
 }
 void launch_is_settle(const Launch& L, const DevArrays& A, hipStream_t s) {
   ALV_LAUNCH(k_is_settle, L, s, A);
 }
 void launch_ii_finish(const Launch& L, const DevArrays& A, hipStream_t s) {
-  ALV_LAUNCH_W2(k_ii_pressure_accel, false, L, s, A);
+  ALV_LAUNCH_PASS("k_ii_pressure_accel", K_II_PRESSURE_ACCEL, stiffness_lanes, L, s, A);
   ALV_LAUNCH_W(k_ii_finish, L, s, A);
 }
 void launch_body_sums(const Launch& L, const DevArrays& A, hipStream_t s) {
@@ -3521,22 +3550,22 @@ void launch_pellet_lists(const Launch& L, const Launch& Lp, const DevArrays& A, 
   if (Lp.active) ALV_LAUNCH_QUAD(k_pellet_bead_lists, Lp, s, A);
 }
 void launch_pellet_viscosity(const Launch& L, const DevArrays& A, hipStream_t s) {
-  ALV_LAUNCH_W(k_viscosity_pellets, L, s, A);
+  ALV_LAUNCH_PASS("k_viscosity_pellets", K_VISCOSITY_PELLETS, stiffness_lanes, L, s, A);
 }
 void launch_is_prepare_pellets(const Launch& L, const DevArrays& A, hipStream_t s) {
   ALV_LAUNCH(k_is_advect, L, s, A);
-  ALV_LAUNCH_W2(k_is_diag, true, L, s, A);
+  ALV_LAUNCH_PASS("k_is_diag", K_IS_DIAG_PL, stiffness_lanes, L, s, A);
 }
 void launch_is_iteration_pellets(const Launch& L, const Launch& Lp, const DevArrays& A,
                                  hipStream_t s) {
   if (Lp.active) ALV_LAUNCH_QUAD(k_extrapolate, Lp, s, A, 0);
-  ALV_LAUNCH_W2(k_is_iter, true, L, s, A);
-  ALV_LAUNCH_FIN(k_ii_finalize, L, s, A);
+  ALV_LAUNCH_PASS("k_is_iter", K_IS_ITER_PL, stiffness_lanes, L, s, A);
+  ALV_LAUNCH_FIN(k_ii_finalize, L, s, A, parts_per_block(L));
 }
 void launch_is_finish_pellets(const Launch& L, const Launch& Lp, const DevArrays& A,
                               hipStream_t s) {
   if (Lp.active) ALV_LAUNCH_QUAD(k_extrapolate, Lp, s, A, 1);
-  ALV_LAUNCH_W2(k_ii_pressure_accel, true, L, s, A);
+  ALV_LAUNCH_PASS("k_ii_pressure_accel", K_II_PRESSURE_ACCEL_PL, stiffness_lanes, L, s, A);
   ALV_LAUNCH_W(k_ii_finish, L, s, A);
 }
 

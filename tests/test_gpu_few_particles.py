@@ -77,6 +77,15 @@ def test_both_sides_of_the_limits(n, wrap):
     step_matches(cloud(n, (22, 24, 20), 7, wrap=wrap))
 
 
+@pytest.mark.parametrize("kind", ["ii", "i"])
+@pytest.mark.parametrize("n,cells,kmax", [(17, (4, 4, 4), 64), (900, (4, 4, 4), 7),
+                                          (900, (4, 4, 4), 41), (900, (4, 4, 4), 90),
+                                          (98305, (22, 24, 20), 64)])
+def test_pressure_solvers(n, cells, kmax, kind):
+    # a wave's last particles, lists of one and of several rounds, the other form
+    step_matches(cloud(n, cells, 9, kmax=kmax), kind)
+
+
 @pytest.mark.parametrize("ns", [1, 15, 65, 300])
 @pytest.mark.parametrize("kmax,wrap", [(7, None), (64, None), (40, (True, True, True)),
                                        (64, (True, False, True))])
