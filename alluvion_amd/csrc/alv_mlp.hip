@@ -2,15 +2,16 @@
 // warm-start network (see alv_mlp.hpp for the operand layout), and its C ABI.
 //
 // Training step (all on the device, one stream):
-//   k_mlp_gather      random mini-batch, normalised inputs and targets
-//   k_mlp_fwd_bwd     forward + backward through the activations, per tile
-//                     of 16 samples, register-chained MFMAs; writes the bf16
-//                     activations and deltas feature-major ([unit][sample])
+//   k_mlp_fwd_bwd     draws and normalises its samples; forward + backward
+//                     through the activations, one tile of 16 samples per
+//                     wave, register-chained MFMAs; writes the bf16
+//                     activations and deltas in tiles of 16 samples
 //   k_mlp_wgrad       weight and bias gradients, MFMA with the batch as the
 //                     contraction dimension, one partial per sample chunk
-//   k_mlp_reduce      partials -> gradient, fixed order (deterministic)
-//   k_mlp_adam        Adam on the FP32 master parameters
+//   k_mlp_adam        partials -> gradient in fixed order (deterministic),
+//                     Adam on the FP32 master parameters
 //   k_mlp_pack        FP32 parameters -> permuted bf16 operands
+// The gradient alone (alv_mlp_loss_grad): the first two, then k_mlp_reduce.
 #include <hip/hip_runtime.h>
 
 #include <cmath>

@@ -5,8 +5,9 @@
 // variable.hpp:286-290; ascending particle id inside a cell).  All per-step
 // passes run in that sorted order on SoA arrays, so a wavefront's 64 lanes
 // touch neighbouring particles and the neighbour gathers stay in L2.  The
-// neighbour list stores u32 sorted indices column-major ([slot][particle]) so
-// that slot t of 64 lanes is one 256-byte coalesced load; displacements are
+// neighbour list stores u32 sorted indices in groups of four slots, in tiles
+// of 64 particles (nbr_group), so that a group of 64 lanes is one coalesced
+// 1 KB load; displacements are
 // recomputed from positions (bit-identical to the reference's stored x_ij,
 // because positions do not change inside a step).
 //
