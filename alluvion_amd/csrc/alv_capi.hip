@@ -1890,7 +1890,9 @@ int solver_launch(alv_solver* S, Launch* L) {
   L->scenes = unsigned(ns);
   L->active = active;
   L->tiles = S->A.use_tiles;
-  L->deep = !L->tiles && pblocks <= kDeepMaxBlocks;
+  const bool again = S->kind != ALV_SOLVER_DF && pblocks > kDeepAgainBlocks &&
+                     pblocks <= kDeepAgainMaxBlocks;
+  L->deep = !L->tiles && (pblocks <= kDeepMaxBlocks || again);
   L->quad = !L->tiles && pblocks <= kQuadMaxBlocks;
   L->p0 = S->par_host[0];
   return ALV_OK;

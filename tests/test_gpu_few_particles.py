@@ -80,7 +80,9 @@ def test_both_sides_of_the_limits(n, wrap):
 @pytest.mark.parametrize("kind", ["ii", "i"])
 @pytest.mark.parametrize("n,cells,kmax", [(17, (4, 4, 4), 64), (900, (4, 4, 4), 7),
                                           (900, (4, 4, 4), 41), (900, (4, 4, 4), 90),
-                                          (98305, (22, 24, 20), 64)])
+                                          (98305, (22, 24, 20), 64),
+                                          (131072, (24, 26, 24), 64),
+                                          (131073, (24, 26, 24), 64)])
 def test_pressure_solvers(n, cells, kmax, kind):
     # a wave's last particles, lists of one and of several rounds, the other form
     step_matches(cloud(n, cells, 9, kmax=kmax), kind)
