@@ -72,8 +72,7 @@ def test_empty_solver_steps():
     assert not count.any() and not anomaly.any()
 
 
-@pytest.mark.parametrize("kind", ["df", "ii", "i"])
-def test_free_body_driven_by_fluid_matches_oracle(kind):
+def free_body_matches(kind, tiles=False):
     """A rotated free box hit by a fluid block (no gravity, no viscosity):
     fluid velocities and the body's kinematics over three steps."""
     x = scenes.lattice_block(12, 12, 12, 0.0025, -0.03, 7, 0.00025)
@@ -89,6 +88,7 @@ def test_free_body_driven_by_fluid_matches_oracle(kind):
                       boundary_viscosity=0.0, boundaries=[body], grid_offset=(-8, -8, -8),
                       grid_res=(16, 16, 16))
     dp, pile, solver, _, _ = scenes.build_solver(sc, kind)
+    solver.set_tiles(tiles)
     orc = oracle_like(sc, dp, pile, kind=kind)
     n = sc.n
     for step in range(3):
@@ -108,3 +108,8 @@ def test_free_body_driven_by_fluid_matches_oracle(kind):
         np.testing.assert_allclose([qg.x, qg.y, qg.z, qg.w], rb["q"], rtol=0, atol=1e-6,
                                    err_msg=str(step))
     assert np.abs(orc.rigid(0)["omega"]).max() > 1e-3  # the fluid turns the box
+
+
+@pytest.mark.parametrize("kind", ["df", "ii", "i"])
+def test_free_body_driven_by_fluid_matches_oracle(kind):
+    free_body_matches(kind)

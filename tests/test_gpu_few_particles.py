@@ -30,8 +30,9 @@ def cloud(n, cells, seed, wrap=None, kmax=64, margin=0, density=1.0):
         max_divergence_solve=3, max_density_solve=4)
 
 
-def step_matches(sc, kind="df"):
+def step_matches(sc, kind="df", tiles=False):
     dp, pile, solver, _, _ = scenes.build_solver(sc, kind)
+    solver.set_tiles(tiles)
     orc = oracle_for(sc, dp, [], kind=kind)
     solver.update_particle_neighbors()
     orc.update_particle_neighbors()

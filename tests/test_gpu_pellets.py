@@ -109,10 +109,11 @@ def body_state(pile, b):
             np.array([q.x, q.y, q.z, q.w]), np.array(list(pile.get_omega(b))))
 
 
-def test_isph_steps_with_pellets_match_oracle():
+def isph_steps_match(tiles=False):
     from alluvion_amd import scenes
     sc = small_scene()
     dp, pile, solver, _, _ = scenes.build_solver(sc, kind="i")
+    solver.set_tiles(tiles)
     orc = of.Oracle(sc, precision=4, kind="i")
     n, mx, npel = sc.n, orc.max_n, pile.num_pellets
     for step in range(5):
@@ -137,6 +138,10 @@ def test_isph_steps_with_pellets_match_oracle():
         np.testing.assert_allclose(w, rb["omega"], rtol=1e-4, atol=1e-5, err_msg=str(step))
     assert np.abs(orc.rigid(1)["v"]).max() > 0  # the fluid pushes the sphere
     assert p_o[mx:mx + npel].max() > 0  # pellets carry pressure
+
+
+def test_isph_steps_with_pellets_match_oracle():
+    isph_steps_match()
 
 
 def test_pellet_contacts_match_oracle():
