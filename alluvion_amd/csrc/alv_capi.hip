@@ -1890,9 +1890,7 @@ int solver_launch(alv_solver* S, Launch* L) {
   L->scenes = unsigned(ns);
   L->active = active;
   L->tiles = S->A.use_tiles;
-  const bool again = S->kind != ALV_SOLVER_DF && pblocks > kDeepAgainBlocks &&
-                     pblocks <= kDeepAgainMaxBlocks;
-  L->deep = !L->tiles && (pblocks <= kDeepMaxBlocks || again);
+  L->deep = !L->tiles && pblocks <= kDeepMaxBlocks;
   L->quad = !L->tiles && pblocks <= kQuadMaxBlocks;
   L->p0 = S->par_host[0];
   return ALV_OK;

@@ -134,16 +134,12 @@ constexpr unsigned kDeepBlock = 64;
 // form of the passes: 80,000 particles 258 and 237 us, 101,000 259 and 258,
 // 130,000 263 and 284 (four lanes waste the lists' tails and the chip is
 // full); of the search: 60,000 218 and 202, 80,000 258 and 251, 101,000 259
-// and 264, periodic 85,000 281 and 290.
+// and 264, periodic 85,000 281 and 290.  IISPH and ISPH steps cross over at the
+// same size (with one lane and with four: 91,125 particles IISPH 216 and 208 us,
+// ISPH 183 and 178; 99,452 221 and 222, 190 and 190) and stay with one lane past
+// it: 262,144 particles IISPH 348 and 388, ISPH 276 and 314, with pellets 512
+// and 548; 524,880 621 and 652, 474 and 518.
 constexpr unsigned kDeepMaxBlocks = 384;
-// IISPH and ISPH steps take the deep passes again where one lane per particle
-// leaves the chip in a third, partly empty round of blocks: past two blocks on
-// each of 256 CUs, up to where both forms meet.  Steps with one lane and with
-// four: 115,248 particles IISPH 227 and 233 us, ISPH 190 and 198; 130,050 235 and
-// 245, 191 and 204; 151,686 302 and 280, 236 and 233; 201,840 369 and 340, 287
-// and 278; 405,224 582 and 534, 434 and 423; 1,000,000 1,372 and 1,374, 855 and
-// 849.
-constexpr unsigned kDeepAgainBlocks = 512, kDeepAgainMaxBlocks = 4096;
 constexpr unsigned kQuadMaxBlocks = 320;
 
 // Neighbour slots are stored in groups of four (one uint4 per particle and

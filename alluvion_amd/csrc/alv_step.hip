@@ -3427,9 +3427,7 @@ void launch_export_pairs(const Launch& L, const DevArrays& A, float* x, float* y
   ALV_LAUNCH(k_export_pairs, L, s, A, x, y);
 }
 void launch_density_change(const Launch& L, const DevArrays& A, hipStream_t s) {
-  Launch D = L;  // as in a DFSPH step: no deep form past kDeepMaxBlocks
-  D.deep = L.deep && L.pblocks <= kDeepMaxBlocks;
-  ALV_LAUNCH_PASS("k_density_change", K_DENSITY_CHANGE, change_lanes, D, s, A);
+  ALV_LAUNCH_PASS("k_density_change", K_DENSITY_CHANGE, change_lanes, L, s, A);
 }
 void launch_integrate_velocity(const Launch& L, const DevArrays& A, float dt, hipStream_t s) {
   ALV_LAUNCH_W(k_integrate_velocity, L, s, A, dt);
