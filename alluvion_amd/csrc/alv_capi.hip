@@ -1852,6 +1852,7 @@ int solver_launch(alv_solver* S, Launch* L) {
   const size_t ns = S->scenes.size();
   bool changed = !S->par_valid;
   unsigned pblocks = 0, active = 0;
+  L->loose = 1;
   for (size_t k = 0; k < ns; ++k) {
     const auto& sc = S->scenes[k];
     SimParams p = make_params(S->cn, S->cni, unsigned(sc.pile->bnd.size()), sc.n);
@@ -1860,6 +1861,7 @@ int solver_launch(alv_solver* S, Launch* L) {
       p.off[a] = sc.off[a];
     }
     p.wrap_tight = wrap_is_tight(p);
+    if (p.wrap_tight) L->loose = 0;
     p.num_cells = sc.num_cells;
     p.first = sc.first;
     p.span = sc.span;
@@ -2316,7 +2318,8 @@ int alv_solver_step(alv_solver* S) {
     const MlpDev mv = mlp_device_view(S->net);
     const unsigned long long base = (unsigned long long)L.pblocks << 24 ^
                                     (unsigned long long)(L.active != 0) << 23 ^
-                                    (unsigned long long)(L.p0.wrap_mask != 0) << 22;
+                                    (unsigned long long)(L.p0.wrap_mask != 0) << 22 ^
+                                    (unsigned long long)L.loose << 21;
     const unsigned long long keyA =
         base ^ ((unsigned long long)cdiv << 8) ^ (div << 1) ^ (S->log_features << 2) ^
         ((S->net != nullptr) << 3) ^ (S->net_div << 4) ^

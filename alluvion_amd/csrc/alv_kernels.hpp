@@ -186,6 +186,7 @@ struct Launch {
   int tiles;         // launch the LDS-tile instances of the neighbour passes
   int deep;          // launch the deep instances (few particles)
   int quad;          // launch the four-lane neighbour search (few particles)
+  int loose;         // no scene's cells fill its periodic box (SimParams::wrap_tight)
 };
 // partial sums and maxima of a pass per 256-particle block
 inline unsigned parts_per_block(const Launch& L) {

@@ -616,13 +616,21 @@ __device__ inline unsigned run_shift(unsigned k, unsigned o1, unsigned o2, unsig
   return k >= o3 ? s3 : at;
 }
 
-// One wave per block (its LDS is its own), so that few particles spread over
-// the chip: 10.9 KB a wave, 14 waves per CU.  The tile instance keeps blocks
-// of 256 particles (its tiles') and is bounded to 64 VGPRs.
-template <bool W, bool TL>
-__global__ __launch_bounds__(TL ? 256 : 64, TL ? 8 : 4) void k_neighbors(SceneTab T, DevArrays A,
-                                                                         int with_factor) {
-  constexpr bool kWaveStage = !TL;
+// Forms of the search.  Staged: one wave per block (its LDS is its own), so
+// that few particles spread over the chip: 10.9 KB a wave, 14 waves per CU.
+// The others hold no stage and are bounded to 64 VGPRs for 8 waves per SIMD:
+// from the LDS tile of a block of 256 particles, or from global memory where no
+// wave of a launch could stage its rows (periodic boxes that the cells do not
+// fill).  A neighbour update of a million random particles in such a box,
+// periodic on x, on z and on all axes: 468, 490 and 544 us, in the staged
+// instance's general loop 524, 535 and 545; of 500,000 in a box four cells
+// high 509 and 587.
+enum { kSearchStaged = 0, kSearchPlain = 1, kSearchTile = 2 };
+template <bool W, int F>
+__global__ __launch_bounds__(F == kSearchTile ? 256 : 64, F == kSearchStaged ? 4 : 8)
+void k_neighbors(SceneTab T, DevArrays A, int with_factor) {
+  constexpr bool kWaveStage = F == kSearchStaged;
+  constexpr bool TL = F == kSearchTile;
   __shared__ float4 st[kWaveStage ? kStage + kCB : 1];
   __shared__ unsigned list_[kWaveStage ? kListLds : 1][64];
   __shared__ int4 runs_[kWaveStage ? kRuns : 1];  // column x, y and first and last cell z
@@ -733,6 +741,14 @@ __global__ __launch_bounds__(TL ? 256 : 64, TL ? 8 : 4) void k_neighbors(SceneTa
   using NoClamp = std::integral_constant<bool, false>;
   auto global_x = [&](unsigned j, unsigned) { return A.x[j]; };
   auto wrapped_d = [&](vec3 x) { return wrapd<W>(xi - x, p); };
+  // by axis: cheaper where only one is periodic
+  auto axes_d = [&](vec3 x) {
+    vec3 d = xi - x;
+    if (p.wrap_mask & 1) d.x = wrap1(d.x, p.wrap_len[0], p.wrap_min[0], p.wrap_max[0]);
+    if (p.wrap_mask & 2) d.y = wrap1(d.y, p.wrap_len[1], p.wrap_min[1], p.wrap_max[1]);
+    if (p.wrap_mask & 4) d.z = wrap1(d.z, p.wrap_len[2], p.wrap_min[2], p.wrap_max[2]);
+    return d;
+  };
   // the column of row r, wrapped on periodic axes, whether it can hold a
   // neighbour, and the cells above and below that can
   struct Row {
@@ -880,33 +896,55 @@ __global__ __launch_bounds__(TL ? 256 : 64, TL ? 8 : 4) void k_neighbors(SceneTa
   }
   // The 27 cells in the reference order (dx outer, dz inner): for each
   // (dx, dy) row the up-to-3 cells along z are contiguous in the sorted
-  // order unless a periodic wrap splits them, so each row is 1-3 spans.
+  // order unless a periodic wrap splits them, so each row is 1-3 spans.  A
+  // row's spans are found first, so that the lanes of a wave scan theirs
+  // together: scanned where each lane's cells end, a row costs the wave up to
+  // three scans in place of one (a million particles from LDS tiles 423 us a
+  // search, 290 this way).
   if (!staged) {
+    const bool split = W && (p.wrap_mask & 4);
 #pragma unroll 1
     for (int r = 0; r < 9; ++r) {
       const Row w = row_of(r);
       if (!w.ok) continue;
-      unsigned b = 0u, e = 0u;  // the span being extended
-      int prev = -2;
-#pragma unroll 1
-      for (int dz = w.dz_lo; dz <= w.dz_hi + 1; ++dz) {
-        int nz = ip[2] + dz;
-        if (W && (p.wrap_mask & 4)) nz = nz >= p.res[2] ? nz - p.res[2] : (nz < 0 ? nz + p.res[2] : nz);
-        const bool use = dz <= w.dz_hi && nz >= 0 && nz < p.res[2];
-        const unsigned c = w.column + unsigned(nz);
-        if (use && nz == prev + 1) {
-          e = A.cell_start[c + 1u];
+      unsigned b0 = 0u, e0 = 0u, b1 = 0u, e1 = 0u, b2 = 0u, e2 = 0u;
+      if (split) {
+        int prev = -2, k = 0;  // k spans so far
+#pragma unroll
+        for (int dz = -1; dz <= 1; ++dz) {
+          int nz = ip[2] + dz;
+          nz = nz >= p.res[2] ? nz - p.res[2] : (nz < 0 ? nz + p.res[2] : nz);
+          if (dz < w.dz_lo || dz > w.dz_hi || nz < 0 || nz >= p.res[2]) continue;
+          const unsigned b = A.cell_start[w.column + unsigned(nz)];
+          const unsigned e = A.cell_start[w.column + unsigned(nz) + 1u];
+          if (nz != prev + 1) {
+            ++k;
+            b0 = k == 1 ? b : b0;
+            b1 = k == 2 ? b : b1;
+            b2 = k == 3 ? b : b2;
+          }
+          e0 = k == 1 ? e : e0;
+          e1 = k == 2 ? e : e1;
+          e2 = k == 3 ? e : e2;
           prev = nz;
-          continue;
         }
+      } else {
+        const int z0 = max(ip[2] + w.dz_lo, 0), z1 = min(ip[2] + w.dz_hi, p.res[2] - 1);
+        if (z0 <= z1) {
+          b0 = A.cell_start[w.column + unsigned(z0)];
+          e0 = A.cell_start[w.column + unsigned(z1) + 1u];
+        }
+      }
+#pragma unroll 1
+      for (int q = 0; q < (split ? 3 : 1); ++q) {
+        const unsigned b = q == 0 ? b0 : (q == 1 ? b1 : b2), e = q == 0 ? e0 : (q == 1 ? e1 : e2);
         if (tiled_)
           scan_span(b, e, [&](unsigned j, unsigned) { return tile_.X(j); }, wrapped_d, Clamp(),
                     r == 4 || self_any_row);
+        else if (F == kSearchPlain)
+          scan_span(b, e, global_x, axes_d, Clamp(), r == 4 || self_any_row);
         else
           scan_span(b, e, global_x, wrapped_d, Clamp(), r == 4 || self_any_row);
-        b = use ? A.cell_start[c] : 0u;
-        e = use ? A.cell_start[c + 1u] : 0u;
-        prev = use ? nz : -2;
       }
     }
   }
@@ -3338,15 +3376,18 @@ void launch_neighbors(const Launch& L, const DevArrays& A, int with_factor, hipS
   else if (L.quad)
     hipLaunchKernelGGL(k_neighbors_quad<false>, dim3(L.pblocks * (kBlock / 16u)), dim3(64), 0, s,
                        L.T, A, with_factor);
+  else if (L.p0.wrap_mask && L.loose)
+    hipLaunchKernelGGL((k_neighbors<true, kSearchPlain>), dim3(L.pblocks * (kBlock / 64u)), dim3(64),
+                       0, s, L.T, A, with_factor);
   else if (L.p0.wrap_mask)
-    hipLaunchKernelGGL((k_neighbors<true, false>), dim3(L.pblocks * (kBlock / 64u)), dim3(64), 0, s,
-                       L.T, A, with_factor);
+    hipLaunchKernelGGL((k_neighbors<true, kSearchStaged>), dim3(L.pblocks * (kBlock / 64u)), dim3(64),
+                       0, s, L.T, A, with_factor);
   else if (L.tiles)
-    hipLaunchKernelGGL((k_neighbors<false, true>), dim3(L.pblocks), dim3(kBlock), 0, s, L.T, A,
-                       with_factor);
+    hipLaunchKernelGGL((k_neighbors<false, kSearchTile>), dim3(L.pblocks), dim3(kBlock), 0, s, L.T,
+                       A, with_factor);
   else
-    hipLaunchKernelGGL((k_neighbors<false, false>), dim3(L.pblocks * (kBlock / 64u)), dim3(64), 0, s,
-                       L.T, A, with_factor);
+    hipLaunchKernelGGL((k_neighbors<false, kSearchStaged>), dim3(L.pblocks * (kBlock / 64u)), dim3(64),
+                       0, s, L.T, A, with_factor);
   if (g_profiler) g_profiler->end("k_neighbors", s);
 }
 // instances of the neighbour passes
