@@ -157,6 +157,15 @@ void peirce_table(float out[120]) {
   }
 }
 
+// corner nodes of a map of res cells, and two on every edge
+size_t map_nodes(const unsigned res[3]) {
+  const size_t nv = size_t(res[0] + 1) * (res[1] + 1) * (res[2] + 1);
+  const size_t ne = size_t(res[0]) * (res[1] + 1) * (res[2] + 1) +
+                    size_t(res[0] + 1) * res[1] * (res[2] + 1) +
+                    size_t(res[0] + 1) * (res[1] + 1) * res[2];
+  return nv + 2 * ne;
+}
+
 SimParams make_params(const alv_const& cn, const alv_consti& cni, unsigned num_boundaries,
                       unsigned n) {
   SimParams p;
@@ -800,11 +809,7 @@ int place_boundary(alv_pile* pile, int slot, const alv_const* cn, const alv_dist
     }
     B.map_radius2 = float(r2 * (1.0 + 1e-4) + 1e-12);
   }
-  size_t nv = size_t(res[0] + 1) * (res[1] + 1) * (res[2] + 1);
-  size_t ne = size_t(res[0]) * (res[1] + 1) * (res[2] + 1) +
-              size_t(res[0] + 1) * res[1] * (res[2] + 1) +
-              size_t(res[0] + 1) * (res[1] + 1) * res[2];
-  size_t nodes = nv + 2 * ne;
+  size_t nodes = map_nodes(res);
   const bool pellets = pile->volume_method == ALV_PELLETS;
   if (pellets) nodes = 0;  // build_grid builds no volume map (pile.hpp:523)
   if (nodes >= (1ull << 32)) return fail(ALV_ERR_UNSUPPORTED, "volume map too large");
@@ -2753,11 +2758,7 @@ int alv_node_positions(const float dmin[3], const unsigned res[3], const float c
     g.cs[a] = cs[a];
     g.res[a] = res[a];
   }
-  size_t nv = size_t(res[0] + 1) * (res[1] + 1) * (res[2] + 1);
-  size_t ne = size_t(res[0]) * (res[1] + 1) * (res[2] + 1) +
-              size_t(res[0] + 1) * res[1] * (res[2] + 1) +
-              size_t(res[0] + 1) * (res[1] + 1) * res[2];
-  g.num_nodes = unsigned(nv + 2 * ne);
+  g.num_nodes = unsigned(map_nodes(res));
   if (num_nodes) *num_nodes = g.num_nodes;
   if (!out) return ALV_OK;
   float* d = nullptr;
@@ -2797,7 +2798,11 @@ int alv_check_math(const alv_const* cn, int op, const float* a, const float* b, 
 int alv_volume_from_distance_map(const alv_const* cn, const float dmin[3], const float dmax[3],
                                  const unsigned res[3], const float cs[3], float sign,
                                  const float* distance, float* volume, unsigned num_nodes) {
-  if (!cn || !distance || !volume) return fail(ALV_ERR_ARG, "null argument");
+  if (!cn || !dmin || !dmax || !res || !cs || !distance || !volume)
+    return fail(ALV_ERR_ARG, "null argument");
+  if (num_nodes == 0) return ALV_OK;
+  // every node is computed, from the values of all
+  if (map_nodes(res) != num_nodes) return fail(ALV_ERR_ARG, "not the number of the map's nodes");
   GridGeomDev g;
   memset(&g, 0, sizeof(g));
   for (int a = 0; a < 3; ++a) {

@@ -501,7 +501,8 @@ int alv_node_positions(const float domain_min[3], const unsigned resolution[3],
                        const float cell_size[3], float* out,
                        unsigned* num_nodes);
 /* update_volume_field, distance-map variant (runner.hpp:1616-1658), on host
- * buffers: distance[num_nodes] in, volume[num_nodes] out. */
+ * buffers: distance[num_nodes] in, volume[num_nodes] out; num_nodes is the
+ * number of nodes of the grid (alv_node_positions). */
 int alv_volume_from_distance_map(const alv_const* cn,
                                  const float domain_min[3],
                                  const float domain_max[3],

@@ -42,6 +42,22 @@ def test_error_string_without_gpu_call():
     assert isinstance(lib.alv_last_error(), bytes)
 
 
+def test_volume_map_takes_the_maps_node_count():
+    """The call computes every node of the map: with fewer than that it would
+    write past the caller's array (refused before anything is launched)."""
+    from alluvion_amd import LIB_PATH
+    lib = ctypes.CDLL(LIB_PATH)
+    lib.alv_last_error.restype = ctypes.c_char_p
+    cn = (ctypes.c_float * 20)()
+    lo, hi, cs = ((ctypes.c_float * 3)(*[v] * 3) for v in (0.0, 1.0, 0.25))
+    res, full = (ctypes.c_uint * 3)(4, 4, 4), 5 ** 3 + 6 * 4 * 25
+    dist, vol = (ctypes.c_float * (full + 1))(), (ctypes.c_float * (full + 1))()
+    for count in (1, 125, full - 1, full + 1):
+        rc = lib.alv_volume_from_distance_map(cn, lo, hi, res, cs, ctypes.c_float(1.0), dist, vol,
+                                              count)
+        assert rc == 2 and b"nodes" in lib.alv_last_error(), (count, rc)
+
+
 def test_python_module_names():
     import alluvion_amd._alluvion as al
     for name in ("Store", "Runnerfloat", "Constfloat", "ConstiN", "Pilefloat", "SolverDffloat",
