@@ -72,9 +72,8 @@ def test_empty_solver_steps():
     assert not count.any() and not anomaly.any()
 
 
-def free_body_matches(kind, tiles=False):
-    """A rotated free box hit by a fluid block (no gravity, no viscosity):
-    fluid velocities and the body's kinematics over three steps."""
+def free_body_scene():
+    """A rotated free box hit by a fluid block (no gravity, no viscosity)."""
     x = scenes.lattice_block(12, 12, 12, 0.0025, -0.03, 7, 0.00025)
     x[:, 1] += np.float32(0.044)
     v = np.zeros_like(x)
@@ -83,33 +82,82 @@ def free_body_matches(kind, tiles=False):
     q /= np.linalg.norm(q)
     body = scenes.BoundarySpec("box", (0.03, 0.02, 0.025, 0.0), 1.0, (16, 16, 16), mass=0.05,
                                inertia=(2e-5, 3e-5, 4e-5), x=(0.004, 0.0, 0.003), q=tuple(q))
-    sc = scenes.Scene(name="fluid_on_free_box", x=x.astype(np.float32), v=v.astype(np.float32),
-                      gravity=(0, 0, 0), pile_gravity=(0, 0, 0), viscosity=0.0,
-                      boundary_viscosity=0.0, boundaries=[body], grid_offset=(-8, -8, -8),
-                      grid_res=(16, 16, 16))
+    return scenes.Scene(name="fluid_on_free_box", x=x.astype(np.float32), v=v.astype(np.float32),
+                        gravity=(0, 0, 0), pile_gravity=(0, 0, 0), viscosity=0.0,
+                        boundary_viscosity=0.0, boundaries=[body], grid_offset=(-8, -8, -8),
+                        grid_res=(16, 16, 16))
+
+
+def compare_with_body(dp, pile, solver, orc, step):
+    n = orc.n
+    assert solver.num_density_solve == orc.report()["num_density_solve"], step
+    assert rel_err(dp.coat(solver.particle_v).get()[:n], orc.get("v")[:n]) < REL, step
+    rb = orc.rigid(0)
+    qg = pile.get_q(0)
+    np.testing.assert_allclose(list(pile.get_x(0)), rb["x"], rtol=1e-6, atol=1e-8, err_msg=str(step))
+    np.testing.assert_allclose(list(pile.get_v(0)), rb["v"], rtol=1e-4, atol=1e-6,
+                               err_msg=str(step))
+    np.testing.assert_allclose(list(pile.get_omega(0)), rb["omega"], rtol=1e-4,
+                               atol=1e-5, err_msg=str(step))
+    np.testing.assert_allclose([qg.x, qg.y, qg.z, qg.w], rb["q"], rtol=0, atol=1e-6,
+                               err_msg=str(step))
+
+
+def free_body_matches(kind, tiles=False):
+    """Fluid velocities and the body's kinematics over three steps."""
+    sc = free_body_scene()
     dp, pile, solver, _, _ = scenes.build_solver(sc, kind)
     solver.set_tiles(tiles)
     orc = oracle_like(sc, dp, pile, kind=kind)
-    n = sc.n
     for step in range(3):
         if step:  # each step from the GPU's state, the body's included
             sync(dp, solver, pile, orc, kind=kind)
         solver.step()
         orc.step()
-        assert solver.num_density_solve == orc.report()["num_density_solve"], step
-        assert rel_err(dp.coat(solver.particle_v).get()[:n], orc.get("v")[:n]) < REL, step
-        rb = orc.rigid(0)
-        qg = pile.get_q(0)
-        np.testing.assert_allclose(list(pile.get_x(0)), rb["x"], rtol=1e-6, atol=1e-8, err_msg=str(step))
-        np.testing.assert_allclose(list(pile.get_v(0)), rb["v"], rtol=1e-4, atol=1e-6,
-                                   err_msg=str(step))
-        np.testing.assert_allclose(list(pile.get_omega(0)), rb["omega"], rtol=1e-4,
-                                   atol=1e-5, err_msg=str(step))
-        np.testing.assert_allclose([qg.x, qg.y, qg.z, qg.w], rb["q"], rtol=0, atol=1e-6,
-                                   err_msg=str(step))
+        compare_with_body(dp, pile, solver, orc, step)
     assert np.abs(orc.rigid(0)["omega"]).max() > 1e-3  # the fluid turns the box
 
 
 @pytest.mark.parametrize("kind", ["df", "ii", "i"])
 def test_free_body_driven_by_fluid_matches_oracle(kind):
     free_body_matches(kind)
+
+
+@pytest.mark.parametrize("kind,late,graph", [
+    ("df", "divergence", False), ("df", "density", False), ("df", "both", False),
+    ("df", "divergence", True), ("df", "density", True), ("df", "both", True),
+    ("ii", "density", False), ("i", "density", False)])  # these have no graph
+def test_solve_longer_than_its_chunk(kind, late, graph):
+    """What follows a solve is enqueued before the host has seen it end.  A
+    step whose solves take more iterations than the steps before (a tolerance
+    that is never met and a growing maximum) finishes them and runs the rest
+    once: a second reaction on the body, or a second integration, would show."""
+    sc = free_body_scene()
+    dp, pile, solver, _, _ = scenes.build_solver(sc, kind)
+    solver.set_graph(graph)
+    orc = oracle_like(sc, dp, pile, kind=kind)
+    names = {"divergence": ["density_change"], "density": ["density_error"],
+             "both": ["density_change", "density_error"]}[late]
+    maxima = {"density_change": "max_divergence_solve", "density_error": "max_density_solve"}
+    for step, most in enumerate((None, None, 5, 11, 12)):
+        now = {}
+        for k in maxima if kind == "df" else ["density_error"]:
+            never = most is not None and k in names
+            now[k + "_tolerance"] = -1e30 if never else 1e30
+            now[maxima[k]] = most if never else 20
+        for k, value in now.items():
+            setattr(solver, k, value)
+        orc.update_settings(**now)
+        if step:
+            sync(dp, solver, pile, orc, kind=kind)
+        solver.step()
+        orc.step()
+        compare_with_body(dp, pile, solver, orc, step)
+        counts = {"density_error": solver.num_density_solve}
+        if kind == "df":
+            counts["density_change"] = solver.num_divergence_solve
+        for k, count in counts.items():
+            if most is not None and k in names:
+                assert count == most, step
+            else:
+                assert count < 5, step

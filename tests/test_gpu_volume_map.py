@@ -51,10 +51,28 @@ def test_every_class_matches_oracle(kind, params, sign, res, sampled):
     ("box_shell", (0.1, 0.1, 0.1, 0.02, 0.0), 1.0)])
 def test_both_kernels_give_the_same_sums(kind, params, sign):
     # corner nodes of the coarse grid are corner nodes of the fine one: their
-    # coordinates are the same numbers (cell sizes in the ratio 2)
+    # coordinates are the same numbers (cell sizes in the ratio 4)
     coarse, _ = gpu_map(one_boundary(kind, params, sign, (24,) * 3))
     fine, _ = gpu_map(one_boundary(kind, params, sign, (96,) * 3))
     c = coarse[:25 ** 3].reshape(25, 25, 25)
     f = fine[:97 ** 3].reshape(97, 97, 97)[::4, ::4, ::4]
     assert (c > 0).any()
     np.testing.assert_array_equal(c, f)
+
+
+def test_large_sampled_map_matches_oracle():
+    """A sampled map with more nodes near the surface than run as teams (every
+    node whose volume lies between none and the whole ball is one)."""
+    sc = one_boundary("box", (0.04, 0.05, 0.045, 0.0), 1.0, (48, 50, 52), sampled=True)
+    got, dist = gpu_map(sc)
+    ball = 4 * np.pi / 3 * sc.kernel_radius ** 3
+    near = np.flatnonzero((got > 1e-3 * ball) & (got < 0.99 * ball))
+    assert near.size > 1 << 19
+    dmin, dmax, res, cs = of.Oracle(sc, precision=4).grid_info(0)
+    picked = np.random.default_rng(3).choice(near, 40, replace=False)
+    picked = np.concatenate([picked, [0, got.size - 1], np.flatnonzero(got == 0.0)[:10],
+                             np.argsort(got)[-10:]])
+    for node in picked:
+        ref = of.volume_from_distance_map(4, sc.kernel_radius, dmin, dmax, res, cs, 1.0, dist,
+                                          int(node), int(node) + 1)[0]
+        assert abs(float(got[node]) - ref) <= 1e-5 * ball, node
