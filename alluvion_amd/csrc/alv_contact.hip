@@ -9,7 +9,7 @@
 // the candidates are numbered (pair in (i, j) order, then vertex), one pass
 // over all of them leaves a bit per candidate, and a second one places each
 // hit at the number of bits before its own, so contacts come out in that
-// order on every run.
+// order on every run.  Few candidates are tested and placed by one block.
 #include <hip/hip_runtime.h>
 
 #include "alv_contact.hpp"
@@ -20,6 +20,10 @@ namespace {
 
 constexpr unsigned kContactThreads = 256;
 constexpr unsigned kContactWaves = kContactThreads / 64;
+// Candidates that one block tests and numbers by itself, in one launch: a whole
+// find_contacts of 24 takes 55 us and 57 with the two passes, of 768 62 and 64,
+// of 1,024 both 68; a second round of 1,024 takes one block 8 us more.
+constexpr unsigned kFewCandidates = 1024;
 
 // R diag(v) R^T for the rotation of q, stored as diagonal and (01, 02, 12)
 // off-diagonal (runner.hpp:178-199).
@@ -65,9 +69,9 @@ __device__ inline void put3(float* dst, vec3 v) {
 }
 
 // Tests vertex `vert` of body i against body j: whether it is inside body j
-// (dist < 0) or, with `Record`, the record of a vertex known to be.  World vertices (pellets,
-// collision_test_with_pellets, runner.hpp:3627-3727) are already placed;
-// body-frame vertices are placed with body i's kinematics.  `inertia`
+// (dist < 0) and, with `Record`, the record of one that is.  World vertices
+// (pellets, collision_test_with_pellets, runner.hpp:3627-3727) are already
+// placed; body-frame vertices are placed with body i's kinematics.  `inertia`
 // holds [B][3] principal inertia, then [B][2] (restitution, friction).
 template <bool Record>
 __device__ bool test_vertex(unsigned i, unsigned j, unsigned flags, unsigned nb,
@@ -103,7 +107,8 @@ __device__ bool test_vertex(unsigned i, unsigned j, unsigned flags, unsigned nb,
     dist = sdf_eval(Bj, wrt_j) * Bj.sign - tolerance;
     n = sdf_gradient(Bj, wrt_j, 1e-3f) * Bj.sign;
   }
-  if (!Record) return dist < 0;
+  if (!(dist < 0)) return false;
+  if (!Record) return true;
   n = n * (1.0f / sqrtf(length_sqr(n)));
   const vec3 cp_j = rotate(wrt_j - dist * n, qj) + xj;
   const vec3 nw = rotate(n, qj);
@@ -159,6 +164,27 @@ __device__ bool test_candidate(unsigned c, const ContactJob* jobs, unsigned num_
   const unsigned local = c - J.cbase;
   return test_vertex<Record>(J.i, J.j + local % J.nj, J.flags, nb, bodies, inertia, verts,
                              J.vbase + local / J.nj, tolerance, out);
+}
+
+// Few candidates: one block, the hits numbered by a scan over its waves.
+__global__ __launch_bounds__(kFewCandidates) void k_collision_few(
+    const ContactJob* jobs, unsigned num_jobs, unsigned num_candidates, unsigned nb,
+    const BoundaryDev* bodies, const float* inertia, const float* verts, float tolerance,
+    unsigned max_contacts, alv_contact* contacts, unsigned* count) {
+  __shared__ unsigned wave_sum[kFewCandidates / 64];
+  const unsigned lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  alv_contact rec;
+  const bool hit = threadIdx.x < num_candidates &&
+                   test_candidate<true>(threadIdx.x, jobs, num_jobs, nb, bodies, inertia, verts,
+                                        tolerance, &rec);
+  const unsigned long long mask = __ballot(hit);
+  if (lane == 0) wave_sum[wave] = unsigned(__popcll(mask));
+  __syncthreads();
+  unsigned slot = 0;
+  for (unsigned w = 0; w < wave; ++w) slot += wave_sum[w];
+  if (threadIdx.x == blockDim.x - 1) count[0] = slot + wave_sum[wave];
+  slot += unsigned(__popcll(mask & ((1ull << lane) - 1ull)));
+  if (hit && slot < max_contacts) contacts[slot] = rec;
 }
 
 // One candidate per thread; hits[w]: the candidates 64 w ... that are inside.
@@ -221,6 +247,12 @@ void launch_collision(const ContactJob* jobs, unsigned num_jobs, unsigned num_ca
                       const float* verts, float tolerance, unsigned max_contacts,
                       unsigned long long* hits, alv_contact* contacts, unsigned* count,
                       hipStream_t s) {
+  if (num_candidates <= kFewCandidates) {
+    hipLaunchKernelGGL(k_collision_few, dim3(1), dim3((num_candidates + 63u) / 64u * 64u), 0, s, jobs,
+                       num_jobs, num_candidates, nb, bodies, inertia, verts, tolerance, max_contacts,
+                       contacts, count);
+    return;
+  }
   const dim3 blocks(unsigned(collision_hit_words(num_candidates) / kContactWaves));
   hipLaunchKernelGGL(k_collision_hits, blocks, dim3(kContactThreads), 0, s, jobs, num_jobs,
                      num_candidates, nb, bodies, inertia, verts, tolerance, hits);

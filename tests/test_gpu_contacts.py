@@ -59,7 +59,7 @@ def test_contacts_and_solve_match_oracle():
     np.testing.assert_allclose(w, rb["omega"], rtol=1e-5, atol=1e-5)
 
 
-@pytest.mark.parametrize("nv", [1, 63, 64, 65, 255, 256, 257, 1025])
+@pytest.mark.parametrize("nv", [1, 63, 64, 65, 255, 256, 257, 1024, 1025])
 @pytest.mark.parametrize("kept", [512, 40])
 def test_candidates_over_waves_and_blocks(nv, kept):
     """Contacts numbered over the ends of waves and blocks, with runs of
