@@ -2311,8 +2311,8 @@ int alv_solver_step(alv_solver* S) {
   if (S->kind != ALV_SOLVER_DF && (!A.pressure || !A.last_pressure || !A.aii || !A.pacc))
     return fail(ALV_ERR_STATE, "pressure-solve arrays are not allocated");
   if (S->kind == ALV_SOLVER_DF) {
-    // SolverDf::step (solver_df.hpp:74-359) in three segments; the host
-    // checks convergence between them
+    // SolverDf::step (solver_df.hpp:74-359) in three segments; for a batch the
+    // host checks convergence between them, for one scene at the end
     const int div = S->set.enable_divergence_solve != 0;
     const int dens = S->set.enable_density_solve != 0;
     const int learned_dens = S->net != nullptr && S->net_dens && div;

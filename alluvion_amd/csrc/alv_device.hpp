@@ -174,9 +174,13 @@ __device__ inline vec3 gradW(vec3 d, const SimParams& p) { return gradW_scale<fa
 // these the hardware gives only the estimate 2^-k for r = 2^k (1 - 2^-24)
 // (checked on the GPU for every significand), where rr is one ulp low; a
 // quotient by that r still rounds correctly unless the dividend is a power of
-// two.  Seven instructions with one transcendental where sqrt_rn and rcp_rn
-// take twelve with two.  x is raised to 2^-96 (a pair at distance 0: q is then
-// 2^-48 / h and the kernel values are those of q = 0).
+// two.  So the gradient has the bits of the IEEE division but at one distance
+// of a few radii: h with 1 - r / h a power of two at an r = 2^k (1 - 2^-24), as
+// 2^-7 (and not 0.01), where the quotient is one ulp off; and at r = h, where
+// its zero may have the other sign.  Seven instructions with one transcendental
+// where sqrt_rn and rcp_rn take twelve with two.  x is raised to 2^-96 (a pair
+// at distance 0): q is then 2^-48 / h and, for h above 2^-23, the kernel values
+// are those of q = 0.
 struct PairRoot {
   float r, rr;
 };

@@ -1930,9 +1930,11 @@ __global__ __launch_bounds__(pass_threads(M, stiffness_lanes(M))) void k_ws_div1
 // the solve's last: the last pass that runs sees the final velocities, which
 // k_viscosity would read.  This pass is the last only if the control block
 // says no iteration follows; an iteration's k_div_err is not the last while
-// the iteration count stays below the minimum and the maximum.  Both passes
-// are bounded to 64 VGPRs (8 waves per SIMD); unbounded, the viscosity terms
-// take 66 (7 waves per SIMD), which measured 2 % slower.
+// the iteration count stays below the minimum and the maximum.  In the gather
+// and tile forms both passes are bounded to 64 VGPRs (8 waves per SIMD);
+// unbounded, the viscosity terms take 66 (7 waves per SIMD), which measured 2 %
+// slower.  The deep form holds all gathers of a particle (109 VGPRs) and has
+// fewer waves than the chip takes, so it is bounded to 3 per SIMD only.
 template <bool W, int M>
 __global__ __launch_bounds__(pass_threads(M, change_lanes(M)), M == kDeep ? 3 : 8) void k_vel_density_change(SceneTab T, DevArrays A) {
   __shared__ float lds[pass_threads(M, change_lanes(M)) / 64];

@@ -384,7 +384,9 @@ __global__ __launch_bounds__(256) void k_ball_sums(SimParams p, D dist, float ma
 
 // Few nodes: 64 nodes per block of 16 waves.  Waves 1 to 15 evaluate the
 // terms of one unit each (five rays a round) into LDS, wave 0 adds the
-// previous round's terms in order meanwhile.
+// previous round's terms in order meanwhile.  The instance for distance maps
+// spills five registers at its bound of 64 and is the faster for it: 42 ms
+// against 43 for a sampled 32^3 map.
 constexpr unsigned kTeam = 16;
 constexpr unsigned kRoundRays = (kTeam - 1u) * kUnit / kRadii;
 static_assert((kTeam - 1u) * kUnit % kRadii == 0u && kRays % kRoundRays == 0u, "whole rays");

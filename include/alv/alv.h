@@ -414,13 +414,14 @@ int alv_solver_step(alv_solver* solver);
  * step runs as three HIP graphs (neighbour search and divergence warm start,
  * viscosity to density warm start, final integration), captured on first use
  * and replayed; each graph holds the last step's Jacobi iteration count plus
- * `slack` iterations, iterations past convergence return at once, and the
- * host adds more only when a scene has not converged.  Results are identical
+ * `slack` iterations (grown at once, shrunk after 16 smaller steps, as for
+ * direct launches), iterations past convergence return at once, and the host
+ * adds more only when a scene has not converged.  Results are identical
  * with and without graphs.  Per-kernel profiling uses direct launches. */
 int alv_solver_set_graph(alv_solver* solver, int enable, unsigned slack);
 /* Neighbour passes that copy each 256-particle block's neighbourhood (three
  * contiguous ranges of sorted particles) into LDS before their loops (no
- * counterpart in the reference; on by default).  Blocks whose neighbourhood
+ * counterpart in the reference; off by default).  Blocks whose neighbourhood
  * does not fit, and periodic grids, read neighbours from global memory.
  * Results are identical either way. */
 int alv_solver_set_tiles(alv_solver* solver, int enable);
